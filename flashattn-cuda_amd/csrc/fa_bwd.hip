@@ -251,9 +251,8 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
                                              const f16* __restrict__ V, const f16* __restrict__ dO,
                                              const float* __restrict__ NL,
                                              const float* __restrict__ ND, float* __restrict__ dK,
-                                             float* __restrict__ dV, const Geom& geo, int num_kb,
-                                             int total, float c, float scale, int block,
-                                             char* smem /* dkdv_pp_smem<D>() bytes */) {
+                                             float* __restrict__ dV, const HeadView& hv, int kb, float c,
+                                             float scale, char* smem /* dkdv_pp_smem<D>() bytes */) {
   static_assert(D == 64, "a 32-row half of a tile is 4 blocks, the register budget D = 64's");
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
@@ -269,15 +268,10 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   const int grp = wave >> 2;                   // also this group's query half of a tile
   const int qb = grp;
   const int hi = lane >> 5;
-  const int logical = xcd_remap(block, total, geo.nxcd);
-  const int bh = logical / num_kb;
-  const int kb = logical - bh * num_kb;
   const int k0 = kb * kBlk;
   const int key = k0 + 32 * kw + (lane & 31);
 
-  const HeadView hv = head_view<D>(geo, bh);
   const int N = hv.n;
-  if (k0 >= N) return;   // varlen: past this sequence (whole workgroup)
   const size_t head = hv.q;
   const int head_bytes = N * D * 2;
   const char* Qh = reinterpret_cast<const char*>(Q + head);
@@ -456,8 +450,7 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
                                            const f16* __restrict__ V, const f16* __restrict__ dO,
                                            const float* __restrict__ NL,
                                            const float* __restrict__ ND, float* __restrict__ dQ,
-                                           const Geom& geo, int num_qb, int total, float c,
-                                           float scale, int block,
+                                           const HeadView& hv, int qblk, float c, float scale,
                                            char* smem /* dq_pp_smem<D>() bytes */) {
   static_assert(D == 64, "a 32-row half of a tile is 4 blocks, the register budget D = 64's");
   constexpr int TILE = kBQ * D * 2;
@@ -474,16 +467,10 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   const int grp = wave >> 2;                   // also this group's key half of a tile
   const int half = grp;
   const int hi = lane >> 5;
-  const int logical = xcd_remap(block, total, geo.nxcd);
-  const int bh = logical / num_qb;
-  int qblk = logical - bh * num_qb;
-  if (CAUSAL) qblk = num_qb - 1 - qblk;   // longest rows first
   const int q0 = qblk * kBlk;
   const int query = q0 + 32 * qw + (lane & 31);
 
-  const HeadView hv = head_view<D>(geo, bh);
   const int N = hv.n;
-  if (q0 >= N) return;   // varlen: past this sequence (whole workgroup)
   const size_t head = hv.q;
   const int head_bytes = N * D * 2;
   const char* Kh = reinterpret_cast<const char*>(K + hv.kv);
@@ -665,8 +652,7 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
                                                 const float* __restrict__ NL,
                                                 const float* __restrict__ ND,
                                                 float* __restrict__ dK, float* __restrict__ dV,
-                                                const Geom& geo, int num_kb, int total, float c,
-                                                float scale, int block,
+                                                const HeadView& hv, int kb, float c, float scale,
                                                 char* smem /* dkdv_pp128_smem<D>() bytes */) {
   static_assert(D == 128, "a 32-row half of a tile is 8 blocks");
   constexpr int TILE = kBQ * D * 2;
@@ -687,14 +673,9 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   const int grp = wave >> 2;                   // also this group's query half of a tile
   const int qb = grp;
   const int hi = lane >> 5;
-  const int logical = xcd_remap(block, total, geo.nxcd);
-  const int bh = logical / num_kb;
-  const int kb = logical - bh * num_kb;
   const int k0 = kb * kBlk;
 
-  const HeadView hv = head_view<D>(geo, bh);
   const int N = hv.n;
-  if (k0 >= N) return;   // varlen: past this sequence (whole workgroup)
   const size_t head = hv.q;
   const int head_bytes = N * D * 2;
   const char* Qh = reinterpret_cast<const char*>(Q + head);
@@ -889,8 +870,7 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
                                               const f16* __restrict__ dO,
                                               const float* __restrict__ NL,
                                               const float* __restrict__ ND, float* __restrict__ dQ,
-                                              const Geom& geo, int num_qb, int total, float c,
-                                              float scale, int block,
+                                              const HeadView& hv, int qblk, float c, float scale,
                                               char* smem /* dq_pp128_smem<D>() bytes */) {
   static_assert(D == 128, "a 32-row half of a tile is 8 blocks");
   constexpr int TILE = kBQ * D * 2;
@@ -909,16 +889,10 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
   const int grp = wave >> 2;                   // also this group's key half of a tile
   const int half = grp;
   const int hi = lane >> 5;
-  const int logical = xcd_remap(block, total, geo.nxcd);
-  const int bh = logical / num_qb;
-  int qblk = logical - bh * num_qb;
-  if (CAUSAL) qblk = num_qb - 1 - qblk;   // longest rows first
   const int q0 = qblk * kBlk;
   const int query = q0 + 32 * qw + (lane & 31);
 
-  const HeadView hv = head_view<D>(geo, bh);
   const int N = hv.n;
-  if (q0 >= N) return;   // varlen: past this sequence (whole workgroup)
   const size_t head = hv.q;
   const int head_bytes = N * D * 2;
   const char* Kh = reinterpret_cast<const char*>(K + hv.kv);
@@ -1065,38 +1039,50 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
 }
 
 // dK/dV and dQ in one launch (both bodies take 8 waves and share one LDS
-// buffer): blocks [0, total) run the dK/dV body, [total, 2 total) the dQ
-// body. Each half is dispatched longest unit first, so a CU that
-// finished a short dK/dV unit (late keys of a causal head) picks up a long
-// dQ unit: the causal triangle's two halves even out across the CUs instead
-// of each kernel waiting for its own longest unit.
+// buffer): the first half of the blocks runs the dK/dV body of a key block,
+// the second half the dQ body of a query block, each half longest unit first
+// (unit_of). A CU that finished a short dK/dV unit (late keys of a causal
+// head) picks up a long dQ unit, and the short dQ units fill the end. The
+// halves are not interleaved: a dK/dV unit takes 4/3 of a dQ unit's time, and
+// where each CU gets one of both, two dK/dV units on one CU are the longest
+// (B1 H8 N4096 D64 non-causal 136 us, interleaved 150).
 template <int D, bool CAUSAL, bool BF16>
 __global__ void __launch_bounds__(512)
 fa_bwd_fused_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
                     const f16* __restrict__ V, const f16* __restrict__ dO,
                     const float* __restrict__ NL, const float* __restrict__ ND,
                     float* __restrict__ dK, float* __restrict__ dV, float* __restrict__ dQ,
-                    Geom geo, int nb, int total, float c, float scale) {
+                    Geom geo, UnitMap um, float c, float scale) {
   // One LDS buffer serves whichever body this workgroup runs.
   constexpr int SK = D == 64 ? dkdv_pp_smem<D>() : dkdv_pp128_smem<D>();
   constexpr int SQ = D == 64 ? dq_pp_smem<D>() : dq_pp128_smem<D>();
   __shared__ __attribute__((aligned(1024))) char smem[SK > SQ ? SK : SQ];
-  const int blk = (int)blockIdx.x;
-  if (blk < total) {
+  const int total = um.heads * um.per_head;
+  const bool dq_role = (int)blockIdx.x >= total;
+  const Unit un = unit_of(dq_role ? blockIdx.x - total : blockIdx.x, um);
+  HeadView hv;
+  int kb = un.idx;
+  if (geo.cu != nullptr) {
+    const SeqBlock sb = varlen_block(geo, un.idx, kBlk, threadIdx.x & 63);
+    if (sb.n == 0) return;   // the grid is a bound on the units (whole workgroup)
+    hv = seq_view<D>(geo, un.head, sb.start, sb.n);
+    kb = sb.block;
+  } else {
+    hv = dense_view<D>(geo, un.head);
+  }
+  // Causal: the first key blocks and the last query blocks are the longest.
+  const int qblk = CAUSAL ? (hv.n + kBlk - 1) / kBlk - 1 - kb : kb;
+  if (!dq_role) {
     if constexpr (D == 64) {
-      dkdv_body_pp<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dK, dV, geo, nb, total, c, scale, blk,
-                                    smem);
+      dkdv_body_pp<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dK, dV, hv, kb, c, scale, smem);
     } else {
-      dkdv_body_pp128<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dK, dV, geo, nb, total, c, scale,
-                                       blk, smem);
+      dkdv_body_pp128<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dK, dV, hv, kb, c, scale, smem);
     }
   } else {
     if constexpr (D == 64) {
-      dq_body_pp<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dQ, geo, nb, total, c, scale, blk - total,
-                                  smem);
+      dq_body_pp<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dQ, hv, qblk, c, scale, smem);
     } else {
-      dq_body_pp128<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dQ, geo, nb, total, c, scale,
-                                     blk - total, smem);
+      dq_body_pp128<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dQ, hv, qblk, c, scale, smem);
     }
   }
 }
@@ -1121,12 +1107,12 @@ fa_bwd_group_sum_kernel(const float* __restrict__ part, float* __restrict__ out,
 
 // The three passes (-D_i and -L log2 e, dK/dV, dQ) and, with H_kv < H, the
 // group sums. geo is dense (B heads of N rows per head) or varlen (heads of
-// geo.total packed rows; units = B*H (b, h) pairs either way); `rows` is the
-// number of L rows: B*H*N dense, H*total varlen.
+// geo.total packed rows); `rows` is the number of L rows: B*H*N dense, H*total
+// varlen.
 template <int D, bool CAUSAL, bool BF16>
 static hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o,
                              const void* dout, const float* lse, float* dq, float* dk, float* dv,
-                             float* ws, const Geom& geo, int64_t units, int64_t rows,
+                             float* ws, const Geom& geo, const UnitMap& um, int64_t rows,
                              int64_t out_heads, int64_t head_rows, hipStream_t s) {
   const float scale = (float)(1.0 / sqrt((double)D));
   const float c = scale * kLog2e;
@@ -1135,7 +1121,7 @@ static hipError_t launch_bwd(const void* q, const void* k, const void* v, const 
   const f16* V = (const f16*)v;
   const f16* O = (const f16*)o;
   const f16* G = (const f16*)dout;
-  const int group = geo.group;
+  const int group = (int)geo.group.d;
   float* nd = ws;
   float* nl = ws + rows;
   // GQA: per-query-head dK/dV partials in the workspace, summed per KV head.
@@ -1144,15 +1130,13 @@ static hipError_t launch_bwd(const void* q, const void* k, const void* v, const 
   float* dv_q = group == 1 ? dv : ws + part0 + rows * D;
   hipLaunchKernelGGL((fa_bwd_di_kernel<D, BF16>), dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, s, O,
                      G, lse, nd, nl, rows);
-  const int nb = (geo.N + kBlk - 1) / kBlk;
-  const int total = (int)(units * nb);
-  // dK/dV and dQ in one launch. A causal head's short and long units even
-  // out across the CUs (B1 H8 N4096 D128: 0.237 -> 0.165 ms against two
-  // launches); with units of one length the one launch measured level with
-  // two or slightly ahead (D = 128 non-causal, B1 H8 N4096 256.4 -> 254.5 us,
-  // B4 H16 N4096 1981.8 -> 1972.3 us; same gradients bit for bit).
-  hipLaunchKernelGGL((fa_bwd_fused_kernel<D, CAUSAL, BF16>), dim3(2 * total), dim3(512), 0, s,
-                     Q, K, V, G, nl, nd, dk_q, dv_q, dq, geo, nb, total, c, scale);
+  // dK/dV and dQ in one launch: with units of one length it measured level
+  // with two launches or slightly ahead (D = 128 non-causal, B1 H8 N4096
+  // 256.4 -> 254.5 us, B4 H16 N4096 1981.8 -> 1972.3 us; same gradients bit
+  // for bit), and a causal head's short and long units even out.
+  hipLaunchKernelGGL((fa_bwd_fused_kernel<D, CAUSAL, BF16>),
+                     dim3(2u * um.heads * um.per_head), dim3(512), 0, s, Q, K, V, G,
+                     nl, nd, dk_q, dv_q, dq, geo, um, c, scale);
   if (group > 1) {
     // out_heads KV heads of head_rows rows, each the sum of `group`
     // consecutive query heads' partials
@@ -1189,18 +1173,22 @@ namespace bwd {
 template <bool BF16>
 static int bwd_run(const void* q, const void* k, const void* v, const void* o, const void* dout,
                    const float* lse, float* dq, float* dk, float* dv, float* workspace,
-                   const Geom& geo_in, int64_t units, int64_t rows, int64_t out_heads,
+                   const Geom& geo, int64_t units, int64_t rows, int64_t out_heads,
                    int64_t head_rows, int64_t D, int causal, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  Geom geo = geo_in;
-  geo.nxcd = stream_topology(s).xcds;
+  // Units of a head: its blocks (varlen: a bound on those of its sequences).
+  const int64_t per_head = geo.cu == nullptr ? (geo.N + kBlk - 1) / kBlk
+                                             : varlen_units(geo.B, geo.total, geo.N, kBlk);
+  const int64_t heads = geo.cu == nullptr ? units : geo.H;
+  if (2 * heads * per_head > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
+  const UnitMap um = unit_map(heads, per_head, stream_topology(s), causal != 0 || geo.cu != nullptr);
   hipError_t e;
   if (D == 64) {
-    e = causal ? launch_bwd<64, true, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, units, rows, out_heads, head_rows, s)
-               : launch_bwd<64, false, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, units, rows, out_heads, head_rows, s);
+    e = causal ? launch_bwd<64, true, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
+               : launch_bwd<64, false, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
   } else {
-    e = causal ? launch_bwd<128, true, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, units, rows, out_heads, head_rows, s)
-               : launch_bwd<128, false, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, units, rows, out_heads, head_rows, s);
+    e = causal ? launch_bwd<128, true, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
+               : launch_bwd<128, false, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
   }
   return e == hipSuccess ? FA_OK : -(int)e;
 }
@@ -1214,7 +1202,7 @@ static int bwd_gqa(bool bf16, const void* q, const void* k, const void* v, const
   if (H_kv <= 0 || H % H_kv != 0) return FA_ERR_KV_HEADS;
   // the partials are written and read as 16-byte vectors
   if (H_kv != H && (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) return FA_ERR_ALIGNMENT;
-  const Geom geo{nullptr, (int)N, (int)H, (int)(H / H_kv), 0, 0, 0};   // nxcd: launcher
+  const Geom geo{nullptr, (int)N, (int)H, FastDiv(H / H_kv), 0, 0};
   return bf16 ? bwd_run<true>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, B * H,
                               B * H * N, B * H_kv, N, D, causal, stream)
               : bwd_run<false>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, B * H,
@@ -1257,8 +1245,8 @@ extern "C" int fa_bwd_varlen_f16(const void* q, const void* k, const void* v, co
   if (st != FA_OK) return st;
   if (total == 0) return FA_OK;
   if (H_kv != H && (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) return FA_ERR_ALIGNMENT;
-  const fa::Geom geo{cu_seqlens, (int)max_seqlen, (int)H, (int)(H / H_kv), (int)total,
-                       (int)B, 0};   // nxcd: launcher
+  const fa::Geom geo{cu_seqlens, (int)max_seqlen, (int)H, fa::FastDiv(H / H_kv), (int)total,
+                     (int)B};
   return fa::bwd::bwd_run<false>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, B * H,
                                  H * total, H_kv, total, D, causal, stream);
 }

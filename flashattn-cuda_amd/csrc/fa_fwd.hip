@@ -459,14 +459,14 @@ __device__ __forceinline__ void dma_block_or_zero(const char* head, int head_byt
 // partials normalised over its range and the range's LSE, merged by the LSE
 // combine afterwards.
 // ---------------------------------------------------------------------------
-template <int D, bool CAUSAL, bool WRITE_L, bool FULL, int RING, bool BF16 = false,
-          bool SPLITKV = false, int TG = 2>
-__global__ void __launch_bounds__(512)
-fa_fwd_pp_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
-                 const f16* __restrict__ V, f16* __restrict__ O,
-                 float* __restrict__ L, Geom geo, int num_qb, int total, float c,
-                 float* __restrict__ part_o = nullptr, float* __restrict__ part_lse = nullptr,
-                 int nsplit = 1) {
+// Row block qb of the head hv (split-KV: key range `split` of it); smem holds
+// 2 RING tiles.
+template <int D, bool CAUSAL, bool WRITE_L, bool FULL, int RING, bool BF16, bool SPLITKV, int TG>
+__device__ __forceinline__ void
+fwd_pp_body(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __restrict__ V,
+            f16* __restrict__ O, float* __restrict__ L, const HeadView& hv, int qb, int split,
+            int nsplit, float c, float* __restrict__ part_o, float* __restrict__ part_lse,
+            char* smem) {
   constexpr int NB = 2;                        // 32-key blocks per tile
   constexpr int TILE = kBC * D * 2;            // bytes of a 64-key K or V tile
   constexpr int BLOCKS = TILE / 1024;          // 1 KiB blocks per tile
@@ -486,9 +486,6 @@ fa_fwd_pp_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
   constexpr int PF = D == 64 ? 8 : 4;          // operand prefetch distance, in MFMAs
   constexpr int REC = RB::REC_FLOATS;          // floats per wave record of the merge
   static_assert(!SPLITKV || (TG - 1) * NRG * REC * 4 <= 2 * RING * TILE, "merge area too small");
-  // K slots at [0, RING) * TILE, V slots at [RING, 2 RING) * TILE.
-  __shared__ __attribute__((aligned(1024))) char smem[2 * RING * TILE];
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: SGPR
@@ -498,17 +495,7 @@ fa_fwd_pp_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
   // This wave's tile in step j.
   auto tile_of = [&](int j) { return TG * j + tg; };
 
-  const int logical = xcd_remap(blockIdx.x, total, geo.nxcd);
-  // Split-KV: the splits of one q-block are adjacent (same XCD, same K/V).
-  const int split = SPLITKV ? logical % nsplit : 0;
-  const int unit = SPLITKV ? logical / nsplit : logical;
-  const int bh = unit / num_qb;
-  int qb = unit - bh * num_qb;
-  if (CAUSAL) qb = num_qb - 1 - qb;   // longest rows dispatch first
-
-  const HeadView hv = head_view<D>(geo, bh);
   const int N = hv.n;
-  if (qb * ROWS >= N) return;   // varlen: past this sequence (whole workgroup)
   const size_t head = hv.q;
   const int head_bytes = N * D * 2;
   const int q0 = qb * ROWS;
@@ -779,6 +766,47 @@ fa_fwd_pp_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
   rb.finish_partial(part_o, part_lse, (hv.l + rb.qrow) * nsplit + split);
 }
 
+template <int D, bool CAUSAL, bool WRITE_L, bool FULL, int RING, bool BF16 = false,
+          bool SPLITKV = false, int TG = 2>
+__global__ void __launch_bounds__(512)
+fa_fwd_pp_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
+                 const f16* __restrict__ V, f16* __restrict__ O,
+                 float* __restrict__ L, Geom geo, UnitMap um, float c,
+                 float* __restrict__ part_o = nullptr, float* __restrict__ part_lse = nullptr,
+                 int nsplit = 1) {
+  constexpr int TILE = kBC * D * 2;
+  constexpr int ROWS = 32 * (8 / TG);
+  // K slots at [0, RING) * TILE, V slots at [RING, 2 RING) * TILE.
+  __shared__ __attribute__((aligned(1024))) char smem[2 * RING * TILE];
+  if constexpr (SPLITKV) {
+    // The splits of one row block are adjacent, on the same XCD.
+    const int logical = xcd_remap(blockIdx.x, um.heads * um.per_head * nsplit, (int)um.nxcd.d);
+    const int unit = logical / nsplit;
+    const int split = logical - unit * nsplit;
+    const int bh = unit / um.per_head;
+    int qb = unit - bh * um.per_head;
+    if (CAUSAL) qb = um.per_head - 1 - qb;   // longest rows dispatch first
+    fwd_pp_body<D, CAUSAL, WRITE_L, FULL, RING, BF16, true, TG>(
+        Q, K, V, O, L, dense_view<D>(geo, bh), qb, split, nsplit, c, part_o, part_lse, smem);
+  } else {
+    const Unit un = unit_of(blockIdx.x, um);
+    HeadView hv;
+    int idx = un.idx;
+    if (!FULL && geo.cu != nullptr) {
+      const SeqBlock sb = varlen_block(geo, un.idx, ROWS, threadIdx.x & 63);
+      if (sb.n == 0) return;   // the grid is a bound on the units (whole workgroup)
+      idx = sb.block;
+      hv = seq_view<D>(geo, un.head, sb.start, sb.n);
+    } else {
+      hv = dense_view<D>(geo, un.head);
+    }
+    // Longest rows dispatch first.
+    const int qb = CAUSAL ? (hv.n + ROWS - 1) / ROWS - 1 - idx : idx;
+    fwd_pp_body<D, CAUSAL, WRITE_L, FULL, RING, BF16, false, TG>(
+        Q, K, V, O, L, hv, qb, 0, 1, c, part_o, part_lse, smem);
+  }
+}
+
 // Kernel variants (for fa_probe_fwd_variant; the default path picks one per
 // problem shape): the ping-pong kernel with two tile groups over 128 rows and
 // a ring of 4 tiles (204), or with four tile groups over 64 rows and a ring
@@ -805,21 +833,22 @@ static bool variant_fits(int D, int variant, int causal) {
 // elements either way.
 template <int D, bool CAUSAL, bool WRITE_L, bool FULL, bool BF16>
 static hipError_t launch_fwd(const void* q, const void* k, const void* v, void* o,
-                             float* lse, Geom geo, int num_qb, int total, float c, int variant,
+                             float* lse, const Geom& geo, const UnitMap& um, float c, int variant,
                              hipStream_t stream) {
+  const dim3 grid((unsigned)(um.heads * um.per_head));
   const f16* Q = (const f16*)q;
   const f16* K = (const f16*)k;
   const f16* V = (const f16*)v;
   f16* Op = (f16*)o;
   switch (variant) {
     case kPingPong:
-      hipLaunchKernelGGL((fa_fwd_pp_kernel<D, CAUSAL, WRITE_L, FULL, 4, BF16>), dim3(total),
-                         dim3(512), 0, stream, Q, K, V, Op, lse, geo, num_qb, total, c);
+      hipLaunchKernelGGL((fa_fwd_pp_kernel<D, CAUSAL, WRITE_L, FULL, 4, BF16>), grid,
+                         dim3(512), 0, stream, Q, K, V, Op, lse, geo, um, c);
       break;
     case kPingPong4:
       if constexpr (D == 64) {
         hipLaunchKernelGGL((fa_fwd_pp_kernel<D, CAUSAL, WRITE_L, FULL, 8, BF16, false, 4>),
-                           dim3(total), dim3(512), 0, stream, Q, K, V, Op, lse, geo, num_qb, total, c);
+                           grid, dim3(512), 0, stream, Q, K, V, Op, lse, geo, um, c);
         break;
       }
       return hipErrorInvalidValue;
@@ -831,18 +860,14 @@ static hipError_t launch_fwd(const void* q, const void* k, const void* v, void* 
 
 template <int D, bool CAUSAL, bool BF16>
 static hipError_t dispatch_wl(const void* q, const void* k, const void* v, void* o,
-                              float* lse, Geom geo, int num_qb, int total, float c, bool full,
+                              float* lse, const Geom& geo, const UnitMap& um, float c, bool full,
                               int variant, hipStream_t s) {
   if (lse) {
-    return full ? launch_fwd<D, CAUSAL, true, true, BF16>(q, k, v, o, lse, geo, num_qb, total, c,
-                                                          variant, s)
-                : launch_fwd<D, CAUSAL, true, false, BF16>(q, k, v, o, lse, geo, num_qb, total, c,
-                                                           variant, s);
+    return full ? launch_fwd<D, CAUSAL, true, true, BF16>(q, k, v, o, lse, geo, um, c, variant, s)
+                : launch_fwd<D, CAUSAL, true, false, BF16>(q, k, v, o, lse, geo, um, c, variant, s);
   }
-  return full ? launch_fwd<D, CAUSAL, false, true, BF16>(q, k, v, o, lse, geo, num_qb, total, c,
-                                                         variant, s)
-              : launch_fwd<D, CAUSAL, false, false, BF16>(q, k, v, o, lse, geo, num_qb, total, c,
-                                                          variant, s);
+  return full ? launch_fwd<D, CAUSAL, false, true, BF16>(q, k, v, o, lse, geo, um, c, variant, s)
+              : launch_fwd<D, CAUSAL, false, false, BF16>(q, k, v, o, lse, geo, um, c, variant, s);
 }
 
 // The kernel the forward runs for a problem shape (bh = B * H heads of N
@@ -869,28 +894,35 @@ namespace fa {
 // The forward over a head geometry with an explicit kernel variant (0: the
 // default choice). Arguments are already validated.
 static int fwd_run(const void* q, const void* k, const void* v, void* o, float* lse,
-                   const Geom& geo_in, int64_t B, int64_t D, int causal, int variant, void* stream,
+                   const Geom& geo, int64_t B, int64_t D, int causal, int variant, void* stream,
                    bool bf16 = false) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const Topology topo = stream_topology(s);
-  Geom geo = geo_in;
-  geo.nxcd = topo.xcds;
   // kGuarded + v: variant v through its guarded instance even where N is a
   // multiple of the row block (tests compare it bitwise with the full-tile one).
   const bool guarded = variant >= kGuarded;
   if (guarded) variant -= kGuarded;
-  if (variant == 0) variant = choose_variant(D, causal, B * geo.H, geo.N, topo.cus);
+  if (variant == 0) {
+    // A ragged batch: by the bound on its row blocks (its rows are no single
+    // wave of one length).
+    variant = geo.cu == nullptr
+                  ? choose_variant(D, causal, B * geo.H, geo.N, topo.cus)
+                  : choose_variant(D, 0, geo.H * varlen_units(B, geo.total, geo.N, kBR), kBR, topo.cus);
+  }
   if (!variant_fits((int)D, variant, causal)) return FA_ERR_HEAD_DIM;
   const int rows = variant_rows(variant);
-  const int num_qb = (geo.N + rows - 1) / rows;
+  // Units of a head: its row blocks (varlen: a bound on those of its sequences).
+  const int64_t per_head = geo.cu == nullptr ? (geo.N + rows - 1) / rows
+                                             : varlen_units(B, geo.total, geo.N, rows);
+  const int64_t heads = geo.cu == nullptr ? B * geo.H : geo.H;
   // The validation bounds the grid of 128-row blocks; 64-row blocks double it.
-  if (B * geo.H * (int64_t)num_qb > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
-  const int total = (int)(B * geo.H * num_qb);   // workgroups
+  if (heads * per_head > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
+  const UnitMap um = unit_map(heads, per_head, topo, causal != 0 || geo.cu != nullptr);
   const float c = (float)(1.0 / sqrt((double)D)) * kLog2e;
   const bool full = !guarded && geo.cu == nullptr && (geo.N % variant_full_n(variant)) == 0;
   hipError_t e;
 #define FA_FWD_DISPATCH(DD, CC, BB) \
-  dispatch_wl<DD, CC, BB>(q, k, v, o, lse, geo, num_qb, total, c, full, variant, s)
+  dispatch_wl<DD, CC, BB>(q, k, v, o, lse, geo, um, c, full, variant, s)
   if (D == 64) {
     if (bf16) e = causal ? FA_FWD_DISPATCH(64, true, true) : FA_FWD_DISPATCH(64, false, true);
     else e = causal ? FA_FWD_DISPATCH(64, true, false) : FA_FWD_DISPATCH(64, false, false);
@@ -908,7 +940,7 @@ static int fwd_dense(const void* q, const void* k, const void* v, void* o, float
   const int st = fa_validate_fwd_gqa(q, k, v, o, B, H, H_kv, N, D);
   if (st != FA_OK) return st;
   if (lse != nullptr && (reinterpret_cast<uintptr_t>(lse) & 3u) != 0) return FA_ERR_ALIGNMENT;
-  const Geom geo{nullptr, (int)N, (int)H, (int)(H / H_kv), 0, 0, 0};   // nxcd: launcher
+  const Geom geo{nullptr, (int)N, (int)H, FastDiv(H / H_kv), 0, 0};
   return fwd_run(q, k, v, o, lse, geo, B, D, causal, variant, stream);
 }
 }  // namespace fa
@@ -921,11 +953,11 @@ namespace fa {
 // where the row blocks alone leave CUs idle.
 template <int D, bool CAUSAL, bool FULL>
 static hipError_t launch_splitkv(const f16* Q, const f16* K, const f16* V, f16* O, float* L,
-                                 const Geom& geo, int num_qb, int units, float c, float* part_o,
+                                 const Geom& geo, const UnitMap& um, float c, float* part_o,
                                  float* part_lse, int nsplit, int64_t rows, hipStream_t s) {
   hipLaunchKernelGGL((fa_fwd_pp_kernel<D, CAUSAL, true, FULL, 4, false, true>),
-                     dim3(units * nsplit), dim3(512), 0, s, Q, K, V, O, L, geo, num_qb,
-                     units * nsplit, c, part_o, part_lse, nsplit);
+                     dim3(um.heads * um.per_head * nsplit), dim3(512), 0, s, Q, K, V, O, L, geo, um,
+                     c, part_o, part_lse, nsplit);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int st = fa_lse_combine_f32(part_o, part_lse, rows, 1, D, nsplit, O, L, s);
@@ -983,6 +1015,18 @@ extern "C" int fa_probe_choose_variant(int64_t D, int causal, int64_t bh, int64_
   return fa::choose_variant(D, causal, bh, N, cus);
 }
 
+extern "C" int fa_probe_unit_of(int64_t heads, int64_t per_head, int nxcd, int cus, int uneven,
+                                int64_t g, int* head, int* idx) {
+  if (heads <= 0 || per_head <= 0 || nxcd <= 0 || cus <= 0 || heads * per_head > (int64_t(1) << 31) - 1 ||
+      g < 0 || g >= heads * per_head || head == nullptr || idx == nullptr)
+    return FA_ERR_TOO_LARGE;
+  const fa::UnitMap um = fa::unit_map(heads, per_head, fa::Topology{cus, nxcd}, uneven != 0);
+  const fa::Unit u = fa::unit_of((int)g, um);
+  *head = u.head;
+  *idx = u.idx;
+  return FA_OK;
+}
+
 extern "C" int64_t fa_fwd_splitkv_workspace_floats(int64_t B, int64_t H, int64_t N, int64_t D,
                                                    int64_t num_splits) {
   if (B <= 0 || H <= 0 || N <= 0 || (D != 64 && D != 128) || num_splits < 1) return 0;
@@ -1002,8 +1046,7 @@ extern "C" int fa_fwd_splitkv_f16(const void* q, const void* k, const void* v, v
   if (lse != nullptr && (reinterpret_cast<uintptr_t>(lse) & 3u) != 0) return FA_ERR_ALIGNMENT;
   const int64_t num_qb = (N + kBR - 1) / kBR;
   if (B * H * num_qb > (int64_t(1) << 31) / num_splits) return FA_ERR_TOO_LARGE;
-  Geom geo{nullptr, (int)N, (int)H, (int)(H / H_kv), 0, 0, 1};
-  const int units = (int)(B * H * num_qb);
+  const Geom geo{nullptr, (int)N, (int)H, FastDiv(H / H_kv), 0, 0};
   const float c = (float)(1.0 / sqrt((double)D)) * kLog2e;
   const bool full = (N % kBR) == 0;
   const int64_t rows = B * H * N;
@@ -1014,12 +1057,11 @@ extern "C" int fa_fwd_splitkv_f16(const void* q, const void* k, const void* v, v
   const f16* V = (const f16*)v;
   f16* Op = (f16*)o;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  geo.nxcd = stream_topology(s).xcds;
+  const UnitMap um = unit_map(B * H, num_qb, stream_topology(s), false);
   const int ns = (int)num_splits;
-  const int nq = (int)num_qb;
   hipError_t e;
 #define FA_SPLITKV(DD, CC, FF) \
-  launch_splitkv<DD, CC, FF>(Q, K, V, Op, lse, geo, nq, units, c, part_o, part_lse, ns, rows, s)
+  launch_splitkv<DD, CC, FF>(Q, K, V, Op, lse, geo, um, c, part_o, part_lse, ns, rows, s)
   if (D == 64) {
     e = causal ? (full ? FA_SPLITKV(64, true, true) : FA_SPLITKV(64, true, false))
                : (full ? FA_SPLITKV(64, false, true) : FA_SPLITKV(64, false, false));
@@ -1050,8 +1092,8 @@ extern "C" int fa_fwd_varlen_f16(const void* q, const void* k, const void* v, vo
   const int st = fa_validate_fwd_varlen(q, k, v, o, cu_seqlens, B, H, H_kv, max_seqlen, total, D);
   if (st != FA_OK) return st;
   if (lse != nullptr && (reinterpret_cast<uintptr_t>(lse) & 3u) != 0) return FA_ERR_ALIGNMENT;
-  const fa::Geom geo{cu_seqlens, (int)max_seqlen, (int)H, (int)(H / H_kv), (int)total,
-                       (int)B, 0};   // nxcd: launcher
+  const fa::Geom geo{cu_seqlens, (int)max_seqlen, (int)H, fa::FastDiv(H / H_kv), (int)total,
+                     (int)B};
   return fa::fwd_run(q, k, v, o, lse, geo, B, D, causal, 0, stream);
 }
 
@@ -1062,7 +1104,7 @@ extern "C" int fa_fwd_bf16(const void* q, const void* k, const void* v, void* o,
   const int st = fa_validate_fwd_gqa(q, k, v, o, B, H, H_kv, N, D);
   if (st != FA_OK) return st;
   if (lse != nullptr && (reinterpret_cast<uintptr_t>(lse) & 3u) != 0) return FA_ERR_ALIGNMENT;
-  const Geom geo{nullptr, (int)N, (int)H, (int)(H / H_kv), 0, 0, 0};   // nxcd: launcher
+  const Geom geo{nullptr, (int)N, (int)H, FastDiv(H / H_kv), 0, 0};
   // The fp16 path's kernel choice for the shape, with bf16 operands.
   return fwd_run(q, k, v, o, lse, geo, B, D, causal, 0, stream, true);
 }

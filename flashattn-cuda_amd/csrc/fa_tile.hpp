@@ -310,6 +310,24 @@ __device__ __forceinline__ f16x8 pack_px(const f32x16& p, int half_sel) {
   return f16x8{x0[0], x0[1], x1[0], x1[1], x2[0], x2[1], x3[0], x3[1]};
 }
 
+// Division of 0 <= n < 2^31 by a launch constant d >= 1: n * ceil(2^(31+s) / d)
+// >> (31+s) with 2^s >= d (the rounding adds less than 2^s to the numerator's
+// 2^(31+s), so the quotient is exact). A few scalar instructions where a
+// division by a kernel argument takes about forty vector ones; a workgroup's
+// address waits for several (B1 H8 N1024 D64: 8.39 -> 8.54 us with plain
+// divisions in unit_of).
+struct FastDiv {
+  uint32_t d, mul, shift;
+  FastDiv() = default;
+  explicit FastDiv(int64_t divisor) : d((uint32_t)divisor), shift(31) {
+    while ((uint64_t(1) << (shift - 31)) < d) ++shift;
+    mul = (uint32_t)(((uint64_t(1) << shift) + d - 1) / d);
+  }
+  __host__ __device__ __forceinline__ int div(int n) const {
+    return (int)(((uint64_t)(uint32_t)n * mul) >> shift);
+  }
+};
+
 // Where the heads of one launch live. Dense: Q/O [B, H, N, D], K/V
 // [B, H/group, N, D], L [B, H, N]. Varlen (cu != nullptr): sequences packed
 // head-major, Q/O [H, total, D], K/V [H/group, total, D], L [H, total];
@@ -319,22 +337,74 @@ struct Geom {
   const int32_t* cu;
   int N;
   int H;
-  int group;
+  FastDiv group;
   int total;
   int B;       // varlen: number of sequences
-  int nxcd;    // XCDs of the device the launch runs on (set by the launcher)
 };
 
 // Workgroup g of a 1-D grid of `total` lands on XCD g % nxcd (the dispatcher
 // deals consecutive workgroups to the XCDs in turn). Map it to a logical index
-// so that each XCD gets one contiguous range of logical indices: the row
-// blocks of a head then share one XCD's L2, which serves their K/V after the
-// first fetch. nxcd <= 1 (one XCD, or a partition of one) is the identity.
+// so that each XCD gets one contiguous range of logical indices: the units of
+// a row block then share one XCD's L2, which serves their K/V after the first
+// fetch. nxcd <= 1 (one XCD, or a partition of one) is the identity.
 __device__ __forceinline__ int xcd_remap(int g, int total, int nxcd) {
   if (nxcd <= 1) return g;
   const int q = total / nxcd, r = total % nxcd;
   const int xcd = g % nxcd, slot = g / nxcd;
   return (xcd < r) ? xcd * (q + 1) + slot : r * (q + 1) + (xcd - r) * q + slot;
+}
+
+// The units of a launch: `heads` heads of `per_head` units, unit 0 of a head
+// the longest where lengths differ. One workgroup per unit. See unit_of and,
+// for the fields, unit_map.
+struct UnitMap {
+  int heads, per_head;
+  FastDiv nxcd;
+  int whole;             // whole heads of an XCD
+  FastDiv rem;           // heads that do not divide over the XCDs (at least 1)
+  int dealt;             // their units
+  FastDiv set_units;     // units of a set of heads an XCD works on at a time
+  FastDiv width, last;   // heads of a set, and of the last one
+  int sets;
+};
+
+struct Unit {
+  int head, idx;
+};
+
+// The unit of workgroup g. Workgroup g runs on XCD g % nxcd, and each XCD
+// starts its workgroups in order, so this decides what shares an L2 and what
+// is left for the end:
+//   * an XCD gets heads / nxcd whole heads (their K/V then live in its L2),
+//     `merge` of them at a time, level by level: unit i of each of them before
+//     unit i + 1 of any. The longest units of several heads start first and
+//     the short ones fill the end; one head after the other leaves the last
+//     head's long units to a few CUs.
+//   * heads that do not divide over the XCDs are dealt out unit by unit,
+//     first. A contiguous half of a causal head would give one XCD the long
+//     half of the triangle and its neighbour the short one, 3 : 1.
+// A permutation of the units for every argument.
+__host__ __device__ __forceinline__ Unit unit_of(int g, const UnitMap& m) {
+  const int nx = (int)m.nxcd.d;
+  int s = m.nxcd.div(g);
+  const int x = g - s * nx;
+  Unit u;
+  if (m.dealt > 0) {
+    const int mine = m.nxcd.div(m.dealt + nx - 1 - x);   // this XCD's share of them
+    if (s < mine) {
+      const int v = s * nx + x;
+      u.idx = m.rem.div(v);
+      u.head = m.whole * nx + (v - u.idx * (int)m.rem.d);
+      return u;
+    }
+    s -= mine;
+  }
+  const int set = m.set_units.div(s);
+  s -= set * (int)m.set_units.d;
+  const FastDiv& w = set + 1 < m.sets ? m.width : m.last;
+  u.idx = w.div(s);
+  u.head = x * m.whole + set * (int)m.width.d + (s - u.idx * (int)w.d);
+  return u;
 }
 
 // Compute units and XCDs of a device: read once per device from the runtime
@@ -372,35 +442,184 @@ inline Topology stream_topology(hipStream_t stream) {
   return device_topology(dev);
 }
 
+// Inclusive scan over the wave's 64 lanes of x >= 0 (DPP row shifts and row
+// broadcasts): op is + or max; lanes without a source see 0.
+template <typename Op>
+__device__ __forceinline__ int wave_scan(int x, Op op) {
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));   // row_shr:1
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));   // row_shr:2
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));   // row_shr:4
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));   // row_shr:8
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));   // row_bcast:15
+  x = op(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));   // row_bcast:31
+  return x;
+}
+
+__device__ __forceinline__ int scan_sum(int x) {
+  return wave_scan(x, [](int a, int b) { return a + b; });
+}
+
+__device__ __forceinline__ int scan_max(int x) {
+  return wave_scan(x, [](int a, int b) { return max(a, b); });
+}
+
+// Bounds read from cu are clamped into [0, total], so a malformed table never
+// moves a head's buffer range outside its own rows.
+__device__ __forceinline__ int clamp_row(int r, int total) { return min(max(r, 0), total); }
+
+// Batches of up to kCountedSeqs sequences have their units counted (varlen_block).
+constexpr int kCountedSeqs = 512;
+
+// Blocks of `rows` rows per head in a varlen grid: sequence b has
+// ceil(n_b / rows) of them, and the host knows only that the n_b are at most
+// max_seqlen and sum to at most `total`.
+inline int64_t varlen_units(int64_t B, int64_t total, int64_t max_seqlen, int rows) {
+  const int64_t by_max = B * ((max_seqlen + rows - 1) / rows);
+  const int64_t by_total = total / rows + B;
+  return B > kCountedSeqs || by_max < by_total ? by_max : by_total;
+}
+
+struct SeqBlock {
+  int start, n;   // rows of the sequence; n = 0: there is no such unit
+  int block;
+};
+
+// Unit u of a head's varlen units: the blocks of the sequences longer than half
+// of max_seqlen, sequence by sequence, then those of the others. The short
+// sequences then fill the end of the launch, and an XCD works through one or
+// two sequences at a time (units of equal length of all sequences together
+// keep more K/V in use than an L2 holds). `block` counts from 0 within the
+// sequence. Every wave finds it from two wave scans of the block counts (lane l
+// takes sequences l, l + 64, ...). A full sort by length, with a binary search
+// for the length of unit u, cost a workgroup over 1 us and 4-6 % of a launch
+// with sequences of 2048 rows.
+// Sequence b + 1 starts no earlier than sequence b ends, also where cu
+// decreases, so the units never exceed varlen_units().
+template <int J>
+__device__ __forceinline__ SeqBlock counted_block(const Geom& g, int u, int rows, int lane) {
+  const int half = ((g.N + rows - 1) / rows) / 2;
+  int c0[J], c1[J];
+  bool falls = false;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int b = 64 * j + lane;
+    c0[j] = c1[j] = 0;
+    if (b < g.B) {
+      c0[j] = clamp_row(g.cu[b], g.total);
+      c1[j] = clamp_row(g.cu[b + 1], g.total);
+      falls |= c1[j] < c0[j];
+    }
+  }
+  if (__any(falls)) {   // malformed: from the running maximum on
+    int end = 0;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      c0[j] = scan_max(max(c0[j], end));
+      c1[j] = max(c0[j], c1[j]);
+      end = __builtin_amdgcn_readlane(c1[j], 63);
+    }
+  }
+  int n[J], big[J], small[J];   // blocks; their scans over the two kinds
+  int nbig = 0, nsmall = 0;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    n[j] = (min(c1[j] - c0[j], g.N) + rows - 1) / rows;
+    big[j] = nbig + scan_sum(n[j] > half ? n[j] : 0);
+    small[j] = nsmall + scan_sum(n[j] > half ? 0 : n[j]);
+    nbig = __builtin_amdgcn_readlane(big[j], 63);
+    nsmall = __builtin_amdgcn_readlane(small[j], 63);
+  }
+  const bool in_big = u < nbig;
+  const int v = in_big ? u : u - nbig;
+  SeqBlock out{0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int sum = in_big ? big[j] : small[j];
+    const uint64_t m = __ballot((n[j] > half) == in_big && sum > v);
+    if (m != 0 && out.n == 0) {
+      const int l = __ffsll((unsigned long long)m) - 1;
+      out.start = __builtin_amdgcn_readlane(c0[j], l);
+      out.n = min(__builtin_amdgcn_readlane(c1[j], l) - out.start, g.N);
+      out.block = v - (__builtin_amdgcn_readlane(sum, l) - __builtin_amdgcn_readlane(n[j], l));
+    }
+  }
+  return out;
+}
+
+__device__ __forceinline__ SeqBlock varlen_block(const Geom& g, int u, int rows, int lane) {
+  if (g.B <= 64) return counted_block<1>(g, u, rows, lane);
+  if (g.B <= 256) return counted_block<4>(g, u, rows, lane);
+  if (g.B <= kCountedSeqs) return counted_block<kCountedSeqs / 64>(g, u, rows, lane);
+  const int nbmax = (g.N + rows - 1) / rows;   // more: sequence by sequence
+  const int b = u / nbmax, i = u - b * nbmax;
+  const int s0 = clamp_row(g.cu[b], g.total);
+  const int s1 = max(s0, clamp_row(g.cu[b + 1], g.total));
+  const int n = min(s1 - s0, g.N);
+  return i * rows < n ? SeqBlock{s0, n, i} : SeqBlock{0, 0, 0};
+}
+
+// The map of heads * per_head units onto `topo`. Units of one length run head
+// by head: the K/V of one head then fill the L2. `uneven` ones (causal,
+// ragged) run in sets of as many heads as give every CU of an XCD a unit (a
+// head of 32 blocks alone on MI355X), so that each set's short units meet the
+// next set's long ones; wider sets only take more of the L2 (B4 H16 N4096 D128
+// causal forward: 303 us with sets of one head, 314 with sets of two).
+// Measured, one contiguous range of the head-by-head order per XCD before ->
+// now: bf16 causal forward and cache write of B2 H32 (8 KV heads) N1777 D128,
+// 14 blocks a head, 78.5 -> 72.5 us; bf16 causal backward B1 H32 (8) N2000
+// D128 210 -> 187 us; 12 ragged sequences of up to 4096 rows, H8 D64 causal,
+// forward and backward 702 -> 686 us; 60 of up to 400 rows, forward 50 -> 34
+// us, backward 150 -> 101 us (fewer empty workgroups).
+inline UnitMap unit_map(int64_t heads, int64_t per_head, const Topology& topo, bool uneven) {
+  const int64_t nx = topo.xcds > 1 ? topo.xcds : 1;
+  const int64_t whole = heads / nx, rem = heads % nx;
+  int64_t sets = whole > 0 ? whole : 1;
+  if (uneven && whole > 1 && per_head > 0) {
+    const int64_t cus = (topo.cus + nx - 1) / nx;
+    const int64_t want = (cus + per_head - 1) / per_head;
+    sets = whole / want > 1 ? whole / want : 1;
+  }
+  const int64_t width = whole > 0 ? (whole + sets - 1) / sets : 1;   // sets of about equal width
+  sets = whole > 0 ? (whole + width - 1) / width : 1;
+  UnitMap m;
+  m.heads = (int)heads;
+  m.per_head = (int)per_head;
+  m.nxcd = FastDiv(nx);
+  m.whole = (int)whole;
+  m.rem = FastDiv(rem > 0 ? rem : 1);
+  m.dealt = (int)(rem * per_head);
+  m.set_units = FastDiv(width * per_head > 0 ? width * per_head : 1);
+  m.width = FastDiv(width);
+  m.last = FastDiv(whole > 0 ? whole - (sets - 1) * width : 1);
+  m.sets = (int)sets;
+  return m;
+}
+
 // One (b, h): element offsets of its Q/O and K/V rows, of its L row, and its
-// length. Varlen bounds are clamped into [0, total] and to N, so a malformed
-// cu never moves a head's buffer range outside its own rows.
+// length.
 struct HeadView {
   size_t q, kv, l;
   int n;
 };
 
+// Head bh of a dense launch, or head h of sequence b of a packed one.
 template <int D>
-__device__ __forceinline__ HeadView head_view(const Geom& g, int bh) {
+__device__ __forceinline__ HeadView dense_view(const Geom& g, int bh) {
   HeadView v;
-  if (g.cu == nullptr) {
-    v.n = g.N;
-    v.q = (size_t)bh * g.N * D;
-    v.kv = (size_t)(bh / g.group) * g.N * D;
-    v.l = (size_t)bh * g.N;
-  } else {
-    // Head-major unit order (h, then b): the grid is cut into one contiguous
-    // range per XCD, and a range of whole heads holds every sequence's share
-    // of the work, where a range of whole sequences would give one XCD all of
-    // a long sequence.
-    const int h = bh / g.B, b = bh - h * g.B;
-    const int s0 = min(max(g.cu[b], 0), g.total);
-    const int s1 = min(max(g.cu[b + 1], s0), g.total);
-    v.n = min(s1 - s0, g.N);
-    v.q = ((size_t)h * g.total + s0) * D;
-    v.kv = ((size_t)(h / g.group) * g.total + s0) * D;
-    v.l = (size_t)h * g.total + s0;
-  }
+  v.n = g.N;
+  v.q = (size_t)bh * g.N * D;
+  v.kv = (size_t)g.group.div(bh) * g.N * D;
+  v.l = (size_t)bh * g.N;
+  return v;
+}
+
+template <int D>
+__device__ __forceinline__ HeadView seq_view(const Geom& g, int h, int start, int n) {
+  HeadView v;
+  v.n = n;
+  v.q = ((size_t)h * g.total + start) * D;
+  v.kv = ((size_t)g.group.div(h) * g.total + start) * D;
+  v.l = (size_t)h * g.total + start;
   return v;
 }
 

@@ -19,7 +19,7 @@
 
 #include <stdint.h>
 
-#define FA_PROBE_VERSION 4
+#define FA_PROBE_VERSION 5
 
 #ifdef __cplusplus
 extern "C" {
@@ -77,6 +77,14 @@ int fa_probe_choose_variant(int64_t D, int causal, int64_t bh, int64_t N, int cu
 /* fa_fwd_splitkv_plan for a device of `cus` compute units instead of the
  * current device's. No device needed. */
 int fa_probe_splitkv_plan_cus(int64_t B, int64_t H, int64_t N, int64_t D, int causal, int cus);
+
+/* The unit (head, and index within the head, 0 the longest where lengths
+ * differ) that workgroup g of a launch of heads * per_head units runs on a
+ * device of `cus` compute units in `nxcd` XCDs; `uneven`: the units differ in
+ * length (causal or ragged). FA_ERR_TOO_LARGE for a bad argument. No device
+ * needed. */
+int fa_probe_unit_of(int64_t heads, int64_t per_head, int nxcd, int cus, int uneven, int64_t g,
+                     int* head, int* idx);
 
 /* Writes up to max_out variant codes that exist for head dimension D and the
  * causal flag into out (may be NULL) and returns how many there are. */

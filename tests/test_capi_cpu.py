@@ -368,3 +368,29 @@ def test_kernel_and_split_choice_follow_the_cu_count(capi):
     assert plan(1, 8, 2048, 128, 1, 256) == 1      # 128 blocks, 32 tiles: 2 splits lose
     assert plan(1, 3, 8192, 128, 1, 256) == 1      # 192 blocks
     assert plan(1, 1, 16384, 64, 1, 256) == 1      # D = 64 never splits
+
+
+@pytest.mark.parametrize("heads,per_head", [(1, 1), (8, 32), (4, 32), (12, 16), (64, 14), (7, 5), (128, 8), (3, 70)])
+@pytest.mark.parametrize("nxcd,cus", [(8, 256), (1, 32)])
+@pytest.mark.parametrize("uneven", [0, 1])
+def test_unit_order(capi, heads, per_head, nxcd, cus, uneven):
+    """The workgroup-to-unit map is a permutation, gives every XCD the same
+    share of long and short units (unit i of a head stands for a length of
+    per_head - i), and keeps whole heads on one XCD."""
+    import ctypes as C
+    lib = capi.load()
+    h, i = C.c_int(), C.c_int()
+    units, load, homes = [], [0] * nxcd, {}
+    for g in range(heads * per_head):
+        assert lib.fa_probe_unit_of(heads, per_head, nxcd, cus, uneven, g, C.byref(h), C.byref(i)) == 0
+        units.append((h.value, i.value))
+        load[g % nxcd] += per_head - i.value
+        homes.setdefault(h.value, set()).add(g % nxcd)
+    assert sorted(units) == [(a, b) for a in range(heads) for b in range(per_head)]
+    # the heads that do not divide over the XCDs are dealt out unit by unit, so
+    # two XCDs differ by at most the steps between neighbouring units
+    assert max(load) - min(load) <= per_head + heads % nxcd
+    whole = heads // nxcd * nxcd
+    assert all(len(homes[a]) == 1 for a in range(whole))
+    bad = lib.fa_probe_unit_of(heads, per_head, nxcd, cus, uneven, heads * per_head, C.byref(h), C.byref(i))
+    assert bad == capi.STATUS["FA_ERR_TOO_LARGE"]

@@ -103,6 +103,49 @@ def test_varlen_forward(fa, dev, D, causal, Hkv):
                tag=f"varlen seq {b} (n={n}) D{D} causal={causal} Hkv{Hkv}")
 
 
+@pytest.mark.parametrize("B", [64, 65, 257, 520])
+@pytest.mark.parametrize("causal", [False, True])
+def test_varlen_many_sequences(fa, dev, B, causal):
+    """Every unit of batches around the widths of the per-wave count of blocks
+    (64 and 256 sequences a pass, at most 512 counted), with empty sequences,
+    one long one last, and a head count that no XCD count divides; forward
+    against the oracle, gradients against the dense backward of the sequence
+    (the same arithmetic on the same tiles: equal bit for bit)."""
+    H, D = 3, 64
+    rng = np.random.default_rng(B)
+    lengths = [int(x) for x in rng.integers(0, 40, B)]
+    lengths[B // 2] = 0
+    lengths[-1] = 300
+    cu = _cu(lengths)
+    q, k, v, g = (torch.from_numpy(_randn((H, int(cu[-1]), D), s)).to(dev).half() for s in (40, 41, 42, 43))
+    tcu = torch.from_numpy(cu).to(dev)
+    O, L = fa.forward_varlen(q, k, v, tcu, 300, causal=causal)
+    grads = fa.backward_varlen(q, k, v, O, g, L, tcu, 300, causal=causal)
+    torch.cuda.synchronize()
+    qn, kn, vn = (x.float().cpu().numpy() for x in (q, k, v))
+    for b, n in enumerate(lengths):
+        if n == 0:
+            continue
+        s = slice(int(cu[b]), int(cu[b + 1]))
+        Or, Lr = naive_attention(qn[None, :, s], kn[None, :, s], vn[None, :, s], causal=causal)
+        _check(O[None, :, s], L[None, :, s], Or, Lr, tag=f"varlen {B} seqs, seq {b} (n={n}) causal={causal}")
+        if b % 37 == 0 or b == B - 1:
+            one = [x[None, :, s].contiguous() for x in (q, k, v, O, g, L)]
+            for x, r in zip(grads, fa.backward(*one, causal=causal)):
+                assert torch.equal(x[:, s], r[0]), f"seq {b} (n={n})"
+
+
+def test_varlen_decreasing_bounds(fa, dev):
+    """A table that falls counts as its running maximum: what it did compute
+    stays computed, and no row is computed twice."""
+    H, D, total = 2, 64, 300
+    q, k, v = (torch.from_numpy(_randn((H, total, D), s)).to(dev).half() for s in (44, 45, 46))
+    bad = torch.tensor([0, 250, 100, 10_000], dtype=torch.int32, device=dev)
+    good = torch.tensor([0, 250, 250, 300], dtype=torch.int32, device=dev)
+    for x, r in zip(fa.forward_varlen(q, k, v, bad, 256), fa.forward_varlen(q, k, v, good, 256)):
+        assert torch.equal(x, r)
+
+
 def test_varlen_single_sequence_matches_dense(fa, dev):
     H, N, D = 2, 512, 64
     q, k, v = (_randn((H, N, D), s) for s in (10, 11, 12))
