@@ -457,14 +457,13 @@ torch::Tensor kv_append(torch::Tensor k_new, torch::Tensor v_new, torch::Tensor 
                   (!nl.defined() || nl.device() == dev),
               "kv_append tensors must be on the same device");
   const c10::DeviceGuard guard(dev);
-  auto bad = torch::zeros({B}, page_table.options());
-  const bool bf16 = k_new.scalar_type() == torch::kBFloat16;
-  const auto fn = bf16 ? fa_kv_append_bf16 : fa_kv_append_f16;
-  const int st = fn(k_new.data_ptr(), v_new.data_ptr(), page_table.data_ptr<int32_t>(),
-                    start_pos.data_ptr<int32_t>(), lens, k_pool.data_ptr(), v_pool.data_ptr(),
-                    bad.data_ptr<int32_t>(), B, H, T, D, k_pool.size(2), page_table.size(1),
-                    k_pool.size(0), current_stream(k_new));
-  check_status(st, bf16 ? "fa_kv_append_bf16" : "fa_kv_append_f16");
+  auto bad = torch::empty({B}, page_table.options());
+  const int st = fa_kv_append_set_bad(
+      k_new.data_ptr(), v_new.data_ptr(), page_table.data_ptr<int32_t>(),
+      start_pos.data_ptr<int32_t>(), lens, k_pool.data_ptr(), v_pool.data_ptr(),
+      bad.data_ptr<int32_t>(), B, H, T, D, k_pool.size(2), page_table.size(1), k_pool.size(0),
+      current_stream(k_new));
+  check_status(st, k_new.scalar_type() == torch::kBFloat16 ? "fa_kv_append_bf16" : "fa_kv_append_f16");
   return bad;
 }
 

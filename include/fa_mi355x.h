@@ -275,7 +275,12 @@ int fa_lse_combine_f32(const float* part_o, const float* part_lse,
                        int64_t B, int64_t H, int64_t D, int64_t num_splits,
                        void* o, float* lse, void* stream);
 
-/* Split pass then combine pass, both on `stream`. No reference counterpart. */
+/*
+ * O and L of the paged decode: split pass then combine pass, both on `stream`.
+ * num_splits is the most splits used (fewer where that is faster, by the sizes
+ * and the device; one split needs no combine pass), and part_o / part_lse are
+ * workspace for that many. No reference counterpart.
+ */
 int fa_decode_paged_f16(const void* q, const void* k_pool, const void* v_pool,
                         const int32_t* page_table, const int32_t* ctx_lens,
                         int64_t B, int64_t H, int64_t D, int64_t page_size,
@@ -371,6 +376,16 @@ int fa_kv_append_bf16(const void* k_new, const void* v_new, const int32_t* page_
                       const int32_t* start_pos, const int32_t* new_lens, void* k_pool,
                       void* v_pool, int32_t* bad, int64_t B, int64_t H, int64_t T, int64_t D,
                       int64_t page_size, int64_t max_pages, int64_t num_pages, void* stream);
+
+/*
+ * fa_kv_append_f16 / fa_kv_append_bf16 (rows and pools of the same 16-bit
+ * type) that writes every bad[b], 0 or 1, itself: `bad` is required and need
+ * not be cleared. No reference counterpart.
+ */
+int fa_kv_append_set_bad(const void* k_new, const void* v_new, const int32_t* page_table,
+                         const int32_t* start_pos, const int32_t* new_lens, void* k_pool,
+                         void* v_pool, int32_t* bad, int64_t B, int64_t H, int64_t T, int64_t D,
+                         int64_t page_size, int64_t max_pages, int64_t num_pages, void* stream);
 
 #ifdef __cplusplus
 }

@@ -189,3 +189,21 @@ def test_decode_agrees_with_causal_forward(fa, dev, D, Hkv):
         d_l = ((Ld - L[:, :, t]).abs() / L[:, :, t].abs().clamp(min=1)).max().item()
         assert d_o <= 4e-3, f"t {t}: O differs by {d_o:.2e}"
         assert d_l <= 1e-4, f"t {t}: L differs by {d_l:.2e}"
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("T", [0, 1, 40, 5000])
+def test_bad_flags_written_over_stale_memory(fa, dev, D, T):
+    """bad is 0 or 1 for every sequence whatever its memory held: good, an
+    invalid id on the last page, a position past the table, a negative start, no new tokens."""
+    B, H, P = 5, 2, 400
+    k = torch.randn(B, H, T, D, device=dev, dtype=torch.half)
+    pool = torch.zeros(2, P * B, H, 16, D, device=dev, dtype=torch.half)
+    table = torch.arange(P * B, dtype=torch.int32, device=dev).reshape(B, P).contiguous()
+    table[1, max(T - 1, 0) // 16] = P * B
+    start = torch.tensor([0, 0, 16 * P - 20, -1, 16 * P], dtype=torch.int32, device=dev)
+    lens = torch.tensor([T, T, T, T, 0], dtype=torch.int32, device=dev)
+    stale = [torch.full((B,), 7, dtype=torch.int32, device=dev) for _ in range(4)]
+    del stale   # the caching allocator hands one of these blocks out next
+    bad = fa.kv_append(k, k, pool[0], pool[1], table, start, lens)
+    assert bad.tolist() == [0, int(T > 0), int(T > 20), int(T > 0), 0]
