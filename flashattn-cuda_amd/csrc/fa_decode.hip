@@ -10,17 +10,18 @@
 // page are 16*D*2 contiguous bytes (4 KiB at D=128), copied into LDS as
 // contiguous 1 KiB requests.
 //
-// Split kernel: one workgroup (4 waves) per (split, KV head, up to 16 query
-// heads of its group, sequence); wave w walks pages p0+w, p0+w+4, ... and
+// Split kernel: one workgroup (W = 4 or 8 waves) per (split, KV head, up to 16
+// query heads of its group, sequence); wave w walks pages p0+w, p0+w+W, ... and
 // computes the scores of every head of the workgroup and their PV products
 // on the matrix cores, so a page is read once per KV head. Each wave keeps
-// its own running max/sum and fp32 partial output per head; the four waves
-// merge through LDS at the end.
+// its own running max/sum and fp32 partial output per head; the waves merge
+// through LDS at the end. With one split the kernel writes O and L itself.
 #include <hip/hip_runtime.h>
 
 #include <math.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "fa_mi355x.h"
@@ -29,8 +30,7 @@
 namespace fa {
 
 constexpr int kPage = 16;
-constexpr int kDecThreads = 256;
-constexpr int kDecWaves = kDecThreads / 64;
+constexpr int kRankSeqs = 256;   // batches up to this size are ordered by length
 
 // Element types of q, the pools and O: fp16, or bf16 (BF16 = true). The
 // matrix products take them as 16-bit operands with fp32 accumulation; P is
@@ -51,12 +51,12 @@ struct DecT<true> {
 // is dispatched first) takes the sequence of rank z by decreasing
 // context length, ties by index. The longest splits then start first and the
 // shortest fill the tail instead of a long sequence dispatched last running
-// alone. Ranks of B <= kDecThreads contexts are computed from a copy in LDS;
+// alone. Ranks of B <= kRankSeqs contexts are computed from a copy in LDS;
 // larger batches keep the identity order. Invalid (negative) lengths rank
 // like any other value and are flagged by the caller as before.
 __device__ __forceinline__ int sequence_of_rank(const int32_t* __restrict__ ctx_lens, int B, int z,
                                                 int* sh_ctx, int* sh_seq) {
-  if (B > kDecThreads) return z;
+  if (B > kRankSeqs || B == 1) return z;
   const int t = threadIdx.x;
   if (t < B) sh_ctx[t] = ctx_lens[t];
   __syncthreads();
@@ -73,7 +73,7 @@ __device__ __forceinline__ int sequence_of_rank(const int32_t* __restrict__ ctx_
   return *sh_seq;
 }
 
-// Split kernel, on the matrix cores: one workgroup (4 waves) per (split, KV
+// Split kernel, on the matrix cores: one workgroup (W waves) per (split, KV
 // head, up to 16 of the query heads that share it, sequence). A wave copies each
 // page's K and V rows of the KV head into LDS (1 KiB per copy instruction,
 // contiguous in the pool, non-temporal), then
@@ -144,27 +144,29 @@ __device__ __forceinline__ float sum_cols(float x) {   // sum over the 4 lane gr
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-template <int D, bool BF16>
-__global__ void __launch_bounds__(kDecThreads)
+template <int D, bool BF16, int W>
+__global__ void __launch_bounds__(64 * W)
 fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
                        const typename DecT<BF16>::e* __restrict__ kpool,
                        const typename DecT<BF16>::e* __restrict__ vpool,
                        const int32_t* __restrict__ page_table,
                        const int32_t* __restrict__ ctx_lens, float* __restrict__ part_o,
-                       float* __restrict__ part_lse, int H, int Hkv, int max_pages,
-                       int num_pages, int S, float c) {
+                       float* __restrict__ part_lse, typename DecT<BF16>::e* __restrict__ o_out,
+                       float* __restrict__ lse_out, int H, int Hkv, int max_pages,
+                       int num_pages, int S, int ordered, float c) {
   using T = DecT<BF16>;
+  static_assert(64 * W >= kRankSeqs, "one thread per ranked sequence");
   constexpr int PAGE = kPage * D * 2;   // bytes of one head's page
   constexpr int CPR = D / 8;            // 16-byte chunks per token row
   constexpr int KB = D / 32;            // k-steps of S = K Q^T
   constexpr int DB = D / 16;            // 16-column blocks of O^T
   constexpr int NC = PAGE / 1024;       // 1 KiB copies per page and pool
-  static_assert(kDecWaves * 16 * D * 4 <= kDecWaves * 4 * PAGE, "merge area within the slots");
-  __shared__ __attribute__((aligned(1024))) char smem[kDecWaves * 4 * PAGE];
-  __shared__ float sh_m[kDecWaves][16];
-  __shared__ float sh_l[kDecWaves][16];
+  static_assert(W * 16 * D * 4 <= W * 4 * PAGE, "merge area within the slots");
+  __shared__ __attribute__((aligned(1024))) char smem[W * 4 * PAGE];
+  __shared__ float sh_m[W][16];
+  __shared__ float sh_l[W][16];
   __shared__ int sh_bad;
-  __shared__ int sh_ctx[kDecThreads];
+  __shared__ int sh_ctx[kRankSeqs];
   __shared__ int sh_seq;
 
   const int s = blockIdx.x;
@@ -173,7 +175,8 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   const int hk = blockIdx.y / ngrp;
   const int h0 = hk * group + 16 * (blockIdx.y % ngrp);   // first query head of this workgroup
   const int G = min(16, hk * group + group - h0);
-  const int b = sequence_of_rank(ctx_lens, (int)gridDim.z, (int)blockIdx.z, sh_ctx, &sh_seq);
+  const int b = ordered ? sequence_of_rank(ctx_lens, (int)gridDim.z, (int)blockIdx.z, sh_ctx, &sh_seq)
+                        : (int)blockIdx.z;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int col = lane & 15, grp = lane >> 4;
@@ -216,13 +219,13 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   }
   const uint32_t lds0 = lds_addr(smem) + (uint32_t)(wave * 4 * PAGE);   // this wave's two slots
   const int32_t* pt = page_table + (size_t)b * max_pages;
-  // Page ids of the wave's pages p0 + wave + 4 k, 64 at a time: lane i of
+  // Page ids of the wave's pages p0 + wave + W k, 64 at a time: lane i of
   // pidv holds the id of page k = 64 j + i, read with readlane (a page
   // table load per page would wait for every copy in flight before it).
   int pidv = -1;
   auto page_id = [&](int k) -> int {
     if ((k & 63) == 0) {
-      const int pi = p0 + wave + 4 * (k + lane);
+      const int pi = p0 + wave + W * (k + lane);
       pidv = pi < p1 ? pt[pi] : -1;
     }
     return __builtin_amdgcn_readlane(pidv, k & 63);
@@ -251,8 +254,8 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   int p = p0 + wave;
   int sl = 0, k = 0;
   bool ok = p < p1 && issue(0, 0);
-  for (; p < p1; p += kDecWaves, sl ^= 1, ++k) {
-    const int pn = p + kDecWaves;
+  for (; p < p1; p += W, sl ^= 1, ++k) {
+    const int pn = p + W;
     const bool ok_n = pn < p1 && issue(k + 1, sl ^ 1);
     if (ok_n) wait_vmcnt<2 * NC>(); else wait_vmem();
     if (!ok) { bad = true; ok = ok_n; continue; }
@@ -323,7 +326,7 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   wait_vmem();
   if (bad) sh_bad = 1;
   __syncthreads();
-  float* sh_o = reinterpret_cast<float*>(smem);   // [kDecWaves][16][D]
+  float* sh_o = reinterpret_cast<float*>(smem);   // [W][16][D]
   if (col < G) {
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -334,15 +337,15 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   __syncthreads();
 
   // Thread x merges column x % D of head x / D across the waves.
-  for (int x = tid; x < G * D; x += kDecThreads) {
+  for (int x = tid; x < G * D; x += 64 * W) {
     const int g = x / D, d = x % D;
     float M = sh_m[0][g];
 #pragma unroll
-    for (int w = 1; w < kDecWaves; ++w) M = fmaxf(M, sh_m[w][g]);
+    for (int w = 1; w < W; ++w) M = fmaxf(M, sh_m[w][g]);
     float acc = 0.f, z = 0.f;
     if (M != -INFINITY) {
 #pragma unroll
-      for (int w = 0; w < kDecWaves; ++w) {
+      for (int w = 0; w < W; ++w) {
         const float e = (sh_m[w][g] == -INFINITY) ? 0.f : exp2_hw(sh_m[w][g] - M);
         acc += e * sh_o[(w * 16 + g) * D + d];
         z += e * sh_l[w][g];
@@ -351,79 +354,134 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
     float out = (z > 0.f) ? acc / z : 0.f;
     float lse = (z > 0.f) ? (M + log2_hw(z)) * kLn2 : -INFINITY;
     if (sh_bad) { out = NAN; lse = NAN; }
-    const size_t pidx = ((size_t)b * H + h0 + g) * S + s;
-    part_o[pidx * D + d] = out;
-    if (d == 0) part_lse[pidx] = lse;
+    const size_t bh = (size_t)b * H + h0 + g;
+    if (o_out != nullptr) {   // one split: its partial is the result
+      o_out[bh * D + d] = (typename T::e)out;
+      if (lse_out != nullptr && d == 0) lse_out[bh] = lse;
+    } else {
+      const size_t pidx = bh * S + s;
+      part_o[pidx * D + d] = out;
+      if (d == 0) part_lse[pidx] = lse;
+    }
   }
 }
 
-// One workgroup of D threads per (b, h): thread d merges column d.
+// Combine: D / 4 threads per row (b, h), four columns each. All of a row's
+// loads (its S logsumexps and the thread's S partials) are issued before the
+// first is used, so the pass waits for memory once (a thread per column with
+// loops over S waited three times and more: B1 H32, 16 splits, decode 47.3 ->
+// 43.2 us, B8 28.5 -> 24.5); the sums run in split order.
+constexpr int kMaxSplits = 16;
+constexpr int kCombThreads = 256;
+
 template <int D, bool BF16>
-__global__ void __launch_bounds__(D)
+__global__ void __launch_bounds__(kCombThreads)
 fa_lse_combine_kernel(const float* __restrict__ part_o, const float* __restrict__ part_lse,
-                      typename DecT<BF16>::e* __restrict__ o, float* __restrict__ lse, int S) {
-  const int bh = blockIdx.x;
-  const int d = threadIdx.x;
-  const float* ls = part_lse + (size_t)bh * S;
+                      typename DecT<BF16>::e* __restrict__ o, float* __restrict__ lse, int S,
+                      int rows) {
+  // Element alignment only, as the pointers promise no more (one wide access
+  // all the same: the target takes unaligned ones).
+  typedef typename DecT<BF16>::e e4v __attribute__((ext_vector_type(4)));
+  typedef e4v e4 __attribute__((aligned(2)));
+  typedef f32x4 f4 __attribute__((aligned(4)));
+  constexpr int PER = D / 4;   // threads of a row
+  const int row = blockIdx.x * (kCombThreads / PER) + (int)threadIdx.x / PER;
+  if (row >= rows) return;
+  const int d = 4 * ((int)threadIdx.x % PER);
+  const float* pl = part_lse + (size_t)row * S;
+  const float* po = part_o + (size_t)row * S * D + d;
+  float ls[kMaxSplits];
+  f32x4 ps[kMaxSplits];
+#pragma unroll
+  for (int s = 0; s < kMaxSplits; ++s) {
+    ls[s] = -INFINITY;
+    ps[s] = f32x4{};
+    if (s < S) {
+      ls[s] = pl[s];
+      ps[s] = *reinterpret_cast<const f4*>(po + (size_t)s * D);
+    }
+  }
   float M = -INFINITY;
   bool nan = false;
-  for (int s = 0; s < S; ++s) {
-    const float x = ls[s];
-    nan |= (x != x);
-    M = fmaxf(M, x);
+#pragma unroll
+  for (int s = 0; s < kMaxSplits; ++s) {
+    nan |= (ls[s] != ls[s]);
+    M = fmaxf(M, ls[s]);
   }
-  float out, L;
+  f32x4 out = f32x4{};
+  float L;
   if (nan) {
-    out = NAN;
+    out = f32x4{NAN, NAN, NAN, NAN};
     L = NAN;
   } else if (M == -INFINITY) {
-    out = 0.f;
     L = -INFINITY;
   } else {
     float z = 0.f;
-    for (int s = 0; s < S; ++s) z += exp2_hw((ls[s] - M) * kLog2e);
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s)
+      if (s < S) z += exp2_hw((ls[s] - M) * kLog2e);
     L = M + log2_hw(z) * kLn2;
-    float acc = 0.f;
-    const float* po = part_o + (size_t)bh * S * D + d;
-    for (int s = 0; s < S; ++s) {
-      const float w = exp2_hw((ls[s] - L) * kLog2e);
-      acc = fmaf(w, po[(size_t)s * D], acc);
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s) {
+      if (s < S) {
+        const float w = exp2_hw((ls[s] - L) * kLog2e);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = fmaf(w, ps[s][i], out[i]);
+      }
     }
-    out = acc;
   }
-  o[(size_t)bh * D + d] = (typename DecT<BF16>::e)out;
-  if (lse != nullptr && d == 0) lse[bh] = L;
+  e4v v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = (typename DecT<BF16>::e)out[i];
+  *reinterpret_cast<e4*>(o + (size_t)row * D + d) = v;
+  if (lse != nullptr && d == 0) lse[row] = L;
 }
 
 }  // namespace fa
 
 namespace fa {
 // Split pass with query heads h reading pool head h / (H / Hkv); arguments
-// already validated.
+// already validated. With o (num_splits 1) the kernel writes the result
+// itself and the partials are not used.
 template <bool BF16>
 static int decode_split(const void* q, const void* k_pool, const void* v_pool,
                         const int32_t* page_table, const int32_t* ctx_lens, int64_t B, int64_t H,
                         int64_t Hkv, int64_t D, int64_t max_pages, int64_t num_pages,
-                        int64_t num_splits, float* part_o, float* part_lse, void* stream) {
+                        int64_t num_splits, float* part_o, float* part_lse, void* o, float* lse,
+                        void* stream) {
   using E = typename DecT<BF16>::e;
-  if (!part_o || !part_lse) return FA_ERR_NULL_POINTER;
+  if (o == nullptr && (!part_o || !part_lse)) return FA_ERR_NULL_POINTER;
   const float c = (float)(1.0 / sqrt((double)D)) * kLog2e;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const E* Q = (const E*)q;
-  const E* Kp = (const E*)k_pool;
-  const E* Vp = (const E*)v_pool;
+  const int cus = stream_topology(s).cus;
   // One workgroup per (split, KV head, 16 of its query heads, sequence).
   const int64_t group = H / Hkv;
   const dim3 grid((unsigned)num_splits, (unsigned)(Hkv * ((group + 15) / 16)), (unsigned)B);
+  const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
+  // A wave has at most two pages in flight and its loop takes about 0.9 us a
+  // page however idle the chip is, so what a launch reads a second is set by
+  // its waves; LDS holds 8 at D = 128. Where the workgroups do not fill the
+  // CUs twice, eight waves each instead of four (us, 4 -> 8: B1 32 over 8
+  // heads, 32000 tokens, 16 splits 43.2 -> 30.1; B32, 2000 tokens, one split
+  // 44.6 -> 41.0), given a page for each; beyond that the smaller workgroups
+  // overlap their starts and ends better (B32 H32 of 1600 tokens 77.0 vs 71.9).
+  const int64_t pages = (max_pages + num_splits - 1) / num_splits;   // of a split, at most
+  const int W = wgs <= 2 * cus && pages >= 8 ? 8 : 4;
+  // Every workgroup resident at once: their order does not matter.
+  const int ordered = wgs * W > (D == 64 ? 16 : 8) * (int64_t)cus;
+#define FA_DECODE_SPLIT(DD, WW)                                                                    \
+  hipLaunchKernelGGL((fa_decode_split_kernel<DD, BF16, WW>), grid, dim3(64 * WW), 0, s,            \
+                     (const E*)q, (const E*)k_pool, (const E*)v_pool, page_table, ctx_lens, part_o, \
+                     part_lse, (E*)o, lse, (int)H, (int)Hkv, (int)max_pages, (int)num_pages,       \
+                     (int)num_splits, ordered, c)
   if (D == 128) {
-    hipLaunchKernelGGL((fa_decode_split_kernel<128, BF16>), grid, dim3(kDecThreads), 0, s, Q, Kp,
-                       Vp, page_table, ctx_lens, part_o, part_lse, (int)H, (int)Hkv,
-                       (int)max_pages, (int)num_pages, (int)num_splits, c);
+    if (W == 8) FA_DECODE_SPLIT(128, 8);
+    else FA_DECODE_SPLIT(128, 4);
   } else {
-    hipLaunchKernelGGL((fa_decode_split_kernel<64, BF16>), grid, dim3(kDecThreads), 0, s, Q, Kp,
-                       Vp, page_table, ctx_lens, part_o, part_lse, (int)H, (int)Hkv,
-                       (int)max_pages, (int)num_pages, (int)num_splits, c);
+    if (W == 8) FA_DECODE_SPLIT(64, 8);
+    else FA_DECODE_SPLIT(64, 4);
   }
+#undef FA_DECODE_SPLIT
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? FA_OK : -(int)e;
 }
@@ -440,12 +498,14 @@ static int lse_combine(const float* part_o, const float* part_lse, int64_t B, in
   if (num_splits < 1 || num_splits > 16) return FA_ERR_NUM_SPLITS;
   if (B * H > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int rows = (int)(B * H), per_wg = kCombThreads / (int)(D / 4);
+  const dim3 grid((unsigned)((rows - 1) / per_wg + 1));
   if (D == 128) {
-    hipLaunchKernelGGL((fa_lse_combine_kernel<128, BF16>), dim3((unsigned)(B * H)), dim3(128), 0,
-                       s, part_o, part_lse, (E*)o, lse, (int)num_splits);
+    hipLaunchKernelGGL((fa_lse_combine_kernel<128, BF16>), grid, dim3(kCombThreads), 0, s, part_o,
+                       part_lse, (E*)o, lse, (int)num_splits, rows);
   } else {
-    hipLaunchKernelGGL((fa_lse_combine_kernel<64, BF16>), dim3((unsigned)(B * H)), dim3(64), 0,
-                       s, part_o, part_lse, (E*)o, lse, (int)num_splits);
+    hipLaunchKernelGGL((fa_lse_combine_kernel<64, BF16>), grid, dim3(kCombThreads), 0, s, part_o,
+                       part_lse, (E*)o, lse, (int)num_splits, rows);
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? FA_OK : -(int)e;
@@ -461,7 +521,7 @@ extern "C" int fa_decode_split_f16(const void* q, const void* k_pool, const void
                               max_pages, num_pages, num_splits);
   if (st != FA_OK) return st;
   return fa::decode_split<false>(q, k_pool, v_pool, page_table, ctx_lens, B, H, H, D, max_pages,
-                                 num_pages, num_splits, part_o, part_lse, stream);
+                                 num_pages, num_splits, part_o, part_lse, nullptr, nullptr, stream);
 }
 
 extern "C" int fa_lse_combine_f32(const float* part_o, const float* part_lse, int64_t B,
@@ -470,19 +530,26 @@ extern "C" int fa_lse_combine_f32(const float* part_o, const float* part_lse, in
   return fa::lse_combine<false>(part_o, part_lse, B, H, D, num_splits, o, lse, stream);
 }
 
-extern "C" int fa_decode_paged_f16(const void* q, const void* k_pool, const void* v_pool,
-                                   const int32_t* page_table, const int32_t* ctx_lens,
-                                   int64_t B, int64_t H, int64_t D, int64_t page_size,
-                                   int64_t max_pages, int64_t num_pages, int64_t num_splits,
-                                   float* part_o, float* part_lse, void* o, float* lse,
-                                   void* stream) {
-  int st = fa_decode_split_f16(q, k_pool, v_pool, page_table, ctx_lens, B, H, D, page_size,
-                               max_pages, num_pages, num_splits, part_o, part_lse, stream);
-  if (st != FA_OK) return st;
-  return fa_lse_combine_f32(part_o, part_lse, B, H, D, num_splits, o, lse, stream);
+namespace fa {
+// Splits that a decode of O and L uses, at most the caller's num_splits (whose
+// partials the workspace holds). max_pages bounds the contexts; the host does
+// not know them. A split costs a workgroup its start and merge (3-4 us) and
+// the partials' way through memory, so no more of them than
+//   * give every CU one workgroup of 8 waves (B32 over 8 KV heads, 2000
+//     tokens: 1 split 41 us, 16 splits 68; B8, 200-4000 tokens: 4 splits 20.7,
+//     16 splits 24.5), with two pages a wave (B1, 4000 tokens: 15 splits 10.9,
+//     7 splits 12.9); up to 32 pages stay in one (500 tokens: 7.2 us, split 10);
+//   * or, of long contexts (64 pages a split), give every CU two: ragged
+//     sequences then even out (B16 H32, 2000-8000 tokens, 4 waves: 1 split 214,
+//     2 splits 201), and two at least (B32 H32, 512-32768 tokens: 1432, 1404).
+static int64_t plan_splits(int64_t B, int64_t H, int64_t Hkv, int64_t max_pages, int64_t num_splits,
+                           int cus) {
+  const int64_t units = B * Hkv * ((H / Hkv + 15) / 16);
+  const int64_t fill = max_pages <= 32 ? 1 : std::min((cus + units - 1) / units, max_pages / 16);
+  const int64_t deep = std::min(max_pages / 64, std::max<int64_t>(2, 2 * cus / units));
+  return std::min(num_splits, std::max<int64_t>(1, std::max(fill, deep)));
 }
 
-namespace fa {
 template <bool BF16>
 static int decode_paged_gqa(const void* q, const void* k_pool, const void* v_pool,
                             const int32_t* page_table, const int32_t* ctx_lens, int64_t B,
@@ -493,12 +560,30 @@ static int decode_paged_gqa(const void* q, const void* k_pool, const void* v_poo
                               max_pages, num_pages, num_splits);
   if (st != FA_OK) return st;
   if (H_kv <= 0 || H % H_kv != 0) return FA_ERR_KV_HEADS;
+  if (!part_o || !part_lse || !o) return FA_ERR_NULL_POINTER;
+  if (B * H > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
+  num_splits = plan_splits(B, H, H_kv, max_pages, num_splits,
+                           stream_topology(reinterpret_cast<hipStream_t>(stream)).cus);
+  if (num_splits == 1)
+    return decode_split<BF16>(q, k_pool, v_pool, page_table, ctx_lens, B, H, H_kv, D, max_pages,
+                              num_pages, 1, part_o, part_lse, o, lse, stream);
   st = decode_split<BF16>(q, k_pool, v_pool, page_table, ctx_lens, B, H, H_kv, D, max_pages,
-                          num_pages, num_splits, part_o, part_lse, stream);
+                          num_pages, num_splits, part_o, part_lse, nullptr, nullptr, stream);
   if (st != FA_OK) return st;
   return lse_combine<BF16>(part_o, part_lse, B, H, D, num_splits, o, lse, stream);
 }
 }  // namespace fa
+
+extern "C" int fa_decode_paged_f16(const void* q, const void* k_pool, const void* v_pool,
+                                   const int32_t* page_table, const int32_t* ctx_lens,
+                                   int64_t B, int64_t H, int64_t D, int64_t page_size,
+                                   int64_t max_pages, int64_t num_pages, int64_t num_splits,
+                                   float* part_o, float* part_lse, void* o, float* lse,
+                                   void* stream) {
+  return fa::decode_paged_gqa<false>(q, k_pool, v_pool, page_table, ctx_lens, B, H, H, D,
+                                     page_size, max_pages, num_pages, num_splits, part_o,
+                                     part_lse, o, lse, stream);
+}
 
 extern "C" int fa_decode_paged_gqa_f16(const void* q, const void* k_pool, const void* v_pool,
                                        const int32_t* page_table, const int32_t* ctx_lens,

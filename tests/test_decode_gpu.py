@@ -111,6 +111,44 @@ def test_gather_bit_exact_one_hot(fa, dev):
             assert np.array_equal(O[b], want), f"seq {b} token {j} S{S}"
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,ctx,width", [
+    (1, 3, [512], 32),            # 32 pages: one split, no combine pass
+    (1, 3, [513], 33),            # 33: two splits of 8 waves
+    (1, 2, [1, ], 2048),          # a table far wider than the context: empty splits
+    (3, 2, [5000, 17, 130], 320),  # ragged, more splits than the short ones have pages
+    (2, 300, [200, 65], 16),      # over two workgroups a CU: four waves each
+    (70, 8, [96 + b for b in range(70)], 12),   # 560 workgroups, ordered by length
+])
+def test_decode_planned_splits(fa, dev, D, B, H, ctx, width):
+    """The split counts and workgroup widths that the decode picks by its sizes
+    (up to 16 splits allowed), at the edges of each."""
+    q, kp, vp, table, ctx = _small(40 + B + D, B, H, D, ctx)
+    wide = np.zeros((B, width), np.int32)
+    wide[:, :table.shape[1]] = table
+    O, L = fa.decode_paged(*_dev(dev, q, kp, vp, wide, ctx), num_splits=16)
+    Or, Lr = decode_attention(q, kp, vp, table, ctx)
+    _check(O, L, Or, Lr, tag=f"B{B} H{H} D{D} width {width}")
+
+
+def test_combine_element_aligned(fa, capi, dev):
+    """Partials and outputs of the combine need only their elements' alignment."""
+    lib = capi.load()
+    B, H, D, S = 2, 3, 128, 5
+    rng = np.random.default_rng(50)
+    po = torch.from_numpy(rng.standard_normal((B, H, S, D)).astype(np.float32)).to(dev)
+    pl = torch.from_numpy(rng.standard_normal((B, H, S)).astype(np.float32)).to(dev)
+    O, L = fa.lse_combine(po, pl)
+    shifted = torch.empty(po.numel() + 1, device=dev)[1:]
+    shifted.copy_(po.flatten())
+    out = torch.empty(O.numel() + 1, device=dev, dtype=torch.half)[1:]
+    lse = torch.empty_like(L)
+    st = lib.fa_lse_combine_f32(shifted.data_ptr(), pl.data_ptr(), B, H, D, S, out.data_ptr(), lse.data_ptr(),
+                                torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert st == 0 and torch.equal(out, O.flatten()) and torch.equal(lse, L)
+
+
 def test_page_permutation_bitwise_invariance(fa, dev):
     """Relabel the pages (move pool rows, rewrite the table): identical bits out."""
     q, kp, vp, table, ctx = _small(9, B=4, H=2, D=128, ctx=[40, 700, 129, 16], extra_pages=7)
