@@ -25,9 +25,12 @@
 //
 // P and dS are packed to fp16 straight from the score accumulators as the B
 // operands of the gradient products (the reduction index is permuted the same
-// way in both operands, as in the forward). Tiles read both as rows (b128)
-// and transposed (ds_read_b64_tr_b16) are stored in LDS twice, once per
-// swizzle, so both reads stay bank-conflict free.
+// way in both operands, as in the forward). Tiles are read both as rows (b128)
+// and transposed (ds_read_b64_tr_b16) from one copy whose swizzle keeps both
+// reads bank-conflict free (t_swz). Two copies, one per kind of read, took
+// twice the copy instructions, LDS and L2 traffic (us, two copies -> one: B4
+// H16 N4096 D128 causal 1187 -> 1079, B1 H32 over 8 heads N2000 D128 causal
+// bf16 187 -> 179, B1 H8 N4096 D64 137.5 -> 135.3).
 #include <hip/hip_runtime.h>
 
 #include <stdlib.h>
@@ -47,15 +50,13 @@ namespace bwd {
 constexpr int kBQ = 64;     // rows of a streamed tile
 constexpr int kBlk = 128;   // rows owned by a workgroup (32 per wave)
 
-// Per-lane source offsets of 1 KiB block b of a 64-row tile, for the K-style
-// (row reads) and V-style (transposed reads) LDS swizzles.
+// Per-lane source offset of 1 KiB block b of a 64-row tile (see t_swz).
 template <int D>
-__device__ __forceinline__ void block_offsets(int b, int lane, uint32_t& koff, uint32_t& voff) {
+__device__ __forceinline__ uint32_t block_offset(int b, int lane) {
   const int o = b * 1024 + 16 * lane;
   const int r = o / (2 * D);
   const int slot = (o % (2 * D)) / 16;
-  koff = (uint32_t)(r * 2 * D + (slot ^ k_swz<D>(r)) * 16);
-  voff = (uint32_t)(r * 2 * D + (slot ^ v_swz<D>(r)) * 16);
+  return (uint32_t)(r * 2 * D + (slot ^ t_swz<D>(r)) * 16);
 }
 
 // A pointer the caller knows to be the same in every lane, moved to SGPRs
@@ -196,11 +197,11 @@ __device__ __forceinline__ void group_reduce(char* smem, int grp, int slot, int 
 // ---------------------------------------------------------------------------
 // dK/dV and dQ bodies (8 waves). A dK/dV workgroup owns 128 keys of one
 // (b, h): wave w holds K^T and V^T of keys k0 + 32 (w % 4) .. +31 as register
-// B operands, and 64-query tiles of Q and dO stream through LDS, each stored
-// twice (row swizzle for the score products, transposed swizzle for the
-// gradient products), with 64 floats each of NL and -D_i. A dQ workgroup
-// owns 128 queries the same way (Q^T and dO^T as register operands, NL and
-// -D_i lane constants) and streams 64-key tiles of K (twice) and V.
+// B operands, and 64-query tiles of Q and dO stream through LDS (read as rows
+// for the score products, transposed for the gradient products), with 64
+// floats each of NL and -D_i. A dQ workgroup owns 128 queries the same way
+// (Q^T and dO^T as register operands, NL and -D_i lane constants) and streams
+// 64-key tiles of K and V.
 //
 // The two wave groups (waves 0-3 and 4-7) hold the same keys (dK/dV) or
 // queries (dQ), each takes one 32-row half of every tile, their partial sums
@@ -221,9 +222,8 @@ __device__ __forceinline__ void group_reduce(char* smem, int grp, int slot, int 
 // staged data, and the barriers keep them one phase apart and sync each
 // group's four waves on their copies.
 //
-// D = 64 (rows 32 g .. +31 of each part are its 1 KiB blocks 4 g .. 4 g + 3
-// in both swizzles): tile j's stage is read
-// from S(j - 1), which loads tile j's A operands into registers (M(j) then
+// D = 64 (rows 32 g .. +31 of each part are its 1 KiB blocks 4 g .. 4 g + 3):
+// tile j's stage is read from S(j - 1), which loads tile j's A operands into registers (M(j) then
 // issues its score products without LDS waits), to M(j + 1), which reads its
 // C operands. S(j) starts the copies of tile j + 3 into the stage of tile
 // j - 1 (last read in M(j), before the barrier that starts S(j)) and M(j + 2)
@@ -234,14 +234,14 @@ constexpr int kPPStages = 4;
 
 template <int D>
 constexpr int dkdv_pp_smem() {
-  constexpr int STAGE = 4 * (kBQ * D * 2) + 2048;
+  constexpr int STAGE = 2 * (kBQ * D * 2) + 2048;
   constexpr int RED = 4 * 2 * (D / 32) * 16 * 64 * 4;
   return kPPStages * STAGE > RED ? kPPStages * STAGE : RED;
 }
 
 template <int D>
 constexpr int dq_pp_smem() {
-  constexpr int STAGE = 3 * (kBQ * D * 2);
+  constexpr int STAGE = 2 * (kBQ * D * 2);
   constexpr int RED = 4 * (D / 32) * 16 * 64 * 4;
   return kPPStages * STAGE > RED ? kPPStages * STAGE : RED;
 }
@@ -257,9 +257,10 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
+  constexpr int PER = OWN / 2;                 // blocks per wave of a group's copies
   constexpr int KSTEPS = D / 16, DB = D / 32;
-  // Qk | Qv | dOk | dOv | row vectors (group g: L at +512 g, D_i at +512 g + 256)
-  constexpr int STAGE = 4 * TILE + 2048;
+  // Q | dO | row vectors (group g: L at +512 g, D_i at +512 g + 256)
+  constexpr int STAGE = 2 * TILE + 2048;
   static_assert(kPPStages * STAGE <= 160 * 1024, "LDS");
 
   const int lane = threadIdx.x & 63;
@@ -294,29 +295,28 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   const int T = n_qt - t0;                 // tiles of this workgroup (>= 1)
 
   const uint32_t lds0 = lds_addr(smem);
+  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
   auto stage_of = [&](int j) { return smem + (j % kPPStages) * STAGE; };
-  // This group's half of tile t into stage st: wave kw copies its 4 blocks of
-  // part kw; waves 0 and 1 also copy the 64-row L and D_i vectors.
+  // This group's half of tile t into stage st: wave kw copies two blocks of
+  // part kw / 2; waves 0 and 1 also copy the 64-row L and D_i vectors.
   auto issue_own = [&](int t, int st) {
     const uint32_t base = lds0 + st * STAGE;
     const char* src = kw < 2 ? Qh : Gh;
 #pragma unroll
-    for (int i = 0; i < OWN; ++i) {
-      const int b = OWN * grp + i;
-      uint32_t ko, vo;
-      block_offsets<D>(b, lane, ko, vo);
-      copy_block<D>(src, head_bytes, t, base + kw * TILE + b * 1024, (kw & 1) ? vo : ko);
+    for (int i = 0; i < PER; ++i) {
+      const int b = OWN * grp + PER * (kw & 1) + i;
+      copy_block<D>(src, head_bytes, t, base + (kw >> 1) * TILE + b * 1024, block_offset<D>(b, lane));
     }
-    if (kw == 0) copy_rowvec(Lh, N, t, base + 4 * TILE + 512 * grp, lane);
-    if (kw == 1) copy_rowvec(Dh, N, t, base + 4 * TILE + 512 * grp + 256, lane);
+    if (kw == 0) copy_rowvec(Lh, N, t, base + 2 * TILE + 512 * grp, lane);
+    if (kw == 1) copy_rowvec(Dh, N, t, base + 2 * TILE + 512 * grp + 256, lane);
   };
   // Copies run three tiles ahead: at the end of M phase j tile j + 1 must
   // have landed, and tile j + 2's copies (this wave's last issue) may still
   // be in flight.
   auto wait_next = [&](bool later_in_flight) {
     if (!later_in_flight) wait_vmem();
-    else if (kw < 2) wait_vmcnt<OWN + 1>();
-    else wait_vmcnt<OWN>();
+    else if (kw < 2) wait_vmcnt<PER + 1>();
+    else wait_vmcnt<PER>();
   };
   issue_own(t0, 0);
   if (T > 1) issue_own(t0 + 1, 1);
@@ -328,11 +328,11 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   f16x8 pb[2], gb[2];       // its packed P and dS (B operands of the two k-steps)
   f16x8 af[KSTEPS][2];      // A operands of its next score products (Q, dO rows)
   auto load_a = [&](int j) {   // of relative tile j
-    const char* sb = stage_of(j);
+    const uint32_t rb = row_base<D>(half0 + (j % kPPStages) * STAGE, lane);
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
-      af[kk][0] = load_k_frag<D>(sb, qb, kk, lane);
-      af[kk][1] = load_k_frag<D>(sb + 2 * TILE, qb, kk, lane);
+      af[kk][0] = load_row_frag<D>(rb, 0, kk);
+      af[kk][1] = load_row_frag<D>(rb, TILE, kk);
     }
   };
   // A: S = Q K^T and dP = dO V^T (C layout: register r holds query
@@ -341,13 +341,12 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
     s = mma32<BF16>(af[kk][0], kf[kk], kk == 0 ? f32x16{} : s);
     dp = mma32<BF16>(af[kk][1], vf[kk], kk == 0 ? f32x16{} : dp);
   };
-  // C of the tile whose stage is sb: dV^T += dO^T P and dK^T += Q^T dS; step
+  // C of the tile whose column base is cb: dV^T += dO^T P and dK^T += Q^T dS; step
   // kk is k-step kk / DB, d-block kk % DB. Operands (dO^T, Q^T) read two
   // steps ahead.
-  auto load_c = [&](const char* sb, int kk, f16x8 (&f)[2]) {
-    const int jj = 2 * qb + kk / DB;
-    f[0] = load_v_frag<D>(sb + 3 * TILE, jj, kk % DB, lane);
-    f[1] = load_v_frag<D>(sb + TILE, jj, kk % DB, lane);
+  auto load_c = [&](uint32_t cb, int kk, f16x8 (&f)[2]) {
+    f[0] = load_col_frag<D>(cb, TILE, kk / DB, kk % DB);
+    f[1] = load_col_frag<D>(cb, 0, kk / DB, kk % DB);
   };
   auto mma_c = [&](const f16x8 (&f)[2], int kk) {
     const int h = kk / DB, db = kk % DB;
@@ -358,7 +357,7 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   // j); then the wait for the copies this wave started in S(j - 1).
   auto mphase = [&](int j, auto with_c, auto with_a) {
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
-    const char* sc = stage_of(j + kPPStages - 1);
+    const uint32_t sc = col_base<D>(half0 + ((j + kPPStages - 1) % kPPStages) * STAGE, lane);
     f16x8 cf[KSTEPS][2];
     if constexpr (WC) {
       load_c(sc, 0, cf[0]);
@@ -381,7 +380,7 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
     if (j + 3 < T) issue_own(t0 + j + 3, (j + 3) % kPPStages);
     const char* sb = stage_of(j);
     const int qt0 = (t0 + j) * kBQ;
-    const float* ls = reinterpret_cast<const float*>(sb + 4 * TILE + 512 * grp);
+    const float* ls = reinterpret_cast<const float*>(sb + 2 * TILE + 512 * grp);
     const float* nds = ls + 64;
     // Row vectors first (LDS reads return in order), then the next tile's A
     // operands, which land while the VALU work below runs.
@@ -456,10 +455,10 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
-  constexpr int PER = 3 * OWN / 4;             // blocks per wave of a group's copies
+  constexpr int PER = OWN / 2;                 // blocks per wave of a group's copies
   constexpr int KSTEPS = D / 16, DB = D / 32;
-  constexpr int STAGE = 3 * TILE;              // Kk | Kv | Vk
-  static_assert(3 * OWN % 4 == 0 && kPPStages * STAGE <= 160 * 1024, "copy split, LDS");
+  constexpr int STAGE = 2 * TILE;              // K | V
+  static_assert(kPPStages * STAGE <= 160 * 1024, "LDS");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -493,20 +492,16 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   const bool rows_edge = q0 + 32 * qw + 32 > N;
 
   const uint32_t lds0 = lds_addr(smem);
-  auto stage_of = [&](int j) { return smem + (j % kPPStages) * STAGE; };
-  // This group's half of tile t into stage st: 4 blocks of each of the 3
-  // parts, PER consecutive ones per wave.
+  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
+  // This group's half of tile t into stage st: wave qw copies two blocks of
+  // part qw / 2.
   auto issue_own = [&](int t, int st) {
     const uint32_t base = lds0 + st * STAGE;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int x = PER * qw + i;
-      const int part = x / OWN;
-      const int b = OWN * grp + x % OWN;
-      uint32_t ko, vo;
-      block_offsets<D>(b, lane, ko, vo);
-      copy_block<D>(part < 2 ? Kh : Vh, head_bytes, t, base + part * TILE + b * 1024,
-                    part == 1 ? vo : ko);
+      const int b = OWN * grp + PER * (qw & 1) + i;
+      copy_block<D>(qw < 2 ? Kh : Vh, head_bytes, t, base + (qw >> 1) * TILE + b * 1024,
+                    block_offset<D>(b, lane));
     }
   };
   // Copies run three tiles ahead (as in the dK/dV body).
@@ -523,11 +518,12 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   f32x16 s = {}, dp = {};
   f16x8 gb[2];
   f16x8 af[KSTEPS][2];   // A operands of the next score products (K, V rows)
-  auto load_a = [&](const char* sb) {
+  auto load_a = [&](int j) {
+    const uint32_t rb = row_base<D>(half0 + (j % kPPStages) * STAGE, lane);
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
-      af[kk][0] = load_k_frag<D>(sb, half, kk, lane);
-      af[kk][1] = load_k_frag<D>(sb + 2 * TILE, half, kk, lane);
+      af[kk][0] = load_row_frag<D>(rb, 0, kk);
+      af[kk][1] = load_row_frag<D>(rb, TILE, kk);
     }
   };
   auto mma_a = [&](int kk) {
@@ -537,12 +533,10 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
     s = mma32<BF16>(af[kk][0], qf[kk], kk == 0 ? f32x16{} : s);
     dp = mma32<BF16>(af[kk][1], gf[kk], kk == 0 ? dp0 : dp);
   };
-  auto load_c = [&](const char* sb, int kk) {
-    return load_v_frag<D>(sb + TILE, 2 * half + kk / DB, kk % DB, lane);
-  };
+  auto load_c = [&](uint32_t cb, int kk) { return load_col_frag<D>(cb, 0, kk / DB, kk % DB); };
   auto mphase = [&](int j, auto with_c, auto with_a) {
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
-    const char* sc = stage_of(j + kPPStages - 1);
+    const uint32_t sc = col_base<D>(half0 + ((j + kPPStages - 1) % kPPStages) * STAGE, lane);
     f16x8 cf[KSTEPS];
     if constexpr (WC) {
       cf[0] = load_c(sc, 0);
@@ -560,7 +554,7 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   };
   auto sphase = [&](int j) {
     if (j + 3 < T) issue_own(j + 3, (j + 3) % kPPStages);
-    if (j + 1 < T) load_a(stage_of(j + 1));
+    if (j + 1 < T) load_a(j + 1);
     const int kt0 = j * kBQ;
     f32x16 p;
 #pragma unroll
@@ -585,7 +579,7 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
 
   using BT = std::true_type;
   using BF = std::false_type;
-  load_a(stage_of(0));
+  load_a(0);
   if (grp == 1) __syncthreads();   // phase 0: group 1 waits
   mphase(0, BF{}, BT{});
   __syncthreads();
@@ -618,20 +612,17 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
 //     before S and dP of tile j are live: the dK/dV body fits the 256 VGPRs
 //     of two waves per SIMD without spilling (K^T, V^T and the two
 //     accumulators alone take 192);
-//   * LDS: the parts of a tile are freed at different times (the row-swizzled
-//     A parts after M(j), the row vectors after S(j), the transposed C parts
-//     after M(j + 1)), so each part has its own ring of slots and S(j) starts
-//     A of tile j + 2, C of tile j + 1 and the row vectors of tile j + 2,
-//     each into the slot its last reader has just left: two A slots, two C
-//     slots and three row-vector slots (131 KiB at D = 128 for dK/dV) give
-//     every copy two phases to land, issued from the VALU phase.
+//   * LDS: a ring of three tiles (99 KiB with the row vectors; the final
+//     reduction takes 128). S(j) starts the copies of tile j + 2 into the slot
+//     of tile j - 1 (last read in M(j)), and its end waits for those of S(j - 1):
+//     every copy has two phases to land, issued from the VALU phase.
 // A group copies and reads only its own 32-row half of every part (rows
-// 32 g .. +31 are 1 KiB blocks 8 g .. 8 g + 7 in both swizzles).
+// 32 g .. +31 are 1 KiB blocks 8 g .. 8 g + 7).
 // ---------------------------------------------------------------------------
 template <int D>
 constexpr int dkdv_pp128_smem() {
   constexpr int TILE = kBQ * D * 2;
-  constexpr int RING = 2 * (2 * TILE) + 2 * (2 * TILE) + 3 * 1024;
+  constexpr int RING = 3 * (2 * TILE) + 3 * 1024;
   constexpr int RED = 4 * 2 * (D / 32) * 16 * 64 * 4;
   return RING > RED ? RING : RED;
 }
@@ -639,7 +630,7 @@ constexpr int dkdv_pp128_smem() {
 template <int D>
 constexpr int dq_pp128_smem() {
   constexpr int TILE = kBQ * D * 2;
-  constexpr int RING = 2 * (2 * TILE) + 2 * TILE;
+  constexpr int RING = 3 * (2 * TILE);
   constexpr int RED = 4 * (D / 32) * 16 * 64 * 4;
   return RING > RED ? RING : RED;
 }
@@ -658,11 +649,10 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
-  constexpr int PER = OWN / 2;                 // blocks per wave of one part's half
+  constexpr int PER = OWN / 2;                 // blocks per wave of a tile
   constexpr int KSTEPS = D / 16, DB = D / 32;
-  constexpr int SLOT = 2 * TILE;               // A slot: Qk | dOk; C slot: Qv | dOv
-  constexpr int C0 = 2 * SLOT;                 // C ring after the A ring
-  constexpr int R0 = 4 * SLOT;                 // row vectors: group g L at +512 g, -D_i +256
+  constexpr int SLOT = 2 * TILE;               // Q | dO
+  constexpr int R0 = 3 * SLOT;                 // row vectors: group g L at +512 g, -D_i +256
   static_assert(R0 + 3 * 1024 <= dkdv_pp128_smem<D>() && dkdv_pp128_smem<D>() <= 160 * 1024,
                 "ring inside the buffer, LDS");
   static_assert(2 * KSTEPS == 2 * 2 * DB, "C and A take the same number of steps");
@@ -698,50 +688,34 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   const int T = n_qt - t0;                 // tiles of this workgroup (>= 1)
 
   const uint32_t lds0 = lds_addr(smem);
+  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
   // Wave kw copies blocks 8 grp + 4 (kw & 1) .. +3 of part kw >> 1 (Q or dO)
-  // of a ring; the per-lane offsets are recomputed per copy (volatile lane
-  // id: held across the loop they would take registers the body needs).
-  auto issue_part = [&](int t, uint32_t base, bool vsw) {
+  // of relative tile j, waves 0 and 1 also its row vectors; the per-lane
+  // offsets are recomputed per copy (volatile lane id: held across the loop
+  // they would take registers the body needs).
+  auto issue_tile = [&](int j) {
     int ln;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
     const char* src = kw < 2 ? Qh : Gh;
+    const uint32_t base = lds0 + (j % 3) * SLOT + (kw >> 1) * TILE;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int b = OWN * grp + PER * (kw & 1) + i;
-      uint32_t ko, vo;
-      block_offsets<D>(b, ln, ko, vo);
-      copy_block<D>(src, head_bytes, t, base + (kw >> 1) * TILE + b * 1024, vsw ? vo : ko);
+      copy_block<D>(src, head_bytes, t0 + j, base + b * 1024, block_offset<D>(b, ln));
     }
-  };
-  auto issue_a = [&](int j) {   // A parts and row vectors of relative tile j
-    issue_part(t0 + j, lds0 + (j & 1) * SLOT, false);
     const uint32_t rv = lds0 + R0 + (j % 3) * 1024 + 512 * grp;
-    int ln;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
     if (kw == 0) copy_rowvec(Lh, N, t0 + j, rv, ln);
     if (kw == 1) copy_rowvec(Dh, N, t0 + j, rv + 256, ln);
   };
-  auto issue_c = [&](int j) { issue_part(t0 + j, lds0 + C0 + (j & 1) * SLOT, true); };
-  // Copies issued by this wave in one S phase: A (PER, + 1 row vector for
-  // waves 0 and 1) and C (PER). The end of S(j) leaves S(j)'s copies in
-  // flight and waits for the rest.
-  auto wait_for = [&](bool a, bool cc) {
-    if (a && cc) {
-      if (kw < 2) wait_vmcnt<2 * PER + 1>();
-      else wait_vmcnt<2 * PER>();
-    } else if (a) {
-      if (kw < 2) wait_vmcnt<PER + 1>();
-      else wait_vmcnt<PER>();
-    } else if (cc) {
-      wait_vmcnt<PER>();
-    } else {
-      wait_vmem();
-    }
+  // All copies but those of the last tile issued (if `last` was).
+  auto wait_for = [&](bool last) {
+    if (!last) wait_vmem();
+    else if (kw < 2) wait_vmcnt<PER + 1>();
+    else wait_vmcnt<PER>();
   };
-  issue_a(0);
-  issue_c(0);
-  if (T > 1) issue_a(1);
-  wait_vmem();
+  issue_tile(0);
+  if (T > 1) issue_tile(1);
+  wait_for(T > 1);
   __syncthreads();
 
   f32x16 s = {}, dp = {};   // this wave's scores of its current tile
@@ -752,18 +726,17 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   auto mphase = [&](int j, auto with_c, auto with_a) {
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
     constexpr int X0 = WC ? 0 : KSTEPS, X1 = WA ? 2 * KSTEPS : KSTEPS;
-    const char* sc = smem + C0 + ((j + 1) & 1) * SLOT;   // C slot of tile j - 1
-    const char* sa = smem + (j & 1) * SLOT;              // A slot of tile j
+    const uint32_t sc = col_base<D>(half0 + ((j + 2) % 3) * SLOT, lane);   // tile j - 1
+    const uint32_t sa = row_base<D>(half0 + (j % 3) * SLOT, lane);         // tile j
     f16x8 f[2 * KSTEPS][2];
     auto load = [&](auto xi) {
       constexpr int x = decltype(xi)::value;
       if constexpr (x < KSTEPS) {
-        const int jj = 2 * qb + x / DB;
-        f[x][0] = load_v_frag<D>(sc + TILE, jj, x % DB, lane);   // dO^T
-        f[x][1] = load_v_frag<D>(sc, jj, x % DB, lane);          // Q^T
+        f[x][0] = load_col_frag<D>(sc, TILE, x / DB, x % DB);   // dO^T
+        f[x][1] = load_col_frag<D>(sc, 0, x / DB, x % DB);      // Q^T
       } else {
-        f[x][0] = load_k_frag<D>(sa, qb, x - KSTEPS, lane);          // Q rows
-        f[x][1] = load_k_frag<D>(sa + TILE, qb, x - KSTEPS, lane);   // dO rows
+        f[x][0] = load_row_frag<D>(sa, 0, x - KSTEPS);      // Q rows
+        f[x][1] = load_row_frag<D>(sa, TILE, x - KSTEPS);   // dO rows
       }
     };
     // Operands two steps ahead within each part; A's first two are loaded
@@ -790,13 +763,12 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
     });
     __builtin_amdgcn_sched_barrier(0);   // keep every product in this phase
   };
-  // S phase of relative tile j: the copies of A(j + 2), C(j + 1) and the row
-  // vectors of j + 2, then P and dS into pb, gb; at the end, the wait for
-  // the copies of S(j - 1) (A(j + 1), C(j): M(j + 1) reads them).
+  // S phase of relative tile j: the copies of tile j + 2, then P and dS into
+  // pb, gb; at the end, the wait for the copies of S(j - 1) (tile j + 1:
+  // M(j + 1) reads it).
   auto sphase = [&](int j) {
-    const bool ca = j + 2 < T, cc = j + 1 < T;
-    if (cc) issue_c(j + 1);
-    if (ca) issue_a(j + 2);
+    const bool more = j + 2 < T;
+    if (more) issue_tile(j + 2);
     const int qt0 = (t0 + j) * kBQ;
     const float* ls = reinterpret_cast<const float*>(smem + R0 + (j % 3) * 1024 + 512 * grp);
     const float* nds = ls + 64;
@@ -830,7 +802,7 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
       pb[h] = pack_px<BF16>(p, h);
       gb[h] = pack_px<BF16>(g, h);
     }
-    wait_for(ca, cc);
+    wait_for(more);
   };
   auto pin_s = [&] { asm volatile("" : "+v"(s), "+v"(dp)); };
   auto pin_p = [&] { asm volatile("" : "+v"(pb[0]), "+v"(pb[1]), "+v"(gb[0]), "+v"(gb[1])); };
@@ -876,12 +848,11 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
-  constexpr int PA = OWN / 2, PC = OWN / 4;    // blocks per wave: A parts, C part
+  constexpr int PER = OWN / 2;                 // blocks per wave of a tile
   constexpr int KSTEPS = D / 16, DB = D / 32;
-  constexpr int SLOT = 2 * TILE;               // A slot: Kk | Vk
-  constexpr int C0 = 2 * SLOT;                 // C slots (Kv), TILE bytes each
-  static_assert(C0 + 2 * TILE <= dq_pp128_smem<D>() && dq_pp128_smem<D>() <= 160 * 1024 &&
-                OWN % 4 == 0, "ring inside the buffer, LDS, copy split");
+  constexpr int SLOT = 2 * TILE;               // K | V
+  static_assert(3 * SLOT <= dq_pp128_smem<D>() && dq_pp128_smem<D>() <= 160 * 1024,
+                "ring inside the buffer, LDS");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -914,42 +885,25 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
   const bool rows_edge = q0 + 32 * qw + 32 > N;
 
   const uint32_t lds0 = lds_addr(smem);
-  // A parts (Kk, Vk): wave qw copies blocks 8 grp + 4 (qw & 1) .. +3 of part
-  // qw >> 1; C part (Kv): blocks 8 grp + 2 qw .. +1.
-  auto issue_a = [&](int j) {
+  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
+  // Wave qw copies blocks 8 grp + 4 (qw & 1) .. +3 of part qw >> 1 (K or V).
+  auto issue_tile = [&](int j) {
     int ln;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-    const uint32_t base = lds0 + (j & 1) * SLOT + (qw >> 1) * TILE;
+    const uint32_t base = lds0 + (j % 3) * SLOT + (qw >> 1) * TILE;
 #pragma unroll
-    for (int i = 0; i < PA; ++i) {
-      const int b = OWN * grp + PA * (qw & 1) + i;
-      uint32_t ko, vo;
-      block_offsets<D>(b, ln, ko, vo);
-      copy_block<D>(qw < 2 ? Kh : Vh, head_bytes, j, base + b * 1024, ko);
+    for (int i = 0; i < PER; ++i) {
+      const int b = OWN * grp + PER * (qw & 1) + i;
+      copy_block<D>(qw < 2 ? Kh : Vh, head_bytes, j, base + b * 1024, block_offset<D>(b, ln));
     }
   };
-  auto issue_c = [&](int j) {
-    int ln;
-    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-    const uint32_t base = lds0 + C0 + (j & 1) * TILE;
-#pragma unroll
-    for (int i = 0; i < PC; ++i) {
-      const int b = OWN * grp + PC * qw + i;
-      uint32_t ko, vo;
-      block_offsets<D>(b, ln, ko, vo);
-      copy_block<D>(Kh, head_bytes, j, base + b * 1024, vo);
-    }
-  };
-  auto wait_for = [&](bool a, bool cc) {
-    if (a && cc) wait_vmcnt<PA + PC>();
-    else if (a) wait_vmcnt<PA>();
-    else if (cc) wait_vmcnt<PC>();
+  auto wait_for = [&](bool last) {   // all copies but those of the last tile issued
+    if (last) wait_vmcnt<PER>();
     else wait_vmem();
   };
-  issue_a(0);
-  issue_c(0);
-  if (T > 1) issue_a(1);
-  wait_vmem();
+  issue_tile(0);
+  if (T > 1) issue_tile(1);
+  wait_for(T > 1);
   __syncthreads();
 
   f32x16 s = {}, dp = {};
@@ -960,16 +914,16 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
     constexpr int CX = 2 * DB;   // C steps
     constexpr int X0 = WC ? 0 : CX, X1 = WA ? CX + KSTEPS : CX;
-    const char* sc = smem + C0 + ((j + 1) & 1) * TILE;   // C slot of tile j - 1
-    const char* sa = smem + (j & 1) * SLOT;              // A slot of tile j
+    const uint32_t sc = col_base<D>(half0 + ((j + 2) % 3) * SLOT, lane);   // tile j - 1
+    const uint32_t sa = row_base<D>(half0 + (j % 3) * SLOT, lane);         // tile j
     f16x8 f[CX + KSTEPS][2];
     auto load = [&](auto xi) {
       constexpr int x = decltype(xi)::value;
       if constexpr (x < CX) {
-        f[x][0] = load_v_frag<D>(sc, 2 * half + x / DB, x % DB, lane);   // K^T
+        f[x][0] = load_col_frag<D>(sc, 0, x / DB, x % DB);   // K^T
       } else {
-        f[x][0] = load_k_frag<D>(sa, half, x - CX, lane);          // K rows
-        f[x][1] = load_k_frag<D>(sa + TILE, half, x - CX, lane);   // V rows
+        f[x][0] = load_row_frag<D>(sa, 0, x - CX);      // K rows
+        f[x][1] = load_row_frag<D>(sa, TILE, x - CX);   // V rows
       }
     };
     static_for<X0, X0 + 2 < X1 ? X0 + 2 : X1>(load);
@@ -988,9 +942,8 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
     __builtin_amdgcn_sched_barrier(0);
   };
   auto sphase = [&](int j) {
-    const bool ca = j + 2 < T, cc = j + 1 < T;
-    if (cc) issue_c(j + 1);
-    if (ca) issue_a(j + 2);
+    const bool more = j + 2 < T;
+    if (more) issue_tile(j + 2);
     const int kt0 = j * kBQ;
     f32x16 p;
 #pragma unroll
@@ -1009,7 +962,7 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
     for (int r = 0; r < 16; ++r) g[r] = p[r] * (dp[r] + dq_i);
 #pragma unroll
     for (int h = 0; h < 2; ++h) gb[h] = pack_px<BF16>(g, h);
-    wait_for(ca, cc);
+    wait_for(more);
   };
   auto pin_s = [&] { asm volatile("" : "+v"(s), "+v"(dp)); };
   auto pin_p = [&] { asm volatile("" : "+v"(gb[0]), "+v"(gb[1])); };

@@ -266,6 +266,64 @@ __device__ __forceinline__ f16x8 load_v_frag(const char* vs, int j, int db, int 
   return v_frag_at<D>(vs + 16 * j * 2 * D + v_frag_off<D>(db, lane));
 }
 
+// One layout for both reads (the backward's tiles, read as rows and
+// transposed): chunk c of row r at slot c ^ t_swz(r). Row reads (b128: 16
+// lanes take one chunk of 16 consecutive rows, 256 bytes = every bank once)
+// need t_swz one to one over 16 rows at D = 128, over 8 row pairs at D = 64.
+// Transposed reads (32 lanes take 64 bytes of 4 consecutive rows) need its
+// top bits (64-byte column blocks) to differ between rows of the same bank
+// half: over r % 4 at D = 128, over (r / 2) % 2 at D = 64. Putting the row's
+// low bits on top gives both, so a tile is copied and kept once.
+template <int D>
+__device__ __forceinline__ int t_swz(int r) {
+  if constexpr (D == 64) {
+    return (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+  } else {
+    return ((r & 3) << 2) | ((r >> 2) & 3);
+  }
+}
+
+// Byte address of a lane's first row read (rows 0 .. 31, k-step 0) and first
+// transposed read (rows 0 .. 15, column block 0) of a tile at LDS address
+// `tile` (1 KiB aligned). The other reads flip bits of it or add constants, so
+// a phase needs one base of each kind; opaque, or the compiler keeps a
+// loop-invariant offset for every flip (21 spilled registers in the D = 128
+// backward).
+template <int D>
+__device__ __forceinline__ uint32_t row_base(uint32_t tile, int lane) {
+  const int r = lane & 31;
+  uint32_t a = tile + r * 2 * D + ((lane >> 5) ^ t_swz<D>(r)) * 16;
+  asm("" : "+v"(a));
+  return a;
+}
+
+template <int D>
+__device__ __forceinline__ uint32_t col_base(uint32_t tile, int lane) {
+  const int s = lane & 15;
+  const int r = 4 * (lane >> 5) + (s >> 2);
+  const int c = 2 * ((lane >> 4) & 1) + ((s & 3) >> 1);
+  uint32_t a = tile + r * 2 * D + (c ^ t_swz<D>(r)) * 16 + 8 * (s & 1);
+  asm("" : "+v"(a));
+  return a;
+}
+
+// Rows 0 .. 31 of the tile as an A operand (k-step kk of D), `off` bytes on
+// (a constant): as load_k_frag.
+template <int D>
+__device__ __forceinline__ f16x8 load_row_frag(uint32_t base, int off, int kk) {
+  return lds_b128((lds_cp)(size_t)(base ^ (32 * kk)) + off);
+}
+
+// Columns 32 db .. + 31 of rows 16 j .. + 15 as an A operand (transposed),
+// `off` bytes on: as load_v_frag. Eight rows up, t_swz differs in its bit 1,
+// address bit 5.
+template <int D>
+__device__ __forceinline__ f16x8 load_col_frag(uint32_t base, int off, int j, int db) {
+  const f16x4 lo = lds_tr16((lds_cp)(size_t)(base ^ (64 * db)) + off + 16 * j * 2 * D);
+  const f16x4 up = lds_tr16((lds_cp)(size_t)(base ^ (64 * db + 32)) + off + (16 * j + 8) * 2 * D);
+  return f16x8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
+}
+
 // Key index (within a 64-key tile) held by register r of key block kb in lane l.
 __device__ __forceinline__ int st_key(int kb, int r, int lane) {
   return 32 * kb + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
