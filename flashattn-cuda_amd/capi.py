@@ -50,6 +50,9 @@ SIGNATURES = {
     "fa_kv_append_f16": (C.c_int, [_vp] * 8 + [_i64] * 7 + [_vp]),
     "fa_kv_append_bf16": (C.c_int, [_vp] * 8 + [_i64] * 7 + [_vp]),
     "fa_kv_append_set_bad": (C.c_int, [_vp] * 8 + [_i64] * 7 + [_vp]),
+    "fa_cast_f32": (C.c_int, [_vp] * 3 + [C.c_int, _vp]),
+    "fa_bwd_cast_f32": (C.c_int, [_vp] * 7 + [_i64] * 5 + [C.c_int, C.c_int, _vp]),
+    "fa_varlen_fill_outside": (C.c_int, [_vp] + [_i64] * 3 + [_vp] * 5),
     "fa_bwd_gqa_workspace_floats": (_i64, [_i64] * 5),
     "fa_bwd_gqa_f16": (C.c_int, [_vp] * 10 + [_i64] * 5 + [C.c_int, _vp]),
     "fa_bwd_bf16": (C.c_int, [_vp] * 10 + [_i64] * 5 + [C.c_int, _vp]),

@@ -133,37 +133,63 @@ __device__ __forceinline__ void store_transposed(float* out, int n, int row0, in
 // log2(e), so that P = exp2(S c + NL) takes one fma and dP - D_i = dP + ND
 // one add (or an MFMA chain's initial value). 8 lanes per row, one 16-byte
 // chunk each per step (coalesced 128-byte runs), reduced with xor shuffles.
+// O and dO may come in fp32 (o32, g32; then rounded to the operand type
+// first, and dO also stored so): the pass reads them anyway, and the blocks
+// after its own convert Q, K and V, so a caller with fp32 tensors needs no
+// launches of its own for that (five conversions cost half of a B2 H8 N512
+// D64 backward).
 // ---------------------------------------------------------------------------
+struct RowTermArgs {
+  const f16* o;
+  f16* g;            // dO: given, or written from g32
+  const float* o32;
+  const float* g32;
+  const float* l;
+  float* nd;
+  float* nl;
+  int64_t rows;
+  int blocks;        // 32 rows each; later workgroups convert
+};
+
 template <int D, bool BF16>
 __global__ void __launch_bounds__(256)
-fa_bwd_di_kernel(const f16* __restrict__ O, const f16* __restrict__ dO,
-                 const float* __restrict__ L, float* __restrict__ ND, float* __restrict__ NL,
-                 int64_t rows) {
+fa_bwd_di_kernel(RowTermArgs a, CastJobs jobs) {
+  if ((int)blockIdx.x >= a.blocks) {
+    cast_block<BF16>(jobs, (int)blockIdx.x - a.blocks);
+    return;
+  }
   const int64_t row = (int64_t)blockIdx.x * 32 + (threadIdx.x >> 3);
   const int part = threadIdx.x & 7;
   float acc = 0.f;
-  if (row < rows) {
-    const f16x8* o = reinterpret_cast<const f16x8*>(O + row * D);
-    const f16x8* g = reinterpret_cast<const f16x8*>(dO + row * D);
+  if (row < a.rows) {
 #pragma unroll
     for (int i = part; i < D / 8; i += 8) {
-      const f16x8 a = o[i], b = g[i];
+      const int64_t at = row * D + 8 * i;
+      const f16x8 x = a.o32 != nullptr ? cvt8x<BF16>(a.o32 + at)
+                                       : *reinterpret_cast<const f16x8*>(a.o + at);
+      f16x8 y;
+      if (a.g32 != nullptr) {
+        y = cvt8x<BF16>(a.g32 + at);
+        *reinterpret_cast<f16x8*>(a.g + at) = y;
+      } else {
+        y = *reinterpret_cast<const f16x8*>(a.g + at);
+      }
       if constexpr (BF16) {
-        const bf16x8 ab = __builtin_bit_cast(bf16x8, a), bb = __builtin_bit_cast(bf16x8, b);
+        const bf16x8 xb = __builtin_bit_cast(bf16x8, x), yb = __builtin_bit_cast(bf16x8, y);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc = fmaf((float)ab[e], (float)bb[e], acc);
+        for (int e = 0; e < 8; ++e) acc = fmaf((float)xb[e], (float)yb[e], acc);
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) acc = fmaf((float)a[e], (float)b[e], acc);
+        for (int e = 0; e < 8; ++e) acc = fmaf((float)x[e], (float)y[e], acc);
       }
     }
   }
   acc += __shfl_xor(acc, 1, 8);
   acc += __shfl_xor(acc, 2, 8);
   acc += __shfl_xor(acc, 4, 8);
-  if (row < rows && part == 0) {
-    ND[row] = -acc;
-    NL[row] = -L[row] * kLog2e;
+  if (row < a.rows && part == 0) {
+    a.nd[row] = -acc;
+    a.nl[row] = -a.l[row] * kLog2e;
   }
 }
 
@@ -1040,12 +1066,15 @@ fa_bwd_fused_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
   }
 }
 
-// GQA: dK, dV of KV head hk = sum over its `group` query heads of the
-// per-query-head partials (fp32 [B*H, N*D] -> [B*Hkv, N*D]), four floats per
-// thread.
+// GQA: dK (blockIdx.y 0) and dV (1) of KV head hk = sum over its `group` query
+// heads of the per-query-head partials (fp32 [B*H, N*D] -> [B*Hkv, N*D]), four
+// floats per thread.
 __global__ void __launch_bounds__(256)
-fa_bwd_group_sum_kernel(const float* __restrict__ part, float* __restrict__ out, int64_t head_elems,
+fa_bwd_group_sum_kernel(const float* __restrict__ part_k, const float* __restrict__ part_v,
+                        float* __restrict__ dk, float* __restrict__ dv, int64_t head_elems,
                         int64_t kv_heads, int group) {
+  const float* part = blockIdx.y == 0 ? part_k : part_v;
+  float* out = blockIdx.y == 0 ? dk : dv;
   const int64_t i4 = (int64_t)blockIdx.x * 256 + threadIdx.x;   // float4 index in out
   const int64_t n4 = kv_heads * head_elems / 4;
   if (i4 >= n4) return;
@@ -1058,13 +1087,21 @@ fa_bwd_group_sum_kernel(const float* __restrict__ part, float* __restrict__ out,
   reinterpret_cast<f32x4*>(out)[i4] = acc;
 }
 
+// Inputs of a backward that come in fp32: O and dO (null: 16-bit), and the
+// conversions of Q, K and V.
+struct Fp32Inputs {
+  const float* o;
+  const float* g;
+  CastJobs qkv;
+};
+
 // The three passes (-D_i and -L log2 e, dK/dV, dQ) and, with H_kv < H, the
 // group sums. geo is dense (B heads of N rows per head) or varlen (heads of
 // geo.total packed rows); `rows` is the number of L rows: B*H*N dense, H*total
 // varlen.
 template <int D, bool CAUSAL, bool BF16>
 static hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o,
-                             const void* dout, const float* lse, float* dq, float* dk, float* dv,
+                             const void* dout, const Fp32Inputs& in, const float* lse, float* dq, float* dk, float* dv,
                              float* ws, const Geom& geo, const UnitMap& um, int64_t rows,
                              int64_t out_heads, int64_t head_rows, hipStream_t s) {
   const float scale = (float)(1.0 / sqrt((double)D));
@@ -1072,7 +1109,6 @@ static hipError_t launch_bwd(const void* q, const void* k, const void* v, const 
   const f16* Q = (const f16*)q;
   const f16* K = (const f16*)k;
   const f16* V = (const f16*)v;
-  const f16* O = (const f16*)o;
   const f16* G = (const f16*)dout;
   const int group = (int)geo.group.d;
   float* nd = ws;
@@ -1081,8 +1117,11 @@ static hipError_t launch_bwd(const void* q, const void* k, const void* v, const 
   const int64_t part0 = (2 * rows + 3) / 4 * 4;   // 16-byte aligned start of the partials
   float* dk_q = group == 1 ? dk : ws + part0;
   float* dv_q = group == 1 ? dv : ws + part0 + rows * D;
-  hipLaunchKernelGGL((fa_bwd_di_kernel<D, BF16>), dim3((unsigned)((rows + 31) / 32)), dim3(256), 0, s, O,
-                     G, lse, nd, nl, rows);
+  const RowTermArgs rt{(const f16*)o, (f16*)const_cast<void*>(dout), in.o, in.g, lse, nd, nl, rows,
+                       (int)((rows + 31) / 32)};
+  hipLaunchKernelGGL((fa_bwd_di_kernel<D, BF16>),
+                     dim3((unsigned)(rt.blocks + in.qkv.blocks[0] + in.qkv.blocks[1] + in.qkv.blocks[2])),
+                     dim3(256), 0, s, rt, in.qkv);
   // dK/dV and dQ in one launch: with units of one length it measured level
   // with two launches or slightly ahead (D = 128 non-causal, B1 H8 N4096
   // 256.4 -> 254.5 us, B4 H16 N4096 1981.8 -> 1972.3 us; same gradients bit
@@ -1095,11 +1134,9 @@ static hipError_t launch_bwd(const void* q, const void* k, const void* v, const 
     // consecutive query heads' partials
     const int64_t head_elems = head_rows * D;
     const int64_t n4 = out_heads * head_elems / 4;
-    const dim3 grid((unsigned)((n4 + 255) / 256));
-    hipLaunchKernelGGL(fa_bwd_group_sum_kernel, grid, dim3(256), 0, s, dk_q, dk, head_elems,
-                       out_heads, group);
-    hipLaunchKernelGGL(fa_bwd_group_sum_kernel, grid, dim3(256), 0, s, dv_q, dv, head_elems,
-                       out_heads, group);
+    const dim3 grid((unsigned)((n4 + 255) / 256), 2);
+    hipLaunchKernelGGL(fa_bwd_group_sum_kernel, grid, dim3(256), 0, s, dk_q, dv_q, dk, dv,
+                       head_elems, out_heads, group);
   }
   return hipGetLastError();
 }
@@ -1125,7 +1162,7 @@ namespace fa {
 namespace bwd {
 template <bool BF16>
 static int bwd_run(const void* q, const void* k, const void* v, const void* o, const void* dout,
-                   const float* lse, float* dq, float* dk, float* dv, float* workspace,
+                   const Fp32Inputs& in, const float* lse, float* dq, float* dk, float* dv, float* workspace,
                    const Geom& geo, int64_t units, int64_t rows, int64_t out_heads,
                    int64_t head_rows, int64_t D, int causal, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
@@ -1137,11 +1174,11 @@ static int bwd_run(const void* q, const void* k, const void* v, const void* o, c
   const UnitMap um = unit_map(heads, per_head, stream_topology(s), causal != 0 || geo.cu != nullptr);
   hipError_t e;
   if (D == 64) {
-    e = causal ? launch_bwd<64, true, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
-               : launch_bwd<64, false, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
+    e = causal ? launch_bwd<64, true, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
+               : launch_bwd<64, false, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
   } else {
-    e = causal ? launch_bwd<128, true, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
-               : launch_bwd<128, false, BF16>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
+    e = causal ? launch_bwd<128, true, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
+               : launch_bwd<128, false, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
   }
   return e == hipSuccess ? FA_OK : -(int)e;
 }
@@ -1149,16 +1186,16 @@ static int bwd_run(const void* q, const void* k, const void* v, const void* o, c
 static int bwd_gqa(bool bf16, const void* q, const void* k, const void* v, const void* o,
                    const void* dout, const float* lse, float* dq, float* dk, float* dv,
                    float* workspace, int64_t B, int64_t H, int64_t H_kv, int64_t N, int64_t D,
-                   int causal, void* stream) {
+                   int causal, void* stream, const Fp32Inputs& in = Fp32Inputs{}) {
   int st = fa_validate_bwd(q, k, v, o, dout, lse, dq, dk, dv, workspace, B, H, N, D);
   if (st != FA_OK) return st;
   if (H_kv <= 0 || H % H_kv != 0) return FA_ERR_KV_HEADS;
   // the partials are written and read as 16-byte vectors
   if (H_kv != H && (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) return FA_ERR_ALIGNMENT;
   const Geom geo{nullptr, (int)N, (int)H, FastDiv(H / H_kv), 0, 0};
-  return bf16 ? bwd_run<true>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, B * H,
+  return bf16 ? bwd_run<true>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, B * H,
                               B * H * N, B * H_kv, N, D, causal, stream)
-              : bwd_run<false>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, B * H,
+              : bwd_run<false>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, B * H,
                                B * H * N, B * H_kv, N, D, causal, stream);
 }
 }  // namespace bwd
@@ -1188,6 +1225,28 @@ extern "C" int fa_bwd_bf16(const void* q, const void* k, const void* v, const vo
                           causal, stream);
 }
 
+extern "C" int fa_bwd_cast_f32(const float* const f32[5], void* const h16[5], const float* lse,
+                               float* dq, float* dk, float* dv, float* workspace, int64_t B,
+                               int64_t H, int64_t H_kv, int64_t N, int64_t D, int causal, int bf16,
+                               void* stream) {
+  using namespace fa;
+  if (!f32 || !h16) return FA_ERR_NULL_POINTER;
+  // O needs no 16-bit copy: the row terms are its only use.
+  const void* o = h16[3] != nullptr ? h16[3] : (const void*)f32[3];
+  int st = fa_validate_bwd(h16[0], h16[1], h16[2], o, h16[4], lse, dq, dk, dv, workspace, B, H, N, D);
+  if (st != FA_OK) return st;
+  if (H_kv <= 0 || H % H_kv != 0) return FA_ERR_KV_HEADS;
+  for (int i = 0; i < 5; ++i)
+    if ((reinterpret_cast<uintptr_t>(f32[i]) & 15u) != 0) return FA_ERR_ALIGNMENT;
+  const int64_t nq = B * H * N * D, nkv = B * H_kv * N * D;
+  if (nq / 8 / kCastVecs + 2 * (nkv / 8 / kCastVecs) + B * H * N / 32 > (int64_t(1) << 31) - 8)
+    return FA_ERR_TOO_LARGE;
+  const int64_t n[3] = {nq, nkv, nkv};
+  const bwd::Fp32Inputs in{f32[3], f32[4], cast_jobs(f32, h16, n)};
+  return bwd::bwd_gqa(bf16 != 0, h16[0], h16[1], h16[2], o, h16[4], lse, dq, dk, dv, workspace, B,
+                      H, H_kv, N, D, causal, stream, in);
+}
+
 extern "C" int fa_bwd_varlen_f16(const void* q, const void* k, const void* v, const void* o,
                                  const void* dout, const float* lse, float* dq, float* dk,
                                  float* dv, float* workspace, const int32_t* cu_seqlens,
@@ -1200,6 +1259,6 @@ extern "C" int fa_bwd_varlen_f16(const void* q, const void* k, const void* v, co
   if (H_kv != H && (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0) return FA_ERR_ALIGNMENT;
   const fa::Geom geo{cu_seqlens, (int)max_seqlen, (int)H, fa::FastDiv(H / H_kv), (int)total,
                      (int)B};
-  return fa::bwd::bwd_run<false>(q, k, v, o, dout, lse, dq, dk, dv, workspace, geo, B * H,
+  return fa::bwd::bwd_run<false>(q, k, v, o, dout, fa::bwd::Fp32Inputs{}, lse, dq, dk, dv, workspace, geo, B * H,
                                  H * total, H_kv, total, D, causal, stream);
 }

@@ -346,6 +346,52 @@ __device__ __forceinline__ f16x2 cvt2x(float a, float b) {
   }
 }
 
+// Eight fp32 values as 16-bit operands (round to nearest even), raw bits.
+template <bool BF16>
+__device__ __forceinline__ f16x8 cvt8x(const float* __restrict__ src) {
+  const f32x4 a = *reinterpret_cast<const f32x4*>(src), b = *reinterpret_cast<const f32x4*>(src + 4);
+  const f16x2 x0 = cvt2x<BF16>(a[0], a[1]), x1 = cvt2x<BF16>(a[2], a[3]);
+  const f16x2 x2 = cvt2x<BF16>(b[0], b[1]), x3 = cvt2x<BF16>(b[2], b[3]);
+  return f16x8{x0[0], x0[1], x1[0], x1[1], x2[0], x2[1], x3[0], x3[1]};
+}
+
+// Up to three fp32 tensors to convert in one launch, `vecs` groups of eight
+// values each (16-byte aligned on both sides). Workgroups of 256 threads take
+// kCastVecs groups: first src[0]'s, then src[1]'s, then src[2]'s.
+constexpr int kCastVecs = 512;
+struct CastJobs {
+  const float* src[3];
+  f16* dst[3];
+  int64_t vecs[3];
+  int blocks[3];   // of each
+};
+
+inline CastJobs cast_jobs(const float* const src[3], void* const dst[3], const int64_t n[3]) {
+  CastJobs j;
+  for (int i = 0; i < 3; ++i) {
+    j.src[i] = src[i];
+    j.dst[i] = (f16*)dst[i];
+    j.vecs[i] = src[i] != nullptr ? n[i] / 8 : 0;
+    j.blocks[i] = (int)((j.vecs[i] + kCastVecs - 1) / kCastVecs);
+  }
+  return j;
+}
+
+template <bool BF16>
+__device__ __forceinline__ void cast_block(const CastJobs& j, int block) {
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    if (block >= 0 && block < j.blocks[t]) {
+#pragma unroll
+      for (int i = 0; i < kCastVecs / 256; ++i) {
+        const int64_t v = (int64_t)block * kCastVecs + 256 * i + threadIdx.x;
+        if (v < j.vecs[t]) reinterpret_cast<f16x8*>(j.dst[t])[v] = cvt8x<BF16>(j.src[t] + 8 * v);
+      }
+    }
+    block -= j.blocks[t];
+  }
+}
+
 // B operand (P^T) of PV k-step j from the S^T accumulators p[2] of a tile.
 __device__ __forceinline__ f16x8 pack_p(const f32x16& p, int half_sel) {
   const int b = 8 * half_sel;

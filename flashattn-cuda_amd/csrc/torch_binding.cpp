@@ -13,11 +13,10 @@
 // include/fa_mi355x.h; this file makes no HIP call of its own.
 #include <torch/extension.h>
 
-#include <limits>
-
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
+#include <array>
 #include <vector>
 
 #include "fa_mi355x.h"
@@ -31,6 +30,60 @@ void* current_stream(const torch::Tensor& t) {
 
 void check_status(int st, const char* what) {
   TORCH_CHECK(st == FA_OK, what, " failed: ", fa_status_str(st), " (status ", st, ")");
+}
+
+bool plain_f32(const torch::Tensor& t) {
+  return t.scalar_type() == torch::kFloat && t.numel() > 0 && t.is_contiguous() && !t.is_neg() &&
+         !t._is_zerotensor() &&
+         (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15u) == 0;
+}
+
+// t as a contiguous tensor of `type`, or, of a plain fp32 t, an empty one that
+// the caller fills from t; `src` then is t's data, and NULL otherwise.
+torch::Tensor operand(const torch::Tensor& t, torch::ScalarType type, const float*& src) {
+  if (plain_f32(t)) {
+    src = t.data_ptr<float>();
+    return torch::empty(t.sizes(), t.options().dtype(type));
+  }
+  src = nullptr;
+  return t.to(type).contiguous();
+}
+
+// Q, K and V as contiguous 16-bit tensors, fp32 ones converted in one launch.
+std::array<torch::Tensor, 3> operands(const torch::Tensor& Q, const torch::Tensor& K,
+                                      const torch::Tensor& V, torch::ScalarType type) {
+  const float* src[3];
+  std::array<torch::Tensor, 3> r = {operand(Q, type, src[0]), operand(K, type, src[1]),
+                                    operand(V, type, src[2])};
+  if (src[0] || src[1] || src[2]) {
+    void* dst[3] = {r[0].data_ptr(), r[1].data_ptr(), r[2].data_ptr()};
+    const int64_t n[3] = {r[0].numel(), r[1].numel(), r[2].numel()};
+    check_status(fa_cast_f32(src, dst, n, type == torch::kBFloat16, current_stream(r[0])), "fa_cast_f32");
+  }
+  return r;
+}
+
+// Sets the rows of up to three packed tensors [heads, total, ...] that belong
+// to no sequence (32-bit words per row, value).
+struct Outside {
+  torch::Tensor t;
+  int64_t words;
+  uint32_t value;
+};
+void fill_outside(const torch::Tensor& cu, int64_t max_seqlen, int64_t total,
+                  const std::vector<Outside>& bufs) {
+  void* p[3] = {};
+  int64_t heads[3] = {}, words[3] = {};
+  uint32_t value[3] = {};
+  for (size_t i = 0; i < bufs.size(); ++i) {
+    p[i] = bufs[i].t.numel() > 0 ? bufs[i].t.data_ptr() : nullptr;
+    heads[i] = bufs[i].t.size(0);
+    words[i] = bufs[i].words;
+    value[i] = bufs[i].value;
+  }
+  check_status(fa_varlen_fill_outside(cu.data_ptr<int32_t>(), cu.size(0) - 1, max_seqlen, total, p,
+                                      heads, words, value, current_stream(cu)),
+               "fa_varlen_fill_outside");
 }
 
 // variant 0: the default kernel, split over the keys where
@@ -57,9 +110,7 @@ std::pair<torch::Tensor, torch::Tensor> forward_impl(torch::Tensor Q, torch::Ten
 
   const c10::DeviceGuard guard(Q.device());
   const int64_t BH = B * H;
-  auto Qh = Q.to(torch::kHalf).reshape({BH, N, D}).contiguous();
-  auto Kh = K.to(torch::kHalf).reshape({B * Hkv, N, D}).contiguous();
-  auto Vh = V.to(torch::kHalf).reshape({B * Hkv, N, D}).contiguous();
+  auto [Qh, Kh, Vh] = operands(Q, K, V, torch::kHalf);
   auto O = torch::empty({BH, N, D}, Qh.options());
   torch::Tensor L;
   float* L_ptr = nullptr;
@@ -115,9 +166,7 @@ std::vector<torch::Tensor> forward_bf16(torch::Tensor Q, torch::Tensor K, torch:
   TORCH_CHECK(K.device() == Q.device() && V.device() == Q.device(),
               "Q/K/V must be on the same device");
   const c10::DeviceGuard guard(Q.device());
-  auto q = Q.to(torch::kBFloat16).contiguous();
-  auto k = K.to(torch::kBFloat16).contiguous();
-  auto v = V.to(torch::kBFloat16).contiguous();
+  auto [q, k, v] = operands(Q, K, V, torch::kBFloat16);
   auto O = torch::empty({B, H, N, D}, q.options());
   torch::Tensor L;
   float* L_ptr = nullptr;
@@ -153,19 +202,17 @@ std::vector<torch::Tensor> forward_varlen(torch::Tensor q, torch::Tensor k, torc
               "q/k/v/cu_seqlens must be on the same device");
   const c10::DeviceGuard guard(dev);
   const int64_t B = cu_seqlens.size(0) - 1, Hkv = k.size(0);
-  auto qh = q.to(torch::kHalf).contiguous();
-  auto kh = k.to(torch::kHalf).contiguous();
-  auto vh = v.to(torch::kHalf).contiguous();
+  auto [qh, kh, vh] = operands(q, k, v, torch::kHalf);
   auto cu = cu_seqlens.contiguous();
-  // Rows outside every sequence (past cu_seqlens[B]) are not written by the
-  // kernel: they keep O = 0 and L = -inf, the logsumexp of no keys.
-  auto O = torch::zeros({H, total, D}, qh.options());
-  auto L = torch::full({H, total}, -std::numeric_limits<float>::infinity(),
-                       qh.options().dtype(torch::kFloat));
+  auto O = torch::empty({H, total, D}, qh.options());
+  auto L = torch::empty({H, total}, qh.options().dtype(torch::kFloat));
   const int st = fa_fwd_varlen_f16(qh.data_ptr(), kh.data_ptr(), vh.data_ptr(), O.data_ptr(),
                                    L.data_ptr<float>(), cu.data_ptr<int32_t>(), B, H, Hkv,
                                    max_seqlen, total, D, causal ? 1 : 0, current_stream(qh));
   check_status(st, "fa_fwd_varlen_f16");
+  // Rows outside every sequence (past cu_seqlens[B]) are not written by the
+  // kernel: O = 0 and L = -inf there, the logsumexp of no keys.
+  fill_outside(cu, max_seqlen, total, {{O, D / 2, 0}, {L, 1, 0xff800000u}});
   return {O, L};
 }
 
@@ -201,19 +248,23 @@ static std::vector<torch::Tensor> backward_impl(torch::Tensor Q, torch::Tensor K
   const c10::DeviceGuard guard(dev);
   const int64_t BH = B * H;
   const auto in_type = bf16 ? torch::kBFloat16 : torch::kHalf;
-  auto half = [&](const torch::Tensor& t) { return t.to(in_type).contiguous(); };
-  auto Qh = half(Q), Kh = half(K), Vh = half(V), Oh = half(O), dOh = half(dO);
+  // fp32 inputs are rounded in the row-term pass (O without a copy).
+  const float* src32[5];
+  auto Qh = operand(Q, in_type, src32[0]), Kh = operand(K, in_type, src32[1]),
+       Vh = operand(V, in_type, src32[2]), dOh = operand(dO, in_type, src32[4]);
+  src32[3] = plain_f32(O) ? O.data_ptr<float>() : nullptr;
+  auto Oh = src32[3] != nullptr ? torch::Tensor() : O.to(in_type).contiguous();
   auto Lf = L.to(torch::kFloat).reshape({BH, N}).contiguous();
   auto f32 = Qh.options().dtype(torch::kFloat);
   auto dQ = torch::empty({B, H, N, D}, f32);
   auto dK = torch::empty({B, Hkv, N, D}, f32);
   auto dV = torch::empty({B, Hkv, N, D}, f32);
   auto ws = torch::empty({fa_bwd_gqa_workspace_floats(B, H, Hkv, N, D)}, f32);
-  auto entry = bf16 ? fa_bwd_bf16 : fa_bwd_gqa_f16;
-  const int st = entry(Qh.data_ptr(), Kh.data_ptr(), Vh.data_ptr(), Oh.data_ptr(), dOh.data_ptr(),
-                       Lf.data_ptr<float>(), dQ.data_ptr<float>(), dK.data_ptr<float>(),
-                       dV.data_ptr<float>(), ws.data_ptr<float>(), B, H, Hkv, N, D,
-                       causal ? 1 : 0, current_stream(Qh));
+  void* h16[5] = {Qh.data_ptr(), Kh.data_ptr(), Vh.data_ptr(), Oh.defined() ? Oh.data_ptr() : nullptr,
+                  dOh.data_ptr()};
+  const int st = fa_bwd_cast_f32(src32, h16, Lf.data_ptr<float>(), dQ.data_ptr<float>(),
+                                 dK.data_ptr<float>(), dV.data_ptr<float>(), ws.data_ptr<float>(), B,
+                                 H, Hkv, N, D, causal ? 1 : 0, bf16 ? 1 : 0, current_stream(Qh));
   check_status(st, bf16 ? "fa_bwd_bf16" : "fa_bwd_gqa_f16");
   return {dQ, dK, dV};
 }
@@ -261,24 +312,25 @@ std::vector<torch::Tensor> backward_varlen(torch::Tensor q, torch::Tensor k, tor
   const c10::DeviceGuard guard(dev);
   const int64_t B = cu_seqlens.size(0) - 1, Hkv = k.size(0);
   TORCH_CHECK(Hkv > 0 && H % Hkv == 0, "H must be a positive multiple of k/v's head count");
-  auto half = [&](const torch::Tensor& t) { return t.to(torch::kHalf).contiguous(); };
-  auto qh = half(q), kh = half(k), vh = half(v), oh = half(o), gh = half(dO);
+  auto [qh, kh, vh] = operands(q, k, v, torch::kHalf);
+  auto oh = o.to(torch::kHalf).contiguous(), gh = dO.to(torch::kHalf).contiguous();
   auto Lf = L.to(torch::kFloat).reshape({H, total}).contiguous();
   auto cu = cu_seqlens.contiguous();
   auto f32 = qh.options().dtype(torch::kFloat);
-  auto dQ = torch::zeros({H, total, D}, f32);
-  auto dK = torch::zeros({Hkv, total, D}, f32);
-  auto dV = torch::zeros({Hkv, total, D}, f32);
+  auto dQ = torch::empty({H, total, D}, f32);
+  auto dK = torch::empty({Hkv, total, D}, f32);
+  auto dV = torch::empty({Hkv, total, D}, f32);
   const int64_t wsn = fa_bwd_gqa_workspace_floats(1, H, Hkv, total > 0 ? total : 1, D);
-  // zeros: with H_kv < H the group sums also read the partials of rows
-  // outside every sequence
-  auto ws = torch::zeros({wsn}, f32);
+  auto ws = torch::empty({wsn}, f32);
   const int st = fa_bwd_varlen_f16(qh.data_ptr(), kh.data_ptr(), vh.data_ptr(), oh.data_ptr(),
                                    gh.data_ptr(), Lf.data_ptr<float>(), dQ.data_ptr<float>(),
                                    dK.data_ptr<float>(), dV.data_ptr<float>(),
                                    ws.data_ptr<float>(), cu.data_ptr<int32_t>(), B, H, Hkv,
                                    max_seqlen, total, D, causal ? 1 : 0, current_stream(qh));
   check_status(st, "fa_bwd_varlen_f16");
+  // Rows outside every sequence; with H_kv < H after the group sums, which
+  // also sum the unwritten partials of those rows.
+  fill_outside(cu, max_seqlen, total, {{dQ, D, 0}, {dK, D, 0}, {dV, D, 0}});
   return {dQ, dK, dV};
 }
 

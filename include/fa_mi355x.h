@@ -387,6 +387,36 @@ int fa_kv_append_set_bad(const void* k_new, const void* v_new, const int32_t* pa
                          void* v_pool, int32_t* bad, int64_t B, int64_t H, int64_t T, int64_t D,
                          int64_t page_size, int64_t max_pages, int64_t num_pages, void* stream);
 
+/*
+ * Rounds up to three fp32 tensors to fp16 (bf16 != 0: bfloat16) in one launch,
+ * to nearest even: dst[i] from src[i], n[i] values (a multiple of 8), both
+ * 16-byte aligned; src[i] NULL skips i. The reference casts each input with a
+ * tensor operation of its own (cuda/flash_attn_fa3_db_full.cu:366-368).
+ */
+int fa_cast_f32(const float* const src[3], void* const dst[3], const int64_t n[3], int bf16,
+                void* stream);
+
+/*
+ * fa_bwd_gqa_f16 / fa_bwd_bf16 (bf16 != 0) of inputs that come in fp32, rounded
+ * in the row-term pass: f32 and h16 hold q, k, v, o, dout. f32[i] not NULL: the
+ * fp32 tensor, and h16[i] a buffer for its 16-bit copy (o: none needed, h16[3]
+ * may be NULL); f32[i] NULL: h16[i] is the input. 16-byte aligned; everything
+ * else as in fa_bwd_gqa_f16.
+ */
+int fa_bwd_cast_f32(const float* const f32[5], void* const h16[5], const float* lse, float* dq,
+                    float* dk, float* dv, float* workspace, int64_t B, int64_t H, int64_t H_kv,
+                    int64_t N, int64_t D, int causal, int bf16, void* stream);
+
+/*
+ * Sets the rows of packed buffers that belong to no sequence of cu_seqlens
+ * (int32 [B+1], as in fa_fwd_varlen_f16; rows past max_seqlen of a sequence
+ * included): buf[i] is heads[i] x total rows of words[i] 32-bit words, each
+ * set to value[i]; buf[i] NULL skips i. No reference counterpart.
+ */
+int fa_varlen_fill_outside(const int32_t* cu_seqlens, int64_t B, int64_t max_seqlen, int64_t total,
+                           void* const buf[3], const int64_t heads[3], const int64_t words[3],
+                           const uint32_t value[3], void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -219,3 +219,26 @@ def test_gqa_backward(fa, dev, D, H, Hkv, N, causal):
     # sums of g per-head gradients: the absolute budget grows with g
     _compare([t.cpu().numpy() for t in (dQ, dK, dV)], [rQ, rK, rV], TIGHT_ATOL * g, TIGHT_RTOL,
              f"GQA H{H} Hkv{Hkv} N{N} D{D} causal={causal}")
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("B,H,Hkv,N,D", [(1, 1, 1, 1, 64), (1, 3, 1, 33, 64), (2, 4, 2, 70, 128), (1, 8, 8, 512, 64)])
+def test_fp32_inputs_are_rounded_first(fa, dev, bf16, B, H, Hkv, N, D):
+    """fp32 tensors, in any mix with 16-bit ones and in any layout, give bit for
+    bit what the same tensors rounded by torch give."""
+    dt = torch.bfloat16 if bf16 else torch.float16
+    fwd, bwd = (fa.forward_bf16, fa.backward_bf16) if bf16 else (fa.forward, fa.backward)
+    g = torch.Generator(device=dev).manual_seed(60)
+    q, k, v, do = (torch.randn(B, h, N, D, generator=g, device=dev) * 3 for h in (H, Hkv, Hkv, H))
+    q[..., 0] = 1e-6                     # an fp16 subnormal
+    O, L = fwd(q.to(dt), k.to(dt), v.to(dt), causal=True)
+    for x, r in zip(fwd(q, k, v, causal=True), (O, L)):
+        assert torch.equal(x, r)
+    want = bwd(q.to(dt), k.to(dt), v.to(dt), O, do.to(dt), L, causal=True)
+    odd = torch.empty(q.numel() + 1, device=dev)[1:].view(q.shape)   # 4-byte aligned only
+    odd.copy_(q)
+    strided = k.transpose(2, 3).contiguous().transpose(2, 3)
+    for args in ((q, k, v, O.float(), do), (q, k, v, O, do), (q.to(dt), k, v.to(dt), O.float(), do.to(dt)),
+                 (odd, strided, v.double(), O.double(), do)):
+        for x, r in zip(bwd(*args, L, causal=True), want):
+            assert torch.equal(x, r)
