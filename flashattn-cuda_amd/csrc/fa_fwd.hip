@@ -86,8 +86,7 @@ struct RowBlock {
     }
   }
 
-  // The functions below work on NB consecutive 32-key blocks of a 64-key
-  // tile, starting at block kb0 (NB = 2: the whole tile).
+  // The functions below work on the NB 32-key blocks of a tile (kb0 = 0).
 
   // S^T of the blocks: s[b] = K[32 (kb0+b) ..] Q^T.
   template <int NB>
@@ -107,7 +106,7 @@ struct RowBlock {
   // if CAUSAL, keys > the lane's query row get -inf.
   template <int NB>
   __device__ __forceinline__ void mask_all(int t, int kb0, f32x16 (&s)[NB]) const {
-    const int lane_key = t * kBC + 4 * hi;
+    const int lane_key = t * (32 * NB) + 4 * hi;
     int lim = N - 1 - lane_key;                    // live iff kofs <= lim
     if (CAUSAL) lim = min(lim, qrow - lane_key);
 #pragma unroll
@@ -123,8 +122,9 @@ struct RowBlock {
   // tiles crossing the causal diagonal); a wave-uniform branch skips the rest.
   template <int NB>
   __device__ __forceinline__ void mask(int t, int kb0, f32x16 (&s)[NB]) const {
-    const int key0 = t * kBC;
-    const bool need = (!FULL && key0 + kBC > N) || (CAUSAL && key0 + kBC - 1 > row_w);
+    constexpr int KEYS = 32 * NB;
+    const int key0 = t * KEYS;
+    const bool need = (!FULL && key0 + KEYS > N) || (CAUSAL && key0 + KEYS - 1 > row_w);
     if (need) mask_all<NB>(t, kb0, s);
   }
 
@@ -416,10 +416,9 @@ __device__ __forceinline__ f16x8 vblk_frag(lds_cp p) {
 // past the end is still issued, with an empty buffer range (it writes zeros
 // and reads no memory), so every wave issues the same number of copies per
 // tile group and vmcnt counts stay exact.
-template <int D, bool FULL>
+template <int TILE, bool FULL>
 __device__ __forceinline__ void dma_block_or_zero(const char* head, int head_bytes, int t,
                                                   bool valid, uint32_t dst, uint32_t off) {
-  constexpr int TILE = kBC * D * 2;
   const int done = valid ? t * TILE : 0;
   const int bytes = !valid ? 0 : (FULL ? TILE : min(TILE, head_bytes - done));
   dma16(make_rsrc_s(head + done, bytes), dst, off);
@@ -459,6 +458,11 @@ __device__ __forceinline__ void dma_block_or_zero(const char* head, int head_byt
 // partials normalised over its range and the range's LSE, merged by the LSE
 // combine afterwards.
 // ---------------------------------------------------------------------------
+// 32-key blocks of a tile: two, or one at D = 128 with four tile groups, whose
+// rings of 8 tiles then fit the LDS (a phase is as long as at D = 64).
+template <int D, int TG>
+constexpr int tile_blocks() { return D == 128 && TG == 4 ? 1 : 2; }
+
 // Row block qb of the head hv (split-KV: key range `split` of it); smem holds
 // 2 RING tiles.
 template <int D, bool CAUSAL, bool WRITE_L, bool FULL, int RING, bool BF16, bool SPLITKV, int TG>
@@ -467,8 +471,9 @@ fwd_pp_body(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __r
             f16* __restrict__ O, float* __restrict__ L, const HeadView& hv, int qb, int split,
             int nsplit, float c, float* __restrict__ part_o, float* __restrict__ part_lse,
             char* smem) {
-  constexpr int NB = 2;                        // 32-key blocks per tile
-  constexpr int TILE = kBC * D * 2;            // bytes of a 64-key K or V tile
+  constexpr int NB = tile_blocks<D, TG>();     // 32-key blocks per tile
+  constexpr int KEYS = 32 * NB;                // keys per tile
+  constexpr int TILE = KEYS * D * 2;           // bytes of a K or V tile
   constexpr int BLOCKS = TILE / 1024;          // 1 KiB blocks per tile
   constexpr int NRG = 8 / TG;                  // row groups (32 rows each)
   constexpr int ROWS = 32 * NRG;               // query rows of the workgroup
@@ -483,7 +488,7 @@ fwd_pp_body(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __r
   constexpr int DB = RB::DB;
   constexpr int KSTEPS = D / 16;
   constexpr int NMM = NB * KSTEPS;             // MFMAs of one QK (= of one PV)
-  constexpr int PF = D == 64 ? 8 : 4;          // operand prefetch distance, in MFMAs
+  constexpr int PF = NMM == 8 ? 8 : 4;         // operand prefetch distance, in MFMAs
   constexpr int REC = RB::REC_FLOATS;          // floats per wave record of the merge
   static_assert(!SPLITKV || (TG - 1) * NRG * REC * 4 <= 2 * RING * TILE, "merge area too small");
   const int tid = threadIdx.x;
@@ -504,7 +509,7 @@ fwd_pp_body(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __r
   rb.init(Q + head, head_bytes, lane, q0 + 32 * rg, N, c);
 
   const int kv_end = CAUSAL ? min(N, q0 + ROWS) : N;
-  int n_tiles = (kv_end + kBC - 1) / kBC;
+  int n_tiles = (kv_end + KEYS - 1) / KEYS;
   // Split-KV: this workgroup's tiles are tb .. tb + n_tiles - 1 of the row
   // block's; K/V pointers and bounds start at tile tb, masking uses absolute
   // key positions.
@@ -531,7 +536,7 @@ fwd_pp_body(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __r
   for (int i = 0; i < LOADS; ++i) dma_offsets<D>(rg * LOADS + i, lane, koff[i], voff[i]);
   // 1 KiB block b of tile t, bounded by the range (zeros past the end).
   auto dma_tile_block = [&](bool is_v, int t, uint32_t dst, uint32_t off) {
-    dma_block_or_zero<D, FULL>(is_v ? Vh : Kh, kv_bytes, t, t < n_tiles, dst, off);
+    dma_block_or_zero<TILE, FULL>(is_v ? Vh : Kh, kv_bytes, t, t < n_tiles, dst, off);
   };
   auto copy_block = [&](bool is_v, int t, int i) {
     const uint32_t at = lds0 + ((is_v ? RING : 0) + t % RING) * TILE + (rg * LOADS + i) * 1024;
@@ -599,8 +604,10 @@ fwd_pp_body(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __r
     // every accumulator is reused four MFMAs later. Without PV, QK m. QK i:
     // block i % NB, k-step i / NB. PV i: k-step i / DB, d-block i % DB: V
     // block i.
-    auto is_pv = [](int m) { return PV && (m & 3) >= 2; };
-    auto idx = [](int m) { return PV ? 2 * (m >> 2) + (m & 1) : m; };
+    // One block per tile: QK and PV alternate (a QK of its own k-step each; two
+    // in a row would wait for the accumulator).
+    auto is_pv = [](int m) { return PV && (NB == 1 ? (m & 1) == 1 : (m & 3) >= 2); };
+    auto idx = [](int m) { return !PV ? m : (NB == 1 ? m >> 1 : 2 * (m >> 2) + (m & 1)); };
     auto fetch = [&](int m) -> f16x8 {
       const int i = idx(m);
       if (is_pv(m)) return vblk_frag(vl + i * 1024);
@@ -641,7 +648,7 @@ fwd_pp_body(const f16* __restrict__ Q, const f16* __restrict__ K, const f16* __r
       wait_vmcnt<((RING - TG) / TG - 1) * 2 * LOADS>();
       return;
     }
-    rb.template mask<2>(tb + t, 0, s);
+    rb.template mask<NB>(tb + t, 0, s);
     const float m_cur = rb.m_run;
     constexpr int PAIRS = 8 * NB;
     float ex[PAIRS][2];
@@ -774,7 +781,7 @@ fa_fwd_pp_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
                  float* __restrict__ L, Geom geo, UnitMap um, float c,
                  float* __restrict__ part_o = nullptr, float* __restrict__ part_lse = nullptr,
                  int nsplit = 1) {
-  constexpr int TILE = kBC * D * 2;
+  constexpr int TILE = 32 * tile_blocks<D, TG>() * D * 2;
   constexpr int ROWS = 32 * (8 / TG);
   // K slots at [0, RING) * TILE, V slots at [RING, 2 RING) * TILE.
   __shared__ __attribute__((aligned(1024))) char smem[2 * RING * TILE];
@@ -810,20 +817,23 @@ fa_fwd_pp_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
 // Kernel variants (for fa_probe_fwd_variant; the default path picks one per
 // problem shape): the ping-pong kernel with two tile groups over 128 rows and
 // a ring of 4 tiles (204), or with four tile groups over 64 rows and a ring
-// of 8 tiles (408, D = 64: twice the workgroups for the same rows).
+// of 8 tiles (twice the workgroups for the same rows): 408 at D = 64, and 432
+// with tiles of 32 keys at D = 128.
 constexpr int kPingPong = 204;
 constexpr int kPingPong4 = 408;
+constexpr int kPingPong4K32 = 432;
 constexpr int kGuarded = 1000;   // probe flag: force the guarded (not full-tile) instance
 
 // Query rows per row block, and the multiple of N that lets every tile group
 // run the same number of whole tiles (the full-tile instance).
-static int variant_rows(int variant) { return variant == kPingPong4 ? 64 : kBR; }
+static int variant_rows(int variant) { return variant == kPingPong ? kBR : 64; }
 static int variant_full_n(int variant) { return variant == kPingPong4 ? 256 : kBR; }
 
 // Variants that exist for head dimension D and the causal flag.
 static bool variant_fits(int D, int variant, int causal) {
   if (variant == kPingPong) return true;
   if (variant == kPingPong4) return D == 64;
+  if (variant == kPingPong4K32) return D == 128;
   (void)causal;
   return false;
 }
@@ -847,6 +857,13 @@ static hipError_t launch_fwd(const void* q, const void* k, const void* v, void* 
       break;
     case kPingPong4:
       if constexpr (D == 64) {
+        hipLaunchKernelGGL((fa_fwd_pp_kernel<D, CAUSAL, WRITE_L, FULL, 8, BF16, false, 4>),
+                           grid, dim3(512), 0, stream, Q, K, V, Op, lse, geo, um, c);
+        break;
+      }
+      return hipErrorInvalidValue;
+    case kPingPong4K32:
+      if constexpr (D == 128) {
         hipLaunchKernelGGL((fa_fwd_pp_kernel<D, CAUSAL, WRITE_L, FULL, 8, BF16, false, 4>),
                            grid, dim3(512), 0, stream, Q, K, V, Op, lse, geo, um, c);
         break;
@@ -880,12 +897,29 @@ static hipError_t dispatch_wl(const void* q, const void* k, const void* v, void*
 // CUs); from one 128-row block per CU on (non-causal) or two (causal) it
 // loses (B1 H16 N2048 21.1 vs 26.5, B2 H8 N4096 causal 45.1 vs 55.5), as it
 // does for causal N = 1024 (B4 H8 12.8 vs 17.6).
-static int choose_variant(int64_t D, int causal, int64_t bh, int64_t N, int cus) {
-  if (D != 64) return kPingPong;
-  const int64_t grid = bh * ((N + kBR - 1) / kBR);
+//
+// D = 128 (us, 128-row -> 64-row workgroups with 32-key tiles): non-causal
+// while the 64-row blocks fit the CUs once (B1 H8 N1024 16.1 -> 12.6, N2048
+// 26.2 -> 23.4, B1 H4 N4096 44.5 -> 40.0; beyond, B1 H12 N1500 22.6 vs 33.4);
+// causal also up to one 128-row block per CU, of long rows, where the longest
+// block sets the time (B1 H8 N4096 49.7 -> 45.5, B1 H4 N8192 91.0 -> 80.6, B1
+// H3 N8000 83.0 -> 67.6, B1 H12 N1500 22.3 -> 18.7; not B2 H16 N1024 18.8 vs
+// 20.8, B4 H8 N700 15.2 vs 17.0, B1 H16 N2048 29.4 both). One 64-row block is
+// no more workgroups than one 128-row block.
+static int choose_by_grid(int64_t D, int causal, int64_t grid, int64_t N, int cus) {
+  if (D != 64) {
+    if (N <= 64) return kPingPong;
+    if (2 * grid <= cus) return kPingPong4K32;
+    if (causal && ((grid <= cus && N > 2048) || (4 * grid <= 3 * cus && N > 1024))) return kPingPong4K32;
+    return kPingPong;
+  }
   if (grid < cus) return kPingPong4;
   if (causal && grid == cus && N >= 2048) return kPingPong4;
   return kPingPong;
+}
+
+static int choose_variant(int64_t D, int causal, int64_t bh, int64_t N, int cus) {
+  return choose_by_grid(D, causal, bh * ((N + kBR - 1) / kBR), N, cus);
 }
 
 }  // namespace fa
@@ -907,7 +941,7 @@ static int fwd_run(const void* q, const void* k, const void* v, void* o, float* 
     // wave of one length).
     variant = geo.cu == nullptr
                   ? choose_variant(D, causal, B * geo.H, geo.N, topo.cus)
-                  : choose_variant(D, 0, geo.H * varlen_units(B, geo.total, geo.N, kBR), kBR, topo.cus);
+                  : choose_by_grid(D, 0, geo.H * varlen_units(B, geo.total, geo.N, kBR), geo.N, topo.cus);
   }
   if (!variant_fits((int)D, variant, causal)) return FA_ERR_HEAD_DIM;
   const int rows = variant_rows(variant);

@@ -65,8 +65,8 @@ int fa_probe_fwd_variant(const void* q, const void* k, const void* v, void* o, f
  * (B = 1, H = 8, N = 4096, non-causal) on the current device (0 for another
  * D). 204 = ping-pong kernel with two tile groups over 128 rows (ring of 4
  * tiles), 408 = with four tile groups over 64 rows (ring of 8 tiles,
- * D = 64); the forward picks 408 for D = 64 where 128-row workgroups leave
- * CUs idle. */
+ * D = 64); the forward picks 408 for D = 64, and 432 (the same with tiles of
+ * 32 keys) for D = 128, where 128-row workgroups leave CUs idle. */
 int fa_probe_default_variant(int64_t D);
 
 /* The variant the forward picks for bh = B*H heads of N rows on a device of
@@ -86,8 +86,8 @@ int fa_probe_splitkv_plan_cus(int64_t B, int64_t H, int64_t N, int64_t D, int ca
 int fa_probe_unit_of(int64_t heads, int64_t per_head, int nxcd, int cus, int uneven, int64_t g,
                      int* head, int* idx);
 
-/* Writes up to max_out variant codes that exist for head dimension D and the
- * causal flag into out (may be NULL) and returns how many there are. */
+/* Writes up to max_out codes of the variants with tiles of 64 keys (all but
+ * 432) that exist for head dimension D and the causal flag into out (may be NULL) and returns how many there are. */
 int fa_probe_fwd_variants(int* out, int max_out, int64_t D, int causal);
 
 /* Streams `bytes` (a multiple of 16, 16-byte aligned) from device memory at p

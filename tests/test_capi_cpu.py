@@ -394,3 +394,11 @@ def test_unit_order(capi, heads, per_head, nxcd, cus, uneven):
     assert all(len(homes[a]) == 1 for a in range(whole))
     bad = lib.fa_probe_unit_of(heads, per_head, nxcd, cus, uneven, heads * per_head, C.byref(h), C.byref(i))
     assert bad == capi.STATUS["FA_ERR_TOO_LARGE"]
+
+
+@pytest.mark.parametrize("causal,bh,N,cus,variant", [
+    (0, 8, 2048, 256, 432), (0, 9, 2048, 256, 204), (0, 8, 4096, 256, 204), (0, 1, 64, 256, 204),
+    (0, 1, 65, 256, 432), (1, 8, 4096, 256, 432), (1, 16, 4096, 256, 204), (1, 16, 2048, 256, 204),
+    (1, 12, 1500, 256, 432), (1, 24, 1024, 256, 204), (0, 8, 2048, 32, 204), (1, 1, 4096, 32, 432)])
+def test_64_row_choice_at_d128(capi, causal, bh, N, cus, variant):
+    assert capi.load().fa_probe_choose_variant(128, causal, bh, N, cus) == variant

@@ -350,6 +350,28 @@ def test_every_kernel_variant(fa, dev, D):
 
 # The 64-row kernel (408) on ragged and small causal shapes: odd block
 # counts, diagonal tiles, rows with fewer keys than one tile.
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [1, 31, 33, 64, 65, 127, 128, 129, 200, 256, 385, 1024, 1100])
+def test_64_row_d128_variant(fa, dev, causal, N):
+    """Variant 432 (D = 128, 64 rows, four tile groups of 32-key tiles) at the
+    edges of its row blocks, tiles and groups: against the oracle, O-only and
+    the guarded instance bitwise, and bf16 through the default path."""
+    B, H, D = 1, 3, 128
+    Q, K, V = make_fwd_inputs(B, H, N, D, seed=900 + N)
+    tq, tk, tv = _to_dev(dev, Q, K, V)
+    O, L = fa.probe.probe_fwd_variant(tq, tk, tv, causal, 432, True)
+    (O2,) = fa.probe.probe_fwd_variant(tq, tk, tv, causal, 432, False)
+    Og, Lg = fa.probe.probe_fwd_variant(tq, tk, tv, causal, 1432, True)
+    torch.cuda.synchronize()
+    assert torch.equal(O, O2) and torch.equal(O, Og) and torch.equal(L, Lg)
+    Or, Lr = naive_attention(half_cast(Q), half_cast(K), half_cast(V), causal=causal)
+    _check(O, L, Or, Lr, 1.0, tag=f"variant 432 N{N} causal={causal}")
+    if N > 64:
+        Od, Ld = fa.forward_bf16(tq.bfloat16(), tk.bfloat16(), tv.bfloat16(), causal=causal)
+        # P and O rounded to bf16: 1e-2 plus half a bf16 ulp below |O| = 4; and the inputs, 3 bits shorter
+        assert (Od.float() - O.float()).abs().max().item() <= 6e-2
+
+
 @pytest.mark.parametrize("N", [1, 63, 65, 127, 129, 191, 257, 383, 449, 577, 1023, 1089])
 def test_64_row_kernel_ragged_causal(fa, dev, N):
     Q, K, V = make_fwd_inputs(1, 2, N, 64, seed=1000 + N, amp=1.0)
