@@ -33,8 +33,6 @@
 // bf16 187 -> 179, B1 H8 N4096 D64 137.5 -> 135.3).
 #include <hip/hip_runtime.h>
 
-#include <stdlib.h>
-
 #include <math.h>
 #include <stdint.h>
 
@@ -48,7 +46,9 @@ namespace fa {
 namespace bwd {
 
 constexpr int kBQ = 64;     // rows of a streamed tile
-constexpr int kBlk = 128;   // rows owned by a workgroup (32 per wave)
+// Rows owned by a workgroup of two (TG = 2) or four (TG = 4) waves per 32 rows.
+template <int TG>
+constexpr int block_rows() { return TG == 2 ? 128 : 64; }
 
 // Per-lane source offset of 1 KiB block b of a 64-row tile (see t_swz).
 template <int D>
@@ -220,6 +220,19 @@ __device__ __forceinline__ void group_reduce(char* smem, int grp, int slot, int 
   }
 }
 
+// The partials of a key (query) block's waves into wave `wi` = kw (wi = qw) of
+// group 0: two groups of the same rows' halves (TG = 2), or four waves, two of
+// each group (TG = 4). True in the waves that hold the sums.
+template <int TG, int NA, int DB>
+__device__ __forceinline__ bool reduce_rows(char* smem, int grp, int wi, int lane,
+                                            f32x16 (&a)[NA][DB]) {
+  group_reduce<NA, DB>(smem, grp, wi, lane, a);
+  if constexpr (TG == 2) return grp == 0;
+  // Group 0's waves 2 and 3 into its waves 0 and 1 (group 1 idles).
+  group_reduce<NA, DB>(smem, grp == 0 ? wi >> 1 : 2, wi & 1, lane, a);
+  return grp == 0 && wi < 2;
+}
+
 // ---------------------------------------------------------------------------
 // dK/dV and dQ bodies (8 waves). A dK/dV workgroup owns 128 keys of one
 // (b, h): wave w holds K^T and V^T of keys k0 + 32 (w % 4) .. +31 as register
@@ -248,6 +261,11 @@ __device__ __forceinline__ void group_reduce(char* smem, int grp, int slot, int 
 // staged data, and the barriers keep them one phase apart and sync each
 // group's four waves on their copies.
 //
+// That is TG = 2. With TG = 4 a workgroup owns 64 keys (queries), so a launch
+// has twice the workgroups: each group takes whole tiles, group 0 the even and
+// group 1 the odd ones, in a ring of its own, two waves hold each 32 keys and
+// take a tile's two halves, and four partial sums are added at the end.
+//
 // D = 64 (rows 32 g .. +31 of each part are its 1 KiB blocks 4 g .. 4 g + 3):
 // tile j's stage is read from S(j - 1), which loads tile j's A operands into registers (M(j) then
 // issues its score products without LDS waits), to M(j + 1), which reads its
@@ -258,21 +276,21 @@ __device__ __forceinline__ void group_reduce(char* smem, int grp, int slot, int 
 // ---------------------------------------------------------------------------
 constexpr int kPPStages = 4;
 
-template <int D>
+template <int D, int TG>
 constexpr int dkdv_pp_smem() {
   constexpr int STAGE = 2 * (kBQ * D * 2) + 2048;
   constexpr int RED = 4 * 2 * (D / 32) * 16 * 64 * 4;
-  return kPPStages * STAGE > RED ? kPPStages * STAGE : RED;
+  return TG / 2 * kPPStages * STAGE > RED ? TG / 2 * kPPStages * STAGE : RED;
 }
 
-template <int D>
+template <int D, int TG>
 constexpr int dq_pp_smem() {
   constexpr int STAGE = 2 * (kBQ * D * 2);
   constexpr int RED = 4 * (D / 32) * 16 * 64 * 4;
-  return kPPStages * STAGE > RED ? kPPStages * STAGE : RED;
+  return TG / 2 * kPPStages * STAGE > RED ? TG / 2 * kPPStages * STAGE : RED;
 }
 
-template <int D, bool CAUSAL, bool BF16>
+template <int D, bool CAUSAL, bool BF16, int TG>
 __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f16* __restrict__ K,
                                              const f16* __restrict__ V, const f16* __restrict__ dO,
                                              const float* __restrict__ NL,
@@ -283,19 +301,20 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
-  constexpr int PER = OWN / 2;                 // blocks per wave of a group's copies
+  constexpr int PER = TG == 2 ? OWN / 2 : OWN; // blocks per wave of a group's copies
   constexpr int KSTEPS = D / 16, DB = D / 32;
+  constexpr int R = kPPStages;                 // stages of a ring (TG = 4: one per group)
   // Q | dO | row vectors (group g: L at +512 g, D_i at +512 g + 256)
   constexpr int STAGE = 2 * TILE + 2048;
-  static_assert(kPPStages * STAGE <= 160 * 1024, "LDS");
+  static_assert(TG / 2 * R * STAGE <= 160 * 1024, "LDS");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kw = wave & 3;
-  const int grp = wave >> 2;                   // also this group's query half of a tile
-  const int qb = grp;
+  const int wi = wave & 3, grp = wave >> 2;
+  const int kw = TG == 2 ? wi : wi & 1;        // keys 32 kw .. +31 of the block
+  const int qb = TG == 2 ? grp : wi >> 1;      // query half of a tile
   const int hi = lane >> 5;
-  const int k0 = kb * kBlk;
+  const int k0 = kb * block_rows<TG>();
   const int key = k0 + 32 * kw + (lane & 31);
 
   const int N = hv.n;
@@ -318,35 +337,41 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
 
   const int n_qt = (N + kBQ - 1) / kBQ;
   const int t0 = CAUSAL ? k0 / kBQ : 0;   // earlier query tiles see none of these keys
-  const int T = n_qt - t0;                 // tiles of this workgroup (>= 1)
+  // Steps of this workgroup (>= 1); its groups take a half each of tile j in
+  // step j, or (TG = 4) tiles 2 j and 2 j + 1, the last possibly past the end.
+  const int T = TG == 2 ? n_qt - t0 : (n_qt - t0 + 1) / 2;
+  auto tile_of = [&](int j) { return TG == 2 ? t0 + j : t0 + 2 * j + grp; };
 
   const uint32_t lds0 = lds_addr(smem);
-  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
-  auto stage_of = [&](int j) { return smem + (j % kPPStages) * STAGE; };
-  // This group's half of tile t into stage st: wave kw copies two blocks of
-  // part kw / 2; waves 0 and 1 also copy the 64-row L and D_i vectors.
-  auto issue_own = [&](int t, int st) {
-    const uint32_t base = lds0 + st * STAGE;
-    const char* src = kw < 2 ? Qh : Gh;
+  const uint32_t half0 = lds0 + qb * 32 * 2 * D;   // this wave's rows of a part
+  auto slot_of = [&](int j) { return (TG == 2 ? 0 : grp * R) + j % R; };
+  const int rv0 = 2 * TILE + (TG == 2 ? 512 * grp : 0);   // this group's row vectors
+  // This group's half (TG = 4: whole) of step j's tile: wave wi copies PER
+  // blocks of part wi / 2; waves 0 and 1 also copy the 64-row L and D_i
+  // vectors.
+  auto issue_own = [&](int j) {
+    const uint32_t base = lds0 + slot_of(j) * STAGE;
+    const char* src = wi < 2 ? Qh : Gh;
+    const int t = tile_of(j);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int b = OWN * grp + PER * (kw & 1) + i;
-      copy_block<D>(src, head_bytes, t, base + (kw >> 1) * TILE + b * 1024, block_offset<D>(b, lane));
+      const int b = (TG == 2 ? OWN * grp : 0) + PER * (wi & 1) + i;
+      copy_block<D>(src, head_bytes, t, base + (wi >> 1) * TILE + b * 1024, block_offset<D>(b, lane));
     }
-    if (kw == 0) copy_rowvec(Lh, N, t, base + 2 * TILE + 512 * grp, lane);
-    if (kw == 1) copy_rowvec(Dh, N, t, base + 2 * TILE + 512 * grp + 256, lane);
+    if (wi == 0) copy_rowvec(Lh, N, t, base + rv0, lane);
+    if (wi == 1) copy_rowvec(Dh, N, t, base + rv0 + 256, lane);
   };
   // Copies run three tiles ahead: at the end of M phase j tile j + 1 must
   // have landed, and tile j + 2's copies (this wave's last issue) may still
   // be in flight.
   auto wait_next = [&](bool later_in_flight) {
     if (!later_in_flight) wait_vmem();
-    else if (kw < 2) wait_vmcnt<PER + 1>();
+    else if (wi < 2) wait_vmcnt<PER + 1>();
     else wait_vmcnt<PER>();
   };
-  issue_own(t0, 0);
-  if (T > 1) issue_own(t0 + 1, 1);
-  if (T > 2) issue_own(t0 + 2, 2);
+  issue_own(0);
+  if (T > 1) issue_own(1);
+  if (T > 2) issue_own(2);
   wait_next(T > 2);
   __syncthreads();
 
@@ -354,7 +379,7 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   f16x8 pb[2], gb[2];       // its packed P and dS (B operands of the two k-steps)
   f16x8 af[KSTEPS][2];      // A operands of its next score products (Q, dO rows)
   auto load_a = [&](int j) {   // of relative tile j
-    const uint32_t rb = row_base<D>(half0 + (j % kPPStages) * STAGE, lane);
+    const uint32_t rb = row_base<D>(half0 + slot_of(j) * STAGE, lane);
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
       af[kk][0] = load_row_frag<D>(rb, 0, kk);
@@ -383,7 +408,7 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   // j); then the wait for the copies this wave started in S(j - 1).
   auto mphase = [&](int j, auto with_c, auto with_a) {
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
-    const uint32_t sc = col_base<D>(half0 + ((j + kPPStages - 1) % kPPStages) * STAGE, lane);
+    const uint32_t sc = col_base<D>(half0 + slot_of(j + R - 1) * STAGE, lane);
     f16x8 cf[KSTEPS][2];
     if constexpr (WC) {
       load_c(sc, 0, cf[0]);
@@ -403,10 +428,9 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   // tile j - 1, whose last reads were this group's M phase j), P and dS into
   // pb, gb, and tile j + 1's A operands.
   auto sphase = [&](int j) {
-    if (j + 3 < T) issue_own(t0 + j + 3, (j + 3) % kPPStages);
-    const char* sb = stage_of(j);
-    const int qt0 = (t0 + j) * kBQ;
-    const float* ls = reinterpret_cast<const float*>(sb + 2 * TILE + 512 * grp);
+    if (j + 3 < T) issue_own(j + 3);
+    const int qt0 = tile_of(j) * kBQ;
+    const float* ls = reinterpret_cast<const float*>(smem + slot_of(j) * STAGE + rv0);
     const float* nds = ls + 64;
     // Row vectors first (LDS reads return in order), then the next tile's A
     // operands, which land while the VALU work below runs.
@@ -463,14 +487,13 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   mphase(T, BT{}, BF{});   // C of the last tile
   __syncthreads();
   if (grp == 0) __syncthreads();   // phase 2T + 1: group 0 waits
-  group_reduce<2, DB>(smem, grp, kw, lane, acc);
-  if (grp == 0) {
+  if (reduce_rows<TG, 2, DB>(smem, grp, wi, lane, acc)) {
     store_transposed<D>(dV + head, N, k0 + 32 * kw, lane, acc[0], 1.f);
     store_transposed<D>(dK + head, N, k0 + 32 * kw, lane, acc[1], scale);
   }
 }
 
-template <int D, bool CAUSAL, bool BF16>
+template <int D, bool CAUSAL, bool BF16, int TG>
 __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16* __restrict__ K,
                                            const f16* __restrict__ V, const f16* __restrict__ dO,
                                            const float* __restrict__ NL,
@@ -481,18 +504,19 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
-  constexpr int PER = OWN / 2;                 // blocks per wave of a group's copies
+  constexpr int PER = TG == 2 ? OWN / 2 : OWN; // blocks per wave of a group's copies
   constexpr int KSTEPS = D / 16, DB = D / 32;
+  constexpr int R = kPPStages;
   constexpr int STAGE = 2 * TILE;              // K | V
-  static_assert(kPPStages * STAGE <= 160 * 1024, "LDS");
+  static_assert(TG / 2 * R * STAGE <= 160 * 1024, "LDS");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int qw = wave & 3;
-  const int grp = wave >> 2;                   // also this group's key half of a tile
-  const int half = grp;
+  const int wi = wave & 3, grp = wave >> 2;
+  const int qw = TG == 2 ? wi : wi & 1;        // queries 32 qw .. +31 of the block
+  const int half = TG == 2 ? grp : wi >> 1;    // key half of a tile
   const int hi = lane >> 5;
-  const int q0 = qblk * kBlk;
+  const int q0 = qblk * block_rows<TG>();
   const int query = q0 + 32 * qw + (lane & 31);
 
   const int N = hv.n;
@@ -512,21 +536,25 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
 #pragma unroll
   for (int db = 0; db < DB; ++db) acc[0][db] = f32x16{};
 
-  const int kv_end = CAUSAL ? min(N, q0 + kBlk) : N;
-  const int T = (kv_end + kBQ - 1) / kBQ;   // >= 1
+  const int kv_end = CAUSAL ? min(N, q0 + block_rows<TG>()) : N;
+  const int n_kt = (kv_end + kBQ - 1) / kBQ;   // >= 1
+  // Steps: as in the dK/dV body.
+  const int T = TG == 2 ? n_kt : (n_kt + 1) / 2;
+  auto tile_of = [&](int j) { return TG == 2 ? j : 2 * j + grp; };
   // rows past N (last block only) and, causal, keys after the wave's first query
   const bool rows_edge = q0 + 32 * qw + 32 > N;
 
   const uint32_t lds0 = lds_addr(smem);
-  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
-  // This group's half of tile t into stage st: wave qw copies two blocks of
-  // part qw / 2.
-  auto issue_own = [&](int t, int st) {
-    const uint32_t base = lds0 + st * STAGE;
+  const uint32_t half0 = lds0 + half * 32 * 2 * D;   // this wave's rows of a part
+  auto slot_of = [&](int j) { return (TG == 2 ? 0 : grp * R) + j % R; };
+  // This group's half (TG = 4: whole) of step j's tile: wave wi copies PER
+  // blocks of part wi / 2.
+  auto issue_own = [&](int j) {
+    const uint32_t base = lds0 + slot_of(j) * STAGE;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int b = OWN * grp + PER * (qw & 1) + i;
-      copy_block<D>(qw < 2 ? Kh : Vh, head_bytes, t, base + (qw >> 1) * TILE + b * 1024,
+      const int b = (TG == 2 ? OWN * grp : 0) + PER * (wi & 1) + i;
+      copy_block<D>(wi < 2 ? Kh : Vh, head_bytes, tile_of(j), base + (wi >> 1) * TILE + b * 1024,
                     block_offset<D>(b, lane));
     }
   };
@@ -535,9 +563,9 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
     if (later_in_flight) wait_vmcnt<PER>();
     else wait_vmem();
   };
-  issue_own(0, 0);
-  if (T > 1) issue_own(1, 1);
-  if (T > 2) issue_own(2, 2);
+  issue_own(0);
+  if (T > 1) issue_own(1);
+  if (T > 2) issue_own(2);
   wait_next(T > 2);
   __syncthreads();
 
@@ -545,7 +573,7 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   f16x8 gb[2];
   f16x8 af[KSTEPS][2];   // A operands of the next score products (K, V rows)
   auto load_a = [&](int j) {
-    const uint32_t rb = row_base<D>(half0 + (j % kPPStages) * STAGE, lane);
+    const uint32_t rb = row_base<D>(half0 + slot_of(j) * STAGE, lane);
 #pragma unroll
     for (int kk = 0; kk < KSTEPS; ++kk) {
       af[kk][0] = load_row_frag<D>(rb, 0, kk);
@@ -562,7 +590,7 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   auto load_c = [&](uint32_t cb, int kk) { return load_col_frag<D>(cb, 0, kk / DB, kk % DB); };
   auto mphase = [&](int j, auto with_c, auto with_a) {
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
-    const uint32_t sc = col_base<D>(half0 + ((j + kPPStages - 1) % kPPStages) * STAGE, lane);
+    const uint32_t sc = col_base<D>(half0 + slot_of(j + R - 1) * STAGE, lane);
     f16x8 cf[KSTEPS];
     if constexpr (WC) {
       cf[0] = load_c(sc, 0);
@@ -579,9 +607,9 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
     wait_next(j + 2 < T);
   };
   auto sphase = [&](int j) {
-    if (j + 3 < T) issue_own(j + 3, (j + 3) % kPPStages);
+    if (j + 3 < T) issue_own(j + 3);
     if (j + 1 < T) load_a(j + 1);
-    const int kt0 = j * kBQ;
+    const int kt0 = tile_of(j) * kBQ;
     f32x16 p;
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = exp2_hw(fmaf(s[r], c, nl));
@@ -624,8 +652,8 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   mphase(T, BT{}, BF{});   // C of the last tile
   __syncthreads();
   if (grp == 0) __syncthreads();   // phase 2T + 1: group 0 waits
-  group_reduce<1, DB>(smem, grp, qw, lane, acc);
-  if (grp == 0) store_transposed<D>(dQ + head, N, q0 + 32 * qw, lane, acc[0], scale);
+  if (reduce_rows<TG, 1, DB>(smem, grp, wi, lane, acc))
+    store_transposed<D>(dQ + head, N, q0 + 32 * qw, lane, acc[0], scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -641,27 +669,31 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
 //   * LDS: a ring of three tiles (99 KiB with the row vectors; the final
 //     reduction takes 128). S(j) starts the copies of tile j + 2 into the slot
 //     of tile j - 1 (last read in M(j)), and its end waits for those of S(j - 1):
-//     every copy has two phases to land, issued from the VALU phase.
+//     every copy has two phases to land, issued from the VALU phase. TG = 4 has
+//     two slots per group: S(j) starts and awaits tile j + 1.
 // A group copies and reads only its own 32-row half of every part (rows
 // 32 g .. +31 are 1 KiB blocks 8 g .. 8 g + 7).
 // ---------------------------------------------------------------------------
-template <int D>
+template <int TG>
+constexpr int pp128_slots() { return TG == 2 ? 3 : 4; }   // tiles in LDS (TG = 4: two per group)
+
+template <int D, int TG>
 constexpr int dkdv_pp128_smem() {
   constexpr int TILE = kBQ * D * 2;
-  constexpr int RING = 3 * (2 * TILE) + 3 * 1024;
+  constexpr int RING = pp128_slots<TG>() * (2 * TILE + 1024);
   constexpr int RED = 4 * 2 * (D / 32) * 16 * 64 * 4;
   return RING > RED ? RING : RED;
 }
 
-template <int D>
+template <int D, int TG>
 constexpr int dq_pp128_smem() {
   constexpr int TILE = kBQ * D * 2;
-  constexpr int RING = 3 * (2 * TILE);
+  constexpr int RING = pp128_slots<TG>() * (2 * TILE);
   constexpr int RED = 4 * (D / 32) * 16 * 64 * 4;
   return RING > RED ? RING : RED;
 }
 
-template <int D, bool CAUSAL, bool BF16>
+template <int D, bool CAUSAL, bool BF16, int TG>
 __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
                                                 const f16* __restrict__ K,
                                                 const f16* __restrict__ V,
@@ -675,21 +707,22 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
-  constexpr int PER = OWN / 2;                 // blocks per wave of a tile
+  constexpr int PER = TG == 2 ? OWN / 2 : OWN; // blocks per wave of a tile
   constexpr int KSTEPS = D / 16, DB = D / 32;
   constexpr int SLOT = 2 * TILE;               // Q | dO
-  constexpr int R0 = 3 * SLOT;                 // row vectors: group g L at +512 g, -D_i +256
-  static_assert(R0 + 3 * 1024 <= dkdv_pp128_smem<D>() && dkdv_pp128_smem<D>() <= 160 * 1024,
+  constexpr int R = TG == 2 ? 3 : 2;           // slots of a ring (TG = 4: one per group)
+  constexpr int R0 = pp128_slots<TG>() * SLOT; // row vectors: group g L at +512 g, -D_i +256
+  static_assert(R0 + pp128_slots<TG>() * 1024 <= dkdv_pp128_smem<D, TG>() && dkdv_pp128_smem<D, TG>() <= 160 * 1024,
                 "ring inside the buffer, LDS");
   static_assert(2 * KSTEPS == 2 * 2 * DB, "C and A take the same number of steps");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int kw = wave & 3;
-  const int grp = wave >> 2;                   // also this group's query half of a tile
-  const int qb = grp;
+  const int wi = wave & 3, grp = wave >> 2;
+  const int kw = TG == 2 ? wi : wi & 1;        // keys 32 kw .. +31 of the block
+  const int qb = TG == 2 ? grp : wi >> 1;      // query half of a tile
   const int hi = lane >> 5;
-  const int k0 = kb * kBlk;
+  const int k0 = kb * block_rows<TG>();
 
   const int N = hv.n;
   const size_t head = hv.q;
@@ -711,37 +744,44 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
 
   const int n_qt = (N + kBQ - 1) / kBQ;
   const int t0 = CAUSAL ? k0 / kBQ : 0;   // earlier query tiles see none of these keys
-  const int T = n_qt - t0;                 // tiles of this workgroup (>= 1)
+  // Steps of this workgroup (>= 1); its groups take a half each of tile j in
+  // step j, or (TG = 4) tiles 2 j and 2 j + 1, the last possibly past the end.
+  const int T = TG == 2 ? n_qt - t0 : (n_qt - t0 + 1) / 2;
+  auto tile_of = [&](int j) { return TG == 2 ? t0 + j : t0 + 2 * j + grp; };
 
   const uint32_t lds0 = lds_addr(smem);
-  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
-  // Wave kw copies blocks 8 grp + 4 (kw & 1) .. +3 of part kw >> 1 (Q or dO)
-  // of relative tile j, waves 0 and 1 also its row vectors; the per-lane
-  // offsets are recomputed per copy (volatile lane id: held across the loop
-  // they would take registers the body needs).
+  const uint32_t half0 = lds0 + qb * 32 * 2 * D;   // this wave's rows of a part
+  auto slot_of = [&](int j) { return (TG == 2 ? 0 : grp * R) + j % R; };
+  const int rv0 = R0 + (TG == 2 ? 512 * grp : 0);   // this group's row vectors
+  // Wave wi copies PER blocks of part wi >> 1 (Q or dO) of this group's half
+  // (TG = 4: whole) of step j's tile, waves 0 and 1 also its row vectors; the
+  // per-lane offsets are recomputed per copy (volatile lane id: held across
+  // the loop they would take registers the body needs).
   auto issue_tile = [&](int j) {
     int ln;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-    const char* src = kw < 2 ? Qh : Gh;
-    const uint32_t base = lds0 + (j % 3) * SLOT + (kw >> 1) * TILE;
+    const char* src = wi < 2 ? Qh : Gh;
+    const int t = tile_of(j);
+    const uint32_t base = lds0 + slot_of(j) * SLOT + (wi >> 1) * TILE;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int b = OWN * grp + PER * (kw & 1) + i;
-      copy_block<D>(src, head_bytes, t0 + j, base + b * 1024, block_offset<D>(b, ln));
+      const int b = (TG == 2 ? OWN * grp : 0) + PER * (wi & 1) + i;
+      copy_block<D>(src, head_bytes, t, base + b * 1024, block_offset<D>(b, ln));
     }
-    const uint32_t rv = lds0 + R0 + (j % 3) * 1024 + 512 * grp;
-    if (kw == 0) copy_rowvec(Lh, N, t0 + j, rv, ln);
-    if (kw == 1) copy_rowvec(Dh, N, t0 + j, rv + 256, ln);
+    const uint32_t rv = lds0 + rv0 + slot_of(j) * 1024;
+    if (wi == 0) copy_rowvec(Lh, N, t, rv, ln);
+    if (wi == 1) copy_rowvec(Dh, N, t, rv + 256, ln);
   };
   // All copies but those of the last tile issued (if `last` was).
   auto wait_for = [&](bool last) {
     if (!last) wait_vmem();
-    else if (kw < 2) wait_vmcnt<PER + 1>();
+    else if (wi < 2) wait_vmcnt<PER + 1>();
     else wait_vmcnt<PER>();
   };
+  constexpr int AHEAD = R - 1;   // S(j) starts the copies of tile j + AHEAD
   issue_tile(0);
-  if (T > 1) issue_tile(1);
-  wait_for(T > 1);
+  if (AHEAD > 1 && T > 1) issue_tile(1);
+  wait_for(AHEAD > 1 && T > 1);
   __syncthreads();
 
   f32x16 s = {}, dp = {};   // this wave's scores of its current tile
@@ -752,8 +792,8 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   auto mphase = [&](int j, auto with_c, auto with_a) {
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
     constexpr int X0 = WC ? 0 : KSTEPS, X1 = WA ? 2 * KSTEPS : KSTEPS;
-    const uint32_t sc = col_base<D>(half0 + ((j + 2) % 3) * SLOT, lane);   // tile j - 1
-    const uint32_t sa = row_base<D>(half0 + (j % 3) * SLOT, lane);         // tile j
+    const uint32_t sc = col_base<D>(half0 + slot_of(j + R - 1) * SLOT, lane);   // tile j - 1
+    const uint32_t sa = row_base<D>(half0 + slot_of(j) * SLOT, lane);           // tile j
     f16x8 f[2 * KSTEPS][2];
     auto load = [&](auto xi) {
       constexpr int x = decltype(xi)::value;
@@ -793,10 +833,10 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   // pb, gb; at the end, the wait for the copies of S(j - 1) (tile j + 1:
   // M(j + 1) reads it).
   auto sphase = [&](int j) {
-    const bool more = j + 2 < T;
-    if (more) issue_tile(j + 2);
-    const int qt0 = (t0 + j) * kBQ;
-    const float* ls = reinterpret_cast<const float*>(smem + R0 + (j % 3) * 1024 + 512 * grp);
+    const bool more = j + AHEAD < T;
+    if (more) issue_tile(j + AHEAD);
+    const int qt0 = tile_of(j) * kBQ;
+    const float* ls = reinterpret_cast<const float*>(smem + rv0 + slot_of(j) * 1024);
     const float* nds = ls + 64;
     f32x16 p, g;
 #pragma unroll
@@ -828,7 +868,7 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
       pb[h] = pack_px<BF16>(p, h);
       gb[h] = pack_px<BF16>(g, h);
     }
-    wait_for(more);
+    wait_for(AHEAD > 1 && more);
   };
   auto pin_s = [&] { asm volatile("" : "+v"(s), "+v"(dp)); };
   auto pin_p = [&] { asm volatile("" : "+v"(pb[0]), "+v"(pb[1]), "+v"(gb[0]), "+v"(gb[1])); };
@@ -855,14 +895,13 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   if (grp == 0) __syncthreads();   // phase 2T + 1: group 0 waits
   int ln;   // the lane id again (not held across the loop)
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-  group_reduce<2, DB>(smem, grp, kw, ln, acc);
-  if (grp == 0) {
+  if (reduce_rows<TG, 2, DB>(smem, grp, wi, ln, acc)) {
     store_transposed<D>(dV + head, N, k0 + 32 * kw, ln, acc[0], 1.f);
     store_transposed<D>(dK + head, N, k0 + 32 * kw, ln, acc[1], scale);
   }
 }
 
-template <int D, bool CAUSAL, bool BF16>
+template <int D, bool CAUSAL, bool BF16, int TG>
 __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f16* __restrict__ K,
                                               const f16* __restrict__ V,
                                               const f16* __restrict__ dO,
@@ -874,19 +913,20 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
   constexpr int TILE = kBQ * D * 2;
   constexpr int BLOCKS = TILE / 1024;
   constexpr int OWN = BLOCKS / 2;              // blocks of a 32-row half
-  constexpr int PER = OWN / 2;                 // blocks per wave of a tile
+  constexpr int PER = TG == 2 ? OWN / 2 : OWN; // blocks per wave of a tile
   constexpr int KSTEPS = D / 16, DB = D / 32;
   constexpr int SLOT = 2 * TILE;               // K | V
-  static_assert(3 * SLOT <= dq_pp128_smem<D>() && dq_pp128_smem<D>() <= 160 * 1024,
-                "ring inside the buffer, LDS");
+  constexpr int R = TG == 2 ? 3 : 2;           // slots of a ring (TG = 4: one per group)
+  static_assert(pp128_slots<TG>() * SLOT <= dq_pp128_smem<D, TG>() &&
+                dq_pp128_smem<D, TG>() <= 160 * 1024, "ring inside the buffer, LDS");
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int qw = wave & 3;
-  const int grp = wave >> 2;                   // also this group's key half of a tile
-  const int half = grp;
+  const int wi = wave & 3, grp = wave >> 2;
+  const int qw = TG == 2 ? wi : wi & 1;        // queries 32 qw .. +31 of the block
+  const int half = TG == 2 ? grp : wi >> 1;    // key half of a tile
   const int hi = lane >> 5;
-  const int q0 = qblk * kBlk;
+  const int q0 = qblk * block_rows<TG>();
   const int query = q0 + 32 * qw + (lane & 31);
 
   const int N = hv.n;
@@ -905,31 +945,37 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
 #pragma unroll
   for (int db = 0; db < DB; ++db) acc[0][db] = f32x16{};
 
-  const int kv_end = CAUSAL ? min(N, q0 + kBlk) : N;
-  const int T = (kv_end + kBQ - 1) / kBQ;   // >= 1
+  const int kv_end = CAUSAL ? min(N, q0 + block_rows<TG>()) : N;
+  const int n_kt = (kv_end + kBQ - 1) / kBQ;   // >= 1
+  // Steps: as in the dK/dV body.
+  const int T = TG == 2 ? n_kt : (n_kt + 1) / 2;
+  auto tile_of = [&](int j) { return TG == 2 ? j : 2 * j + grp; };
   // rows past N (last block only) and, causal, keys after the wave's first query
   const bool rows_edge = q0 + 32 * qw + 32 > N;
 
   const uint32_t lds0 = lds_addr(smem);
-  const uint32_t half0 = lds0 + grp * 32 * 2 * D;   // this group's rows of a part
-  // Wave qw copies blocks 8 grp + 4 (qw & 1) .. +3 of part qw >> 1 (K or V).
+  const uint32_t half0 = lds0 + half * 32 * 2 * D;   // this wave's rows of a part
+  auto slot_of = [&](int j) { return (TG == 2 ? 0 : grp * R) + j % R; };
+  // Wave wi copies PER blocks of part wi >> 1 (K or V) of this group's half
+  // (TG = 4: whole) of step j's tile.
   auto issue_tile = [&](int j) {
     int ln;
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-    const uint32_t base = lds0 + (j % 3) * SLOT + (qw >> 1) * TILE;
+    const uint32_t base = lds0 + slot_of(j) * SLOT + (wi >> 1) * TILE;
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      const int b = OWN * grp + PER * (qw & 1) + i;
-      copy_block<D>(qw < 2 ? Kh : Vh, head_bytes, j, base + b * 1024, block_offset<D>(b, ln));
+      const int b = (TG == 2 ? OWN * grp : 0) + PER * (wi & 1) + i;
+      copy_block<D>(wi < 2 ? Kh : Vh, head_bytes, tile_of(j), base + b * 1024, block_offset<D>(b, ln));
     }
   };
   auto wait_for = [&](bool last) {   // all copies but those of the last tile issued
     if (last) wait_vmcnt<PER>();
     else wait_vmem();
   };
+  constexpr int AHEAD = R - 1;   // S(j) starts the copies of tile j + AHEAD
   issue_tile(0);
-  if (T > 1) issue_tile(1);
-  wait_for(T > 1);
+  if (AHEAD > 1 && T > 1) issue_tile(1);
+  wait_for(AHEAD > 1 && T > 1);
   __syncthreads();
 
   f32x16 s = {}, dp = {};
@@ -940,8 +986,8 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
     constexpr bool WC = decltype(with_c)::value, WA = decltype(with_a)::value;
     constexpr int CX = 2 * DB;   // C steps
     constexpr int X0 = WC ? 0 : CX, X1 = WA ? CX + KSTEPS : CX;
-    const uint32_t sc = col_base<D>(half0 + ((j + 2) % 3) * SLOT, lane);   // tile j - 1
-    const uint32_t sa = row_base<D>(half0 + (j % 3) * SLOT, lane);         // tile j
+    const uint32_t sc = col_base<D>(half0 + slot_of(j + R - 1) * SLOT, lane);   // tile j - 1
+    const uint32_t sa = row_base<D>(half0 + slot_of(j) * SLOT, lane);           // tile j
     f16x8 f[CX + KSTEPS][2];
     auto load = [&](auto xi) {
       constexpr int x = decltype(xi)::value;
@@ -968,9 +1014,9 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
     __builtin_amdgcn_sched_barrier(0);
   };
   auto sphase = [&](int j) {
-    const bool more = j + 2 < T;
-    if (more) issue_tile(j + 2);
-    const int kt0 = j * kBQ;
+    const bool more = j + AHEAD < T;
+    if (more) issue_tile(j + AHEAD);
+    const int kt0 = tile_of(j) * kBQ;
     f32x16 p;
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = exp2_hw(fmaf(s[r], c, nl));
@@ -988,7 +1034,7 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
     for (int r = 0; r < 16; ++r) g[r] = p[r] * (dp[r] + dq_i);
 #pragma unroll
     for (int h = 0; h < 2; ++h) gb[h] = pack_px<BF16>(g, h);
-    wait_for(more);
+    wait_for(AHEAD > 1 && more);
   };
   auto pin_s = [&] { asm volatile("" : "+v"(s), "+v"(dp)); };
   auto pin_p = [&] { asm volatile("" : "+v"(gb[0]), "+v"(gb[1])); };
@@ -1013,8 +1059,8 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
   mphase(T, BT{}, BF{});   // C of the last tile
   __syncthreads();
   if (grp == 0) __syncthreads();   // phase 2T + 1: group 0 waits
-  group_reduce<1, DB>(smem, grp, qw, lane, acc);
-  if (grp == 0) store_transposed<D>(dQ + head, N, q0 + 32 * qw, lane, acc[0], scale);
+  if (reduce_rows<TG, 1, DB>(smem, grp, wi, lane, acc))
+    store_transposed<D>(dQ + head, N, q0 + 32 * qw, lane, acc[0], scale);
 }
 
 // dK/dV and dQ in one launch (both bodies take 8 waves and share one LDS
@@ -1025,7 +1071,7 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
 // halves are not interleaved: a dK/dV unit takes 4/3 of a dQ unit's time, and
 // where each CU gets one of both, two dK/dV units on one CU are the longest
 // (B1 H8 N4096 D64 non-causal 136 us, interleaved 150).
-template <int D, bool CAUSAL, bool BF16>
+template <int D, bool CAUSAL, bool BF16, int TG>
 __global__ void __launch_bounds__(512)
 fa_bwd_fused_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
                     const f16* __restrict__ V, const f16* __restrict__ dO,
@@ -1033,8 +1079,9 @@ fa_bwd_fused_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
                     float* __restrict__ dK, float* __restrict__ dV, float* __restrict__ dQ,
                     Geom geo, UnitMap um, float c, float scale) {
   // One LDS buffer serves whichever body this workgroup runs.
-  constexpr int SK = D == 64 ? dkdv_pp_smem<D>() : dkdv_pp128_smem<D>();
-  constexpr int SQ = D == 64 ? dq_pp_smem<D>() : dq_pp128_smem<D>();
+  constexpr int SK = D == 64 ? dkdv_pp_smem<D, TG>() : dkdv_pp128_smem<D, TG>();
+  constexpr int SQ = D == 64 ? dq_pp_smem<D, TG>() : dq_pp128_smem<D, TG>();
+  constexpr int ROWS = block_rows<TG>();
   __shared__ __attribute__((aligned(1024))) char smem[SK > SQ ? SK : SQ];
   const int total = um.heads * um.per_head;
   const bool dq_role = (int)blockIdx.x >= total;
@@ -1042,7 +1089,7 @@ fa_bwd_fused_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
   HeadView hv;
   int kb = un.idx;
   if (geo.cu != nullptr) {
-    const SeqBlock sb = varlen_block(geo, un.idx, kBlk, threadIdx.x & 63);
+    const SeqBlock sb = varlen_block(geo, un.idx, ROWS, threadIdx.x & 63);
     if (sb.n == 0) return;   // the grid is a bound on the units (whole workgroup)
     hv = seq_view<D>(geo, un.head, sb.start, sb.n);
     kb = sb.block;
@@ -1050,18 +1097,18 @@ fa_bwd_fused_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
     hv = dense_view<D>(geo, un.head);
   }
   // Causal: the first key blocks and the last query blocks are the longest.
-  const int qblk = CAUSAL ? (hv.n + kBlk - 1) / kBlk - 1 - kb : kb;
+  const int qblk = CAUSAL ? (hv.n + ROWS - 1) / ROWS - 1 - kb : kb;
   if (!dq_role) {
     if constexpr (D == 64) {
-      dkdv_body_pp<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dK, dV, hv, kb, c, scale, smem);
+      dkdv_body_pp<D, CAUSAL, BF16, TG>(Q, K, V, dO, NL, ND, dK, dV, hv, kb, c, scale, smem);
     } else {
-      dkdv_body_pp128<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dK, dV, hv, kb, c, scale, smem);
+      dkdv_body_pp128<D, CAUSAL, BF16, TG>(Q, K, V, dO, NL, ND, dK, dV, hv, kb, c, scale, smem);
     }
   } else {
     if constexpr (D == 64) {
-      dq_body_pp<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dQ, hv, qblk, c, scale, smem);
+      dq_body_pp<D, CAUSAL, BF16, TG>(Q, K, V, dO, NL, ND, dQ, hv, qblk, c, scale, smem);
     } else {
-      dq_body_pp128<D, CAUSAL, BF16>(Q, K, V, dO, NL, ND, dQ, hv, qblk, c, scale, smem);
+      dq_body_pp128<D, CAUSAL, BF16, TG>(Q, K, V, dO, NL, ND, dQ, hv, qblk, c, scale, smem);
     }
   }
 }
@@ -1102,7 +1149,7 @@ struct Fp32Inputs {
 template <int D, bool CAUSAL, bool BF16>
 static hipError_t launch_bwd(const void* q, const void* k, const void* v, const void* o,
                              const void* dout, const Fp32Inputs& in, const float* lse, float* dq, float* dk, float* dv,
-                             float* ws, const Geom& geo, const UnitMap& um, int64_t rows,
+                             float* ws, const Geom& geo, const UnitMap& um, bool rows4, int64_t rows,
                              int64_t out_heads, int64_t head_rows, hipStream_t s) {
   const float scale = (float)(1.0 / sqrt((double)D));
   const float c = scale * kLog2e;
@@ -1126,9 +1173,14 @@ static hipError_t launch_bwd(const void* q, const void* k, const void* v, const 
   // with two launches or slightly ahead (D = 128 non-causal, B1 H8 N4096
   // 256.4 -> 254.5 us, B4 H16 N4096 1981.8 -> 1972.3 us; same gradients bit
   // for bit), and a causal head's short and long units even out.
-  hipLaunchKernelGGL((fa_bwd_fused_kernel<D, CAUSAL, BF16>),
-                     dim3(2u * um.heads * um.per_head), dim3(512), 0, s, Q, K, V, G,
-                     nl, nd, dk_q, dv_q, dq, geo, um, c, scale);
+  const dim3 grid(2u * um.heads * um.per_head);
+  if (rows4) {
+    hipLaunchKernelGGL((fa_bwd_fused_kernel<D, CAUSAL, BF16, 4>), grid, dim3(512), 0, s, Q, K, V, G,
+                       nl, nd, dk_q, dv_q, dq, geo, um, c, scale);
+  } else {
+    hipLaunchKernelGGL((fa_bwd_fused_kernel<D, CAUSAL, BF16, 2>), grid, dim3(512), 0, s, Q, K, V, G,
+                       nl, nd, dk_q, dv_q, dq, geo, um, c, scale);
+  }
   if (group > 1) {
     // out_heads KV heads of head_rows rows, each the sum of `group`
     // consecutive query heads' partials
@@ -1166,19 +1218,32 @@ static int bwd_run(const void* q, const void* k, const void* v, const void* o, c
                    const Geom& geo, int64_t units, int64_t rows, int64_t out_heads,
                    int64_t head_rows, int64_t D, int causal, void* stream) {
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const Topology topo = stream_topology(s);
   // Units of a head: its blocks (varlen: a bound on those of its sequences).
-  const int64_t per_head = geo.cu == nullptr ? (geo.N + kBlk - 1) / kBlk
-                                             : varlen_units(geo.B, geo.total, geo.N, kBlk);
   const int64_t heads = geo.cu == nullptr ? units : geo.H;
+  auto blocks_of = [&](int br) {
+    return geo.cu == nullptr ? (int64_t)(geo.N + br - 1) / br
+                             : varlen_units(geo.B, geo.total, geo.N, br);
+  };
+  // 64-row blocks where 128-row ones fill half of the CUs at most, or, causal
+  // and of long rows, all of them once (the longest block then sets the time).
+  // us, 128 -> 64 rows: D = 64 B1 H8 N1024 24.8 -> 18.4, B1 H4 N2048 39.0 ->
+  // 28.2, causal B1 H8 N2048 40.3 -> 32.7, B1 H4 N4000 86.2 -> 49.9; D = 128
+  // 37.6 -> 29.3, 60.1 -> 44.6, 63.4 -> 50.8, 112.2 -> 81.3. Beyond: B1 H8 N1500
+  // D = 64 (192 workgroups) 37.0 vs 39.2, causal B2 H16 N512 (256) 19.3 vs 20.7,
+  // B1 H8 N4096 132.9 vs 144.6, causal 84.5 vs 89.1.
+  const int64_t wide = 2 * heads * blocks_of(block_rows<2>());
+  const bool rows4 = 2 * wide <= topo.cus || (causal && wide <= topo.cus && geo.N >= 1024);
+  const int64_t per_head = blocks_of(rows4 ? block_rows<4>() : block_rows<2>());
   if (2 * heads * per_head > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
-  const UnitMap um = unit_map(heads, per_head, stream_topology(s), causal != 0 || geo.cu != nullptr);
+  const UnitMap um = unit_map(heads, per_head, topo, causal != 0 || geo.cu != nullptr);
   hipError_t e;
   if (D == 64) {
-    e = causal ? launch_bwd<64, true, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
-               : launch_bwd<64, false, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
+    e = causal ? launch_bwd<64, true, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows4, rows, out_heads, head_rows, s)
+               : launch_bwd<64, false, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows4, rows, out_heads, head_rows, s);
   } else {
-    e = causal ? launch_bwd<128, true, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s)
-               : launch_bwd<128, false, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows, out_heads, head_rows, s);
+    e = causal ? launch_bwd<128, true, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows4, rows, out_heads, head_rows, s)
+               : launch_bwd<128, false, BF16>(q, k, v, o, dout, in, lse, dq, dk, dv, workspace, geo, um, rows4, rows, out_heads, head_rows, s);
   }
   return e == hipSuccess ? FA_OK : -(int)e;
 }

@@ -242,3 +242,23 @@ def test_fp32_inputs_are_rounded_first(fa, dev, bf16, B, H, Hkv, N, D):
                  (odd, strided, v.double(), O.double(), do)):
         for x, r in zip(bwd(*args, L, causal=True), want):
             assert torch.equal(x, r)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [1, 33, 64, 65, 127, 129, 200, 321])
+@pytest.mark.parametrize("B,H", [(16, 16), (1, 2)])
+def test_block_widths(fa, dev, D, causal, N, B, H):
+    """Both workgroup widths (256 heads run 128-row blocks, 2 heads 64-row ones)
+    at the edges of their blocks, tiles and tile pairs."""
+    rng = np.random.default_rng(N)
+    Q, K, V, dO = (rng.standard_normal((B, H, N, D)).astype(np.float16) for _ in range(4))
+    tq, tk, tv, tg = (torch.from_numpy(x).to(dev) for x in (Q, K, V, dO))
+    O, L = fa.forward(tq, tk, tv, causal=causal)
+    got = [x.cpu().numpy() for x in fa.backward(tq, tk, tv, O, tg, L, causal=causal)]
+    heads = [(0, 0)] if B == 1 else [(0, 0), (7, 9), (15, 15)]
+    for b, h in heads:
+        ref = naive_attention_backward(*(x[b:b + 1, h:h + 1].astype(np.float32) for x in (Q, K, V, dO)), causal)
+        for name, x, r in zip(("dQ", "dK", "dV"), got, ref):
+            err = np.abs(x[b:b + 1, h:h + 1] - r)
+            assert (err <= 5e-3 + 5e-3 * np.abs(r)).all(), f"{name} N{N} D{D} causal={causal}: {err.max():.3e}"

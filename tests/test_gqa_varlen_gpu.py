@@ -110,7 +110,8 @@ def test_varlen_many_sequences(fa, dev, B, causal):
     (64 and 256 sequences a pass, at most 512 counted), with empty sequences,
     one long one last, and a head count that no XCD count divides; forward
     against the oracle, gradients against the dense backward of the sequence
-    (the same arithmetic on the same tiles: equal bit for bit)."""
+    (the same products; fp32 sums of up to 300 terms perhaps in another order:
+    300 x 2^-24 of the largest gradient)."""
     H, D = 3, 64
     rng = np.random.default_rng(B)
     lengths = [int(x) for x in rng.integers(0, 40, B)]
@@ -134,7 +135,7 @@ def test_varlen_many_sequences(fa, dev, B, causal):
         if b % 37 == 0 or b == B - 1:
             one = [x[None, :, s].contiguous() for x in (q, k, v, O, g, L)]
             for x, r in zip(grads, fa.backward(*one, causal=causal)):
-                assert torch.equal(x[:, s], r[0]), f"seq {b} (n={n})"
+                assert (x[:, s] - r[0]).abs().max() <= 2e-5 * r.abs().max(), f"seq {b} (n={n})"
 
 
 @pytest.mark.parametrize("cu,most,inside", [
