@@ -109,16 +109,16 @@ __device__ __forceinline__ void load_row_operand(const f16* head, int n, int row
   }
 }
 
-// Store a C-layout accumulator pair-block acc[DB] (rows = 32 d of each block,
-// columns = 32 rows of the output) as fp32 rows out[row][d], scaled.
-template <int D>
+// Store the first NDB blocks of a C-layout accumulator acc[DB] (rows = 32 d of
+// each block, columns = 32 rows of the output) as fp32 rows out[row][d], scaled.
+template <int D, int NDB>
 __device__ __forceinline__ void store_transposed(float* out, int n, int row0, int lane,
                                                  const f32x16 (&acc)[D / 32], float scale) {
   const int row = row0 + (lane & 31);
   if (row >= n) return;
   float* dst = out + (size_t)row * D + 4 * (lane >> 5);
 #pragma unroll
-  for (int db = 0; db < D / 32; ++db) {
+  for (int db = 0; db < NDB; ++db) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       f32x4 v = {acc[db][4 * g] * scale, acc[db][4 * g + 1] * scale, acc[db][4 * g + 2] * scale,
@@ -193,44 +193,74 @@ fa_bwd_di_kernel(RowTermArgs a, CastJobs jobs) {
   }
 }
 
-// Partial accumulators of the second wave group, added into the first's
-// through LDS (lane-major, conflict-free): wave slot w, NA arrays of DB
-// blocks of 16 registers.
-template <int NA, int DB>
-__device__ __forceinline__ void group_reduce(char* smem, int grp, int slot, int lane,
-                                             f32x16 (&a)[NA][DB]) {
-  float* buf = reinterpret_cast<float*>(smem) + (size_t)slot * NA * DB * 16 * 64 + lane;
-  __syncthreads();   // every wave is done with the staging buffers
-  if (grp == 1) {
+// Accumulator block x of NA arrays of DB blocks, to and from LDS in 16-byte
+// accesses (lane-major, conflict-free).
+constexpr int kAccBytes = 64 * 16 * 4;   // of a wave's block
+
+__device__ __forceinline__ void put_block(char* at, int lane, const f32x16& a) {
+  f32x4* p = reinterpret_cast<f32x4*>(at) + lane;
 #pragma unroll
-    for (int x = 0; x < NA; ++x)
+  for (int q = 0; q < 4; ++q) p[64 * q] = f32x4{a[4 * q], a[4 * q + 1], a[4 * q + 2], a[4 * q + 3]};
+}
+
+__device__ __forceinline__ void add_block(const char* at, int lane, f32x16& a) {
+  const f32x4* p = reinterpret_cast<const f32x4*>(at) + lane;
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+  for (int q = 0; q < 4; ++q) {
+    const f32x4 v = p[64 * q];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) buf[((x * DB + db) * 16 + r) * 64] = a[x][db][r];
-  }
-  __syncthreads();
-  if (grp == 0) {
-#pragma unroll
-    for (int x = 0; x < NA; ++x)
-#pragma unroll
-      for (int db = 0; db < DB; ++db)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) a[x][db][r] += buf[((x * DB + db) * 16 + r) * 64];
+    for (int e = 0; e < 4; ++e) a[4 * q + e] += v[e];
   }
 }
 
-// The partials of a key (query) block's waves into wave `wi` = kw (wi = qw) of
-// group 0: two groups of the same rows' halves (TG = 2), or four waves, two of
-// each group (TG = 4). True in the waves that hold the sums.
+// Sums of the partials of the waves that hold the same keys (queries). The two
+// groups trade halves, so all eight waves add and store: of the NA x DB blocks
+// group 0 ends with the sums of the first half and group 1 with those of the
+// second, either in blocks 0 .. HALF - 1 of `a`. (Group 0 adding and storing
+// everything, in 4-byte accesses, took B1 H32 N2000 D128 causal 174.9 us, this
+// 173.2; long equal units do not notice.) With TG = 4, waves 2 and 3 of a group then send theirs to waves 0
+// and 1. True in the waves that hold sums.
 template <int TG, int NA, int DB>
 __device__ __forceinline__ bool reduce_rows(char* smem, int grp, int wi, int lane,
                                             f32x16 (&a)[NA][DB]) {
-  group_reduce<NA, DB>(smem, grp, wi, lane, a);
-  if constexpr (TG == 2) return grp == 0;
-  // Group 0's waves 2 and 3 into its waves 0 and 1 (group 1 idles).
-  group_reduce<NA, DB>(smem, grp == 0 ? wi >> 1 : 2, wi & 1, lane, a);
-  return grp == 0 && wi < 2;
+  constexpr int HALF = NA * DB / 2;
+  char* mine = smem + (grp * 4 + wi) * HALF * kAccBytes;          // written by this wave
+  const char* other = smem + ((grp ^ 1) * 4 + wi) * HALF * kAccBytes;
+  __syncthreads();   // every wave is done with the staging buffers
+  // Selects, not branches: a branch over which block is meant would make the
+  // compiler index the accumulators and keep them in scratch.
+  static_for<0, HALF>([&](auto xi) {
+    constexpr int x = decltype(xi)::value, y = x + HALF;
+    f32x16 send;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float lo = a[x / DB][x % DB][r], hi = a[y / DB][y % DB][r];
+      send[r] = grp == 0 ? hi : lo;
+      a[x / DB][x % DB][r] = grp == 0 ? lo : hi;
+    }
+    put_block(mine + x * kAccBytes, lane, send);
+  });
+  __syncthreads();
+  static_for<0, HALF>([&](auto xi) {
+    constexpr int x = decltype(xi)::value;
+    add_block(other + x * kAccBytes, lane, a[x / DB][x % DB]);
+  });
+  if constexpr (TG == 2) return true;
+  __syncthreads();
+  if (wi >= 2) {
+    static_for<0, HALF>([&](auto xi) {
+      constexpr int x = decltype(xi)::value;
+      put_block(mine + x * kAccBytes, lane, a[x / DB][x % DB]);
+    });
+  }
+  __syncthreads();
+  if (wi >= 2) return false;
+  const char* upper = smem + (grp * 4 + wi + 2) * HALF * kAccBytes;
+  static_for<0, HALF>([&](auto xi) {
+    constexpr int x = decltype(xi)::value;
+    add_block(upper + x * kAccBytes, lane, a[x / DB][x % DB]);
+  });
+  return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -244,7 +274,7 @@ __device__ __forceinline__ bool reduce_rows(char* smem, int grp, int wi, int lan
 //
 // The two wave groups (waves 0-3 and 4-7) hold the same keys (dK/dV) or
 // queries (dQ), each takes one 32-row half of every tile, their partial sums
-// are added through LDS at the end (group_reduce), and they run one phase
+// are added through LDS at the end (reduce_rows), and they run one phase
 // apart. Each tile's work splits into the score products A (S and dP
 // MFMAs), the VALU part B (P, dS, packed as B operands) and the gradient
 // products C; a group's matrix phase M(j) issues C of its tile j - 1 and A
@@ -488,8 +518,9 @@ __device__ __forceinline__ void dkdv_body_pp(const f16* __restrict__ Q, const f1
   __syncthreads();
   if (grp == 0) __syncthreads();   // phase 2T + 1: group 0 waits
   if (reduce_rows<TG, 2, DB>(smem, grp, wi, lane, acc)) {
-    store_transposed<D>(dV + head, N, k0 + 32 * kw, lane, acc[0], 1.f);
-    store_transposed<D>(dK + head, N, k0 + 32 * kw, lane, acc[1], scale);
+    // group 0 has dV, group 1 dK
+    store_transposed<D, DB>((grp == 0 ? dV : dK) + head, N, k0 + 32 * kw, lane, acc[0],
+                            grp == 0 ? 1.f : scale);
   }
 }
 
@@ -652,8 +683,10 @@ __device__ __forceinline__ void dq_body_pp(const f16* __restrict__ Q, const f16*
   mphase(T, BT{}, BF{});   // C of the last tile
   __syncthreads();
   if (grp == 0) __syncthreads();   // phase 2T + 1: group 0 waits
-  if (reduce_rows<TG, 1, DB>(smem, grp, wi, lane, acc))
-    store_transposed<D>(dQ + head, N, q0 + 32 * qw, lane, acc[0], scale);
+  if (reduce_rows<TG, 1, DB>(smem, grp, wi, lane, acc)) {
+    // group 1 has the upper half of the columns
+    store_transposed<D, DB / 2>(dQ + head + grp * (D / 2), N, q0 + 32 * qw, lane, acc[0], scale);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -896,8 +929,9 @@ __device__ __forceinline__ void dkdv_body_pp128(const f16* __restrict__ Q,
   int ln;   // the lane id again (not held across the loop)
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
   if (reduce_rows<TG, 2, DB>(smem, grp, wi, ln, acc)) {
-    store_transposed<D>(dV + head, N, k0 + 32 * kw, ln, acc[0], 1.f);
-    store_transposed<D>(dK + head, N, k0 + 32 * kw, ln, acc[1], scale);
+    // group 0 has dV, group 1 dK
+    store_transposed<D, DB>((grp == 0 ? dV : dK) + head, N, k0 + 32 * kw, ln, acc[0],
+                            grp == 0 ? 1.f : scale);
   }
 }
 
@@ -1059,8 +1093,10 @@ __device__ __forceinline__ void dq_body_pp128(const f16* __restrict__ Q, const f
   mphase(T, BT{}, BF{});   // C of the last tile
   __syncthreads();
   if (grp == 0) __syncthreads();   // phase 2T + 1: group 0 waits
-  if (reduce_rows<TG, 1, DB>(smem, grp, wi, lane, acc))
-    store_transposed<D>(dQ + head, N, q0 + 32 * qw, lane, acc[0], scale);
+  if (reduce_rows<TG, 1, DB>(smem, grp, wi, lane, acc)) {
+    // group 1 has the upper half of the columns
+    store_transposed<D, DB / 2>(dQ + head + grp * (D / 2), N, q0 + 32 * qw, lane, acc[0], scale);
+  }
 }
 
 // dK/dV and dQ in one launch (both bodies take 8 waves and share one LDS
