@@ -10,8 +10,8 @@
 // page are 16*D*2 contiguous bytes (4 KiB at D=128), copied into LDS as
 // contiguous 1 KiB requests.
 //
-// Split kernel: one workgroup (W = 4 or 8 waves) per (split, KV head, up to 16
-// query heads of its group, sequence); wave w walks pages p0+w, p0+w+W, ... and
+// Split kernel: one workgroup (4 waves) per (split, KV head, up to 16 query
+// heads of its group, sequence); wave w walks pages p0+w, p0+w+4, ... and
 // computes the scores of every head of the workgroup and their PV products
 // on the matrix cores, so a page is read once per KV head. Each wave keeps
 // its own running max/sum and fp32 partial output per head; the waves merge
@@ -21,16 +21,17 @@
 #include <math.h>
 #include <stdint.h>
 
-#include <algorithm>
 #include <mutex>
 
 #include "fa_mi355x.h"
+#include "fa_probe.h"
 #include "fa_tile.hpp"
 
 namespace fa {
 
 constexpr int kPage = 16;
-constexpr int kRankSeqs = 256;   // batches up to this size are ordered by length
+constexpr int kDecThreads = 256;
+constexpr int kDecWaves = kDecThreads / 64;
 
 // Element types of q, the pools and O: fp16, or bf16 (BF16 = true). The
 // matrix products take them as 16-bit operands with fp32 accumulation; P is
@@ -51,12 +52,12 @@ struct DecT<true> {
 // is dispatched first) takes the sequence of rank z by decreasing
 // context length, ties by index. The longest splits then start first and the
 // shortest fill the tail instead of a long sequence dispatched last running
-// alone. Ranks of B <= kRankSeqs contexts are computed from a copy in LDS;
+// alone. Ranks of B <= kDecThreads contexts are computed from a copy in LDS;
 // larger batches keep the identity order. Invalid (negative) lengths rank
 // like any other value and are flagged by the caller as before.
 __device__ __forceinline__ int sequence_of_rank(const int32_t* __restrict__ ctx_lens, int B, int z,
                                                 int* sh_ctx, int* sh_seq) {
-  if (B > kRankSeqs || B == 1) return z;
+  if (B > kDecThreads || B == 1) return z;
   const int t = threadIdx.x;
   if (t < B) sh_ctx[t] = ctx_lens[t];
   __syncthreads();
@@ -73,7 +74,7 @@ __device__ __forceinline__ int sequence_of_rank(const int32_t* __restrict__ ctx_
   return *sh_seq;
 }
 
-// Split kernel, on the matrix cores: one workgroup (W waves) per (split, KV
+// Split kernel, on the matrix cores: one workgroup (4 waves) per (split, KV
 // head, up to 16 of the query heads that share it, sequence). A wave copies each
 // page's K and V rows of the KV head into LDS (1 KiB per copy instruction,
 // contiguous in the pool, non-temporal), then
@@ -144,8 +145,8 @@ __device__ __forceinline__ float sum_cols(float x) {   // sum over the 4 lane gr
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
-template <int D, bool BF16, int W>
-__global__ void __launch_bounds__(64 * W)
+template <int D, bool BF16>
+__global__ void __launch_bounds__(kDecThreads)
 fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
                        const typename DecT<BF16>::e* __restrict__ kpool,
                        const typename DecT<BF16>::e* __restrict__ vpool,
@@ -155,18 +156,17 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
                        float* __restrict__ lse_out, int H, int Hkv, int max_pages,
                        int num_pages, int S, int ordered, float c) {
   using T = DecT<BF16>;
-  static_assert(64 * W >= kRankSeqs, "one thread per ranked sequence");
   constexpr int PAGE = kPage * D * 2;   // bytes of one head's page
   constexpr int CPR = D / 8;            // 16-byte chunks per token row
   constexpr int KB = D / 32;            // k-steps of S = K Q^T
   constexpr int DB = D / 16;            // 16-column blocks of O^T
   constexpr int NC = PAGE / 1024;       // 1 KiB copies per page and pool
-  static_assert(W * 16 * D * 4 <= W * 4 * PAGE, "merge area within the slots");
-  __shared__ __attribute__((aligned(1024))) char smem[W * 4 * PAGE];
-  __shared__ float sh_m[W][16];
-  __shared__ float sh_l[W][16];
+  static_assert(kDecWaves * 16 * D * 4 <= kDecWaves * 4 * PAGE, "merge area within the slots");
+  __shared__ __attribute__((aligned(1024))) char smem[kDecWaves * 4 * PAGE];
+  __shared__ float sh_m[kDecWaves][16];
+  __shared__ float sh_l[kDecWaves][16];
   __shared__ int sh_bad;
-  __shared__ int sh_ctx[kRankSeqs];
+  __shared__ int sh_ctx[kDecThreads];
   __shared__ int sh_seq;
 
   const int s = blockIdx.x;
@@ -219,13 +219,13 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   }
   const uint32_t lds0 = lds_addr(smem) + (uint32_t)(wave * 4 * PAGE);   // this wave's two slots
   const int32_t* pt = page_table + (size_t)b * max_pages;
-  // Page ids of the wave's pages p0 + wave + W k, 64 at a time: lane i of
+  // Page ids of the wave's pages p0 + wave + 4 k, 64 at a time: lane i of
   // pidv holds the id of page k = 64 j + i, read with readlane (a page
   // table load per page would wait for every copy in flight before it).
   int pidv = -1;
   auto page_id = [&](int k) -> int {
     if ((k & 63) == 0) {
-      const int pi = p0 + wave + W * (k + lane);
+      const int pi = p0 + wave + 4 * (k + lane);
       pidv = pi < p1 ? pt[pi] : -1;
     }
     return __builtin_amdgcn_readlane(pidv, k & 63);
@@ -254,8 +254,8 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   int p = p0 + wave;
   int sl = 0, k = 0;
   bool ok = p < p1 && issue(0, 0);
-  for (; p < p1; p += W, sl ^= 1, ++k) {
-    const int pn = p + W;
+  for (; p < p1; p += kDecWaves, sl ^= 1, ++k) {
+    const int pn = p + kDecWaves;
     const bool ok_n = pn < p1 && issue(k + 1, sl ^ 1);
     if (ok_n) wait_vmcnt<2 * NC>(); else wait_vmem();
     if (!ok) { bad = true; ok = ok_n; continue; }
@@ -326,7 +326,7 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   wait_vmem();
   if (bad) sh_bad = 1;
   __syncthreads();
-  float* sh_o = reinterpret_cast<float*>(smem);   // [W][16][D]
+  float* sh_o = reinterpret_cast<float*>(smem);   // [kDecWaves][16][D]
   if (col < G) {
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -337,15 +337,15 @@ fa_decode_split_kernel(const typename DecT<BF16>::e* __restrict__ q,
   __syncthreads();
 
   // Thread x merges column x % D of head x / D across the waves.
-  for (int x = tid; x < G * D; x += 64 * W) {
+  for (int x = tid; x < G * D; x += kDecThreads) {
     const int g = x / D, d = x % D;
     float M = sh_m[0][g];
 #pragma unroll
-    for (int w = 1; w < W; ++w) M = fmaxf(M, sh_m[w][g]);
+    for (int w = 1; w < kDecWaves; ++w) M = fmaxf(M, sh_m[w][g]);
     float acc = 0.f, z = 0.f;
     if (M != -INFINITY) {
 #pragma unroll
-      for (int w = 0; w < W; ++w) {
+      for (int w = 0; w < kDecWaves; ++w) {
         const float e = (sh_m[w][g] == -INFINITY) ? 0.f : exp2_hw(sh_m[w][g] - M);
         acc += e * sh_o[(w * 16 + g) * D + d];
         z += e * sh_l[w][g];
@@ -440,6 +440,18 @@ fa_lse_combine_kernel(const float* __restrict__ part_o, const float* __restrict_
 }  // namespace fa
 
 namespace fa {
+// Workgroups along y: one per KV head and 16 of its query heads.
+static int64_t decode_head_groups(int64_t H, int64_t Hkv) { return Hkv * ((H / Hkv + 15) / 16); }
+
+// Whether a split launch takes the sequences longest first. Where every
+// workgroup is resident at once their order does not matter, and the ranking
+// is left out: a workgroup's LDS lets two of them share a CU at D = 128, four
+// at D = 64.
+static bool decode_ordered(int64_t B, int64_t H, int64_t Hkv, int64_t D, int64_t num_splits,
+                           int cus) {
+  return B * decode_head_groups(H, Hkv) * num_splits > (D == 64 ? 4 : 2) * (int64_t)cus;
+}
+
 // Split pass with query heads h reading pool head h / (H / Hkv); arguments
 // already validated. With o (num_splits 1) the kernel writes the result
 // itself and the partials are not used.
@@ -453,34 +465,16 @@ static int decode_split(const void* q, const void* k_pool, const void* v_pool,
   if (o == nullptr && (!part_o || !part_lse)) return FA_ERR_NULL_POINTER;
   const float c = (float)(1.0 / sqrt((double)D)) * kLog2e;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int cus = stream_topology(s).cus;
   // One workgroup per (split, KV head, 16 of its query heads, sequence).
-  const int64_t group = H / Hkv;
-  const dim3 grid((unsigned)num_splits, (unsigned)(Hkv * ((group + 15) / 16)), (unsigned)B);
-  const int64_t wgs = (int64_t)grid.x * grid.y * grid.z;
-  // A wave has at most two pages in flight and its loop takes about 0.9 us a
-  // page however idle the chip is, so what a launch reads a second is set by
-  // its waves; LDS holds 8 at D = 128. Where the workgroups do not fill the
-  // CUs twice, eight waves each instead of four (us, 4 -> 8: B1 32 over 8
-  // heads, 32000 tokens, 16 splits 43.2 -> 30.1; B32, 2000 tokens, one split
-  // 44.6 -> 41.0), given a page for each; beyond that the smaller workgroups
-  // overlap their starts and ends better (B32 H32 of 1600 tokens 77.0 vs 71.9).
-  const int64_t pages = (max_pages + num_splits - 1) / num_splits;   // of a split, at most
-  const int W = wgs <= 2 * cus && pages >= 8 ? 8 : 4;
-  // Every workgroup resident at once: their order does not matter.
-  const int ordered = wgs * W > (D == 64 ? 16 : 8) * (int64_t)cus;
-#define FA_DECODE_SPLIT(DD, WW)                                                                    \
-  hipLaunchKernelGGL((fa_decode_split_kernel<DD, BF16, WW>), grid, dim3(64 * WW), 0, s,            \
+  const dim3 grid((unsigned)num_splits, (unsigned)decode_head_groups(H, Hkv), (unsigned)B);
+  const int ordered = decode_ordered(B, H, Hkv, D, num_splits, stream_topology(s).cus);
+#define FA_DECODE_SPLIT(DD)                                                                        \
+  hipLaunchKernelGGL((fa_decode_split_kernel<DD, BF16>), grid, dim3(kDecThreads), 0, s,            \
                      (const E*)q, (const E*)k_pool, (const E*)v_pool, page_table, ctx_lens, part_o, \
                      part_lse, (E*)o, lse, (int)H, (int)Hkv, (int)max_pages, (int)num_pages,       \
                      (int)num_splits, ordered, c)
-  if (D == 128) {
-    if (W == 8) FA_DECODE_SPLIT(128, 8);
-    else FA_DECODE_SPLIT(128, 4);
-  } else {
-    if (W == 8) FA_DECODE_SPLIT(64, 8);
-    else FA_DECODE_SPLIT(64, 4);
-  }
+  if (D == 128) FA_DECODE_SPLIT(128);
+  else FA_DECODE_SPLIT(64);
 #undef FA_DECODE_SPLIT
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? FA_OK : -(int)e;
@@ -512,6 +506,12 @@ static int lse_combine(const float* part_o, const float* part_lse, int64_t B, in
 }
 }  // namespace fa
 
+extern "C" int fa_probe_decode_ordered(int64_t B, int64_t H, int64_t H_kv, int64_t D,
+                                       int64_t num_splits, int cus) {
+  if (B <= 0 || H <= 0 || H_kv <= 0 || H % H_kv != 0 || cus <= 0) return 0;
+  return B <= fa::kDecThreads && fa::decode_ordered(B, H, H_kv, D, num_splits, cus);
+}
+
 extern "C" int fa_decode_split_f16(const void* q, const void* k_pool, const void* v_pool,
                                    const int32_t* page_table, const int32_t* ctx_lens,
                                    int64_t B, int64_t H, int64_t D, int64_t page_size,
@@ -531,25 +531,6 @@ extern "C" int fa_lse_combine_f32(const float* part_o, const float* part_lse, in
 }
 
 namespace fa {
-// Splits that a decode of O and L uses, at most the caller's num_splits (whose
-// partials the workspace holds). max_pages bounds the contexts; the host does
-// not know them. A split costs a workgroup its start and merge (3-4 us) and
-// the partials' way through memory, so no more of them than
-//   * give every CU one workgroup of 8 waves (B32 over 8 KV heads, 2000
-//     tokens: 1 split 41 us, 16 splits 68; B8, 200-4000 tokens: 4 splits 20.7,
-//     16 splits 24.5), with two pages a wave (B1, 4000 tokens: 15 splits 10.9,
-//     7 splits 12.9); up to 32 pages stay in one (500 tokens: 7.2 us, split 10);
-//   * or, of long contexts (64 pages a split), give every CU two: ragged
-//     sequences then even out (B16 H32, 2000-8000 tokens, 4 waves: 1 split 214,
-//     2 splits 201), and two at least (B32 H32, 512-32768 tokens: 1432, 1404).
-static int64_t plan_splits(int64_t B, int64_t H, int64_t Hkv, int64_t max_pages, int64_t num_splits,
-                           int cus) {
-  const int64_t units = B * Hkv * ((H / Hkv + 15) / 16);
-  const int64_t fill = max_pages <= 32 ? 1 : std::min((cus + units - 1) / units, max_pages / 16);
-  const int64_t deep = std::min(max_pages / 64, std::max<int64_t>(2, 2 * cus / units));
-  return std::min(num_splits, std::max<int64_t>(1, std::max(fill, deep)));
-}
-
 template <bool BF16>
 static int decode_paged_gqa(const void* q, const void* k_pool, const void* v_pool,
                             const int32_t* page_table, const int32_t* ctx_lens, int64_t B,
@@ -562,8 +543,6 @@ static int decode_paged_gqa(const void* q, const void* k_pool, const void* v_poo
   if (H_kv <= 0 || H % H_kv != 0) return FA_ERR_KV_HEADS;
   if (!part_o || !part_lse || !o) return FA_ERR_NULL_POINTER;
   if (B * H > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
-  num_splits = plan_splits(B, H, H_kv, max_pages, num_splits,
-                           stream_topology(reinterpret_cast<hipStream_t>(stream)).cus);
   if (num_splits == 1)
     return decode_split<BF16>(q, k_pool, v_pool, page_table, ctx_lens, B, H, H_kv, D, max_pages,
                               num_pages, 1, part_o, part_lse, o, lse, stream);

@@ -278,10 +278,9 @@ int fa_lse_combine_f32(const float* part_o, const float* part_lse,
                        void* o, float* lse, void* stream);
 
 /*
- * O and L of the paged decode: split pass then combine pass, both on `stream`.
- * num_splits is the most splits used (fewer where that is faster, by the sizes
- * and the device; one split needs no combine pass), and part_o / part_lse are
- * workspace for that many. No reference counterpart.
+ * O and L of the paged decode: split pass then combine pass, both on `stream`
+ * (one split needs no combine pass). part_o / part_lse hold the num_splits
+ * partials of every row in between. No reference counterpart.
  */
 int fa_decode_paged_f16(const void* q, const void* k_pool, const void* v_pool,
                         const int32_t* page_table, const int32_t* ctx_lens,

@@ -12,14 +12,15 @@
  * fa_abi_version): 2 added the causal argument of fa_probe_fwd_variants;
  * 3 removed variant 418 and added fa_probe_choose_variant and
  * fa_probe_splitkv_plan_cus (the kernel and split choices for a given
- * compute-unit count, without a device); 4 added fa_probe_gather_bw.
+ * compute-unit count, without a device); 4 added fa_probe_gather_bw; 5 added
+ * fa_probe_unit_of and variant 432; 6 added fa_probe_decode_ordered.
  */
 #ifndef FA_PROBE_H
 #define FA_PROBE_H
 
 #include <stdint.h>
 
-#define FA_PROBE_VERSION 5
+#define FA_PROBE_VERSION 6
 
 #ifdef __cplusplus
 extern "C" {
@@ -85,6 +86,12 @@ int fa_probe_splitkv_plan_cus(int64_t B, int64_t H, int64_t N, int64_t D, int ca
  * needed. */
 int fa_probe_unit_of(int64_t heads, int64_t per_head, int nxcd, int cus, int uneven, int64_t g,
                      int* head, int* idx);
+
+/* 1 if a paged decode of these sizes takes the sequences longest first on a
+ * device of `cus` compute units (up to 256 of them; all workgroups resident at
+ * once run in index order), else 0. No device needed. */
+int fa_probe_decode_ordered(int64_t B, int64_t H, int64_t H_kv, int64_t D, int64_t num_splits,
+                            int cus);
 
 /* Writes up to max_out codes of the variants with tiles of 64 keys (all but
  * 432) that exist for head dimension D and the causal flag into out (may be NULL) and returns how many there are. */

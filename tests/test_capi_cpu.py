@@ -402,3 +402,13 @@ def test_unit_order(capi, heads, per_head, nxcd, cus, uneven):
     (1, 12, 1500, 256, 432), (1, 24, 1024, 256, 204), (0, 8, 2048, 32, 204), (1, 1, 4096, 32, 432)])
 def test_64_row_choice_at_d128(capi, causal, bh, N, cus, variant):
     assert capi.load().fa_probe_choose_variant(128, causal, bh, N, cus) == variant
+
+
+@pytest.mark.parametrize("B,H,Hkv,D,S,cus,ordered", [
+    (40, 4, 4, 64, 3, 256, 0), (40, 4, 4, 64, 7, 256, 1), (64, 4, 4, 64, 4, 256, 0),   # 480, 1120, 1024 workgroups
+    (64, 4, 4, 128, 2, 256, 0), (64, 4, 4, 128, 3, 256, 1),                             # 512, 768
+    (256, 32, 8, 128, 16, 256, 1), (257, 32, 8, 128, 16, 256, 0),                       # more sequences than are ranked
+    (4, 40, 2, 128, 8, 64, 0), (5, 40, 2, 128, 8, 64, 1),                               # groups of 20: two workgroups each
+    (1, 32, 8, 128, 16, 32, 1), (1, 3, 2, 64, 16, 256, 0)])
+def test_decode_order_choice(capi, B, H, Hkv, D, S, cus, ordered):
+    assert capi.load().fa_probe_decode_ordered(B, H, Hkv, D, S, cus) == ordered

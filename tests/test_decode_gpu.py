@@ -112,23 +112,41 @@ def test_gather_bit_exact_one_hot(fa, dev):
 
 
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("S", [1, 2, 7, 16])
+def test_decode_is_its_splits_combined(fa, dev, D, S):
+    """decode_paged runs the num_splits it is given, whatever the sizes: the
+    split pass and the combine pass called one after the other give its O and L
+    bit for bit, over short and long, equal and skewed contexts."""
+    for B, H, ctx in ((1, 2, [500]), (3, 2, [5000, 17, 130]), (2, 40, [33, 700]), (6, 3, [0, 1, 4000, 16, 16, 3])):
+        args = _dev(dev, *_small(70 + B + S, B, H, D, ctx))
+        O, L = fa.decode_paged(*args, num_splits=S)
+        Oc, Lc = fa.lse_combine(*fa.decode_partials(*args, num_splits=S))
+        assert torch.equal(O, Oc) and torch.equal(L, Lc), f"ctx {ctx}"
+
+
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("B,H,ctx,width", [
-    (1, 3, [512], 32),            # 32 pages: one split, no combine pass
-    (1, 3, [513], 33),            # 33: two splits of 8 waves
+    (1, 3, [512], 32),            # two pages a split
+    (1, 3, [513], 33),            # three, the last splits empty
     (1, 2, [1, ], 2048),          # a table far wider than the context: empty splits
     (3, 2, [5000, 17, 130], 320),  # ragged, more splits than the short ones have pages
-    (2, 300, [200, 65], 16),      # over two workgroups a CU: four waves each
-    (70, 8, [96 + b for b in range(70)], 12),   # 560 workgroups, ordered by length
+    (2, 300, [200, 65], 16),      # many heads
+    (70, 8, [96 + b for b in range(70)], 12),   # ordered by length
+    (70, 8, [(b % 5) * 21 for b in range(70)], 12),   # ordered, ties and empty sequences among them
 ])
-def test_decode_planned_splits(fa, dev, D, B, H, ctx, width):
-    """The split counts and workgroup widths that the decode picks by its sizes
-    (up to 16 splits allowed), at the edges of each."""
+def test_decode_split_sizes(fa, capi, dev, D, B, H, ctx, width):
+    """16 splits of short and long contexts, in narrow and wide tables."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    if B == 70:
+        assert capi.load().fa_probe_decode_ordered(B, H, H, D, 16, cus) == 1
     q, kp, vp, table, ctx = _small(40 + B + D, B, H, D, ctx)
     wide = np.zeros((B, width), np.int32)
     wide[:, :table.shape[1]] = table
     O, L = fa.decode_paged(*_dev(dev, q, kp, vp, wide, ctx), num_splits=16)
     Or, Lr = decode_attention(q, kp, vp, table, ctx)
-    _check(O, L, Or, Lr, tag=f"B{B} H{H} D{D} width {width}")
+    empty = ctx == 0
+    assert (O[torch.from_numpy(empty)] == 0).all() and torch.isneginf(L[torch.from_numpy(empty)]).all()
+    _check(O, L.masked_fill(torch.isneginf(L), 0), Or, np.where(np.isneginf(Lr), 0, Lr), tag=f"B{B} H{H} D{D} width {width}")
 
 
 def test_combine_element_aligned(fa, capi, dev):
