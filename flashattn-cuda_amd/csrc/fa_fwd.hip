@@ -1016,19 +1016,20 @@ static int splitkv_plan(int64_t B, int64_t H, int64_t N, int64_t D, int causal, 
   if (2 * units > cus) return 1;
   int64_t sp = cus / units;
   sp = sp < 8 ? sp : 8;
-  if (!causal) {
-    // At least 32 key tiles per split (B1 H1 N16384: 156.5 -> 137.8 us with
-    // 2 splits; B1 H8 N2048, 32 tiles: 27.3 vs 36.4 with 2).
-    sp = sp < tiles / 32 ? sp : tiles / 32;
-  } else {
-    // Causal row blocks differ in length, and the longest sets the time: a
-    // split evens them out down to 8 tiles per split (B1 H1 N8192 78.1 ->
-    // 43.4 us with 4 splits, B1 H1 N2048 25.2 -> 17.6 with 4, B1 H2 N8192
-    // 79.4 -> 68.0 with 2), but a 2-way split needs 64 tiles (B1 H4 N4096
-    // 43.6 -> 41.7; B1 H8 N2048, 32 tiles: 25.9 -> 34.5).
-    sp = sp < tiles / 8 ? sp : tiles / 8;
-    if (sp == 2 && tiles < 64) sp = 1;
-  }
+  // At least 32 key tiles per split; causal row blocks differ in length, and
+  // the longest sets the time, so there 8 tiles are enough (us, 64-row kernel
+  // unsplit -> split: B1 H1 N8192 53.1 -> 47.0 with 4 splits, causal 53.1 ->
+  // 40.6 with 4, causal B1 H1 N2048 17.9 -> 16.7 with 4).
+  const int64_t most = tiles / (causal ? 8 : 32);
+  sp = sp < most ? sp : most;
+  // Two splits of 128-row blocks do the work of the 64-row kernel's twice as
+  // many blocks, and pay for the combine: only over the longest non-causal
+  // rows is that less (us, unsplit -> 2 splits: B1 H1 N12000 90.8 -> 87.4,
+  // N14000 114.7 -> 108.4, N16384 145.1 -> 135.2; not B1 H1 N6000 42.1 vs 43.7,
+  // B1 H2 N8192 74.5 vs 76.5, B1 H4 N4096 40.3 vs 48.1, nor causal B1 H1
+  // N16384 108.1 vs 123.5, B1 H2 N6000 46.0 vs 47.4, B1 H4 N4096 32.5 vs 39.0;
+  // causal B1 H1 N12000 82.6 vs 80.9).
+  if (sp == 2 && (causal || tiles < 160)) sp = 1;
   return sp < 2 ? 1 : (int)sp;
 }
 }  // namespace fa

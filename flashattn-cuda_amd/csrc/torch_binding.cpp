@@ -119,17 +119,8 @@ std::pair<torch::Tensor, torch::Tensor> forward_impl(torch::Tensor Q, torch::Ten
     L_ptr = L.data_ptr<float>();
   }
   TORCH_CHECK(variant == 0 || Hkv == H, "explicit kernel variants take H_kv == H");
-  int64_t nsplit = 1;
-  if (splits > 0) {
-    nsplit = splits;
-  } else if (variant == 0) {
-    nsplit = fa_fwd_splitkv_plan(B, H, N, D, causal ? 1 : 0);
-    // Two splits of 128-row blocks lose to the 64-row kernel that the unsplit
-    // forward then runs (us, two splits -> 64 rows: B1 H4 N4096 47.3 -> 40.0,
-    // causal 38.0 -> 32.8, B1 H2 N6000 50.0 -> 48.6, B1 H2 N8192 74.2 -> 73.7)
-    // but for the longest non-causal rows (B1 H1 N16384 135 vs 143).
-    if (nsplit == 2 && (causal || N < 16384)) nsplit = 1;
-  }
+  const int64_t nsplit =
+      variant != 0 ? 1 : (splits > 0 ? splits : fa_fwd_splitkv_plan(B, H, N, D, causal ? 1 : 0));
   int st;
   if (nsplit > 1) {
     auto ws = torch::empty({fa_fwd_splitkv_workspace_floats(B, H, N, D, nsplit)},

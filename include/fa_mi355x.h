@@ -223,11 +223,9 @@ int fa_validate_bwd_varlen(const void* q, const void* k, const void* v, const vo
  * different lengths). O within the
  * forward's tolerance of the unsplit kernel; lse nullable (O only). The
  * workspace (fa_fwd_splitkv_workspace_floats floats, 16-byte aligned) holds
- * the fp32 partials. fa_fwd_splitkv_plan returns a split count for a
- * shape on the current device (1: no split; it depends on the device's
- * compute-unit count) that beats the unsplit 128-row kernel; the torch binding
- * uses it from three splits on, and two only for non-causal N >= 16384, as
- * fa_fwd_gqa_f16's 64-row kernel is faster elsewhere.
+ * the fp32 partials. fa_fwd_splitkv_plan returns the split count the torch
+ * binding uses (1: no split) for a shape on the current device (it depends on
+ * the device's compute-unit count).
  */
 int fa_fwd_splitkv_plan(int64_t B, int64_t H, int64_t N, int64_t D, int causal);
 int64_t fa_fwd_splitkv_workspace_floats(int64_t B, int64_t H, int64_t N, int64_t D,

@@ -354,17 +354,24 @@ def test_kernel_and_split_choice_follow_the_cu_count(capi):
     # split-KV plan: D = 128 long sequences over few heads split to fill the CUs
     assert plan(1, 1, 16384, 128, 0, 256) == 2     # 128 blocks, 256 tiles / 32 = 8 -> ceil(256/128)
     assert plan(1, 1, 16384, 128, 0, 32) == 1      # 128 blocks >= 32 CUs
-    assert plan(1, 1, 4096, 128, 0, 256) == 2      # 32 blocks: 8 by CUs, 64 tiles / 32 = 2
-    assert plan(1, 1, 4096, 128, 0, 64) == 2
+    assert plan(1, 1, 12000, 128, 0, 256) == 2     # 94 blocks, 188 tiles
+    assert plan(1, 1, 10000, 128, 0, 256) == 3     # 79 blocks, 157 tiles
+    assert plan(1, 1, 8192, 128, 0, 256) == 4 and plan(1, 1, 8192, 128, 0, 192) == 3
+    assert plan(1, 1, 8192, 128, 0, 128) == 1      # two splits of 128 tiles: 64-row blocks instead
+    assert plan(1, 1, 4096, 128, 0, 256) == 1      # 32 blocks: 8 by CUs, 64 tiles / 32 = 2
+    assert plan(1, 2, 8192, 128, 0, 256) == 1
     assert plan(1, 1, 2048, 128, 0, 256) == 1      # 32 tiles: too few per split
     assert plan(1, 8, 4096, 128, 0, 256) == 1      # 256 blocks fill 256 CUs
-    assert plan(1, 8, 4096, 128, 0, 512) == 2      # but not a 512-CU device
+    assert plan(1, 4, 16384, 128, 0, 512) == 1     # 512 blocks
+    assert plan(1, 2, 16384, 128, 0, 512) == 2     # 256 blocks on a 512-CU device
     assert plan(1, 1, 16384, 64, 0, 256) == 1      # D = 64 never splits
     assert plan(1, 3, 8192, 128, 0, 256) == 1      # 192 blocks: two splits would not fit one wave
     # causal D = 128: the longest row block sets the time; splits down to 8 tiles
     assert plan(1, 1, 8192, 128, 1, 256) == 4      # 64 blocks, 128 tiles
     assert plan(1, 1, 2048, 128, 1, 256) == 4      # 16 blocks, 32 tiles: 8 per split
-    assert plan(1, 4, 4096, 128, 1, 256) == 2      # 128 blocks, 64 tiles
+    assert plan(1, 4, 4096, 128, 1, 256) == 1      # 128 blocks, 64 tiles: 2 splits lose
+    assert plan(1, 1, 16384, 128, 1, 256) == 1     # 128 blocks, 256 tiles: 2 splits lose
+    assert plan(1, 2, 5000, 128, 1, 256) == 3      # 80 blocks, 79 tiles
     assert plan(1, 8, 2048, 128, 1, 256) == 1      # 128 blocks, 32 tiles: 2 splits lose
     assert plan(1, 3, 8192, 128, 1, 256) == 1      # 192 blocks
     assert plan(1, 1, 16384, 64, 1, 256) == 1      # D = 64 never splits

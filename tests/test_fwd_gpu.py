@@ -456,6 +456,24 @@ def test_splitkv_plan_and_default_path(fa, dev):
     _check(O, L, Or, Lr, 1.0, tag="default path, causal split 4 B1 H1 N2048 D128")
 
 
+@pytest.mark.parametrize("H,N,causal", [(1, 12000, False), (2, 8192, False), (1, 16384, True), (2, 5000, True),
+                                        (4, 4096, True), (1, 4096, False)])
+def test_forward_runs_the_plan(fa, capi, dev, H, N, causal):
+    """The forward splits the keys exactly as fa_fwd_splitkv_plan says, bit for
+    bit: the planned split count, or the kernel that the shape chooses unsplit."""
+    D = 128
+    tq, tk, tv = _to_dev(dev, *make_fwd_inputs(1, H, N, D, seed=N + H, amp=1.0))
+    O, L = fa.forward(tq, tk, tv, causal=causal)
+    n = fa.probe.probe_fwd_splitkv_plan(1, H, N, D, causal)
+    if n > 1:
+        Or, Lr = fa.probe.probe_fwd_splitkv(tq, tk, tv, causal, n, True)
+    else:
+        cus = torch.cuda.get_device_properties(dev).multi_processor_count
+        v = capi.load().fa_probe_choose_variant(D, int(causal), H, N, cus)
+        Or, Lr = fa.probe.probe_fwd_variant(tq, tk, tv, causal, v, True)
+    assert torch.equal(O, Or) and torch.equal(L, Lr)
+
+
 def test_splitkv_gqa(fa, dev):
     B, H, Hkv, N, D = 2, 8, 2, 700, 64
     rng = np.random.default_rng(5)
