@@ -576,7 +576,7 @@ constexpr int kCountedSeqs = 512;
 
 // Blocks of `rows` rows per head in a varlen grid: sequence b has
 // ceil(n_b / rows) of them, and the host knows only that the n_b are at most
-// max_seqlen and sum to at most `total`.
+// max_seqlen and sum to at most `total`. B of them where max_seqlen <= rows.
 inline int64_t varlen_units(int64_t B, int64_t total, int64_t max_seqlen, int rows) {
   const int64_t by_max = B * ((max_seqlen + rows - 1) / rows);
   const int64_t by_total = total / rows + B;
@@ -650,10 +650,33 @@ __device__ __forceinline__ SeqBlock counted_block(const Geom& g, int u, int rows
   return out;
 }
 
+// The same where no sequence is longer than a block: unit u is sequence u's,
+// which starts at the largest of the bounds up to it. One scan: the two scans
+// and the search of counted_block made forwards of 256 sequences of 64 rows,
+// H32 over 8 D64, 10 % slower (us: in sequence order, without a look at the
+// other bounds, 173; counted 191; so 170; of 500 sequences 338, 363, 354).
+template <int J>
+__device__ __forceinline__ SeqBlock single_block(const Geom& g, int u, int lane) {
+  const int next = g.cu[u + 1];
+  int c = 0;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const int b = 64 * j + lane;
+    if (b <= u) c = max(c, clamp_row(g.cu[b], g.total));
+  }
+  const int start = __builtin_amdgcn_readlane(scan_max(c), 63);
+  return SeqBlock{start, min(max(start, clamp_row(next, g.total)) - start, g.N), 0};
+}
+
+template <int J>
+__device__ __forceinline__ SeqBlock scanned_block(const Geom& g, int u, int rows, int lane) {
+  return g.N <= rows ? single_block<J>(g, u, lane) : counted_block<J>(g, u, rows, lane);
+}
+
 __device__ __forceinline__ SeqBlock varlen_block(const Geom& g, int u, int rows, int lane) {
-  if (g.B <= 64) return counted_block<1>(g, u, rows, lane);
-  if (g.B <= 256) return counted_block<4>(g, u, rows, lane);
-  if (g.B <= kCountedSeqs) return counted_block<kCountedSeqs / 64>(g, u, rows, lane);
+  if (g.B <= 64) return scanned_block<1>(g, u, rows, lane);
+  if (g.B <= 256) return scanned_block<4>(g, u, rows, lane);
+  if (g.B <= kCountedSeqs) return scanned_block<kCountedSeqs / 64>(g, u, rows, lane);
   const int nbmax = (g.N + rows - 1) / rows;   // more: sequence by sequence
   const int b = u / nbmax, i = u - b * nbmax;
   const int s0 = clamp_row(g.cu[b], g.total);

@@ -104,11 +104,13 @@ def test_varlen_forward(fa, dev, D, causal, Hkv):
 
 
 @pytest.mark.parametrize("B", [64, 65, 257, 520])
+@pytest.mark.parametrize("last", [300, 64])
 @pytest.mark.parametrize("causal", [False, True])
-def test_varlen_many_sequences(fa, dev, B, causal):
+def test_varlen_many_sequences(fa, dev, B, last, causal):
     """Every unit of batches around the widths of the per-wave count of blocks
     (64 and 256 sequences a pass, at most 512 counted), with empty sequences,
-    one long one last, and a head count that no XCD count divides; forward
+    one long one last or no sequence over one block (those are not counted),
+    and a head count that no XCD count divides; forward
     against the oracle, gradients against the dense backward of the sequence
     (the same products; fp32 sums of up to 300 terms perhaps in another order:
     300 x 2^-24 of the largest gradient)."""
@@ -116,12 +118,12 @@ def test_varlen_many_sequences(fa, dev, B, causal):
     rng = np.random.default_rng(B)
     lengths = [int(x) for x in rng.integers(0, 40, B)]
     lengths[B // 2] = 0
-    lengths[-1] = 300
+    lengths[-1] = last
     cu = _cu(lengths)
     q, k, v, g = (torch.from_numpy(_randn((H, int(cu[-1]), D), s)).to(dev).half() for s in (40, 41, 42, 43))
     tcu = torch.from_numpy(cu).to(dev)
-    O, L = fa.forward_varlen(q, k, v, tcu, 300, causal=causal)
-    grads = fa.backward_varlen(q, k, v, O, g, L, tcu, 300, causal=causal)
+    O, L = fa.forward_varlen(q, k, v, tcu, last, causal=causal)
+    grads = fa.backward_varlen(q, k, v, O, g, L, tcu, last, causal=causal)
     torch.cuda.synchronize()
     qn, kn, vn = (x.float().cpu().numpy() for x in (q, k, v))
     for b, n in enumerate(lengths):
@@ -143,6 +145,7 @@ def test_varlen_many_sequences(fa, dev, B, causal):
     ([70, 70, 133], 64, [(70, 133)]),                    # a head and a tail, no chunk whole
     ([0, 40, 300], 100, [(0, 140)]),                     # rows past max_seqlen
     ([0, 250, 100, 10_000], 256, [(0, 300)]),            # falling
+    ([0, 50, 20, 10_000], 64, [(0, 114)]),               # falling, no sequence over one block
     ([-5, 10, 20], 64, [(0, 20)]),                       # out of range
     ([5] * 600 + [60], 64, [(5, 60)]),                   # more sequences than are counted
 ])
@@ -168,14 +171,15 @@ def test_varlen_rows_outside(fa, dev, cu, most, inside, Hkv):
         assert torch.isfinite(x.float()).all() and not x[:, ~rows].any()
 
 
-def test_varlen_decreasing_bounds(fa, dev):
+@pytest.mark.parametrize("bad,good,most", [([0, 250, 100, 10_000], [0, 250, 250, 300], 256),
+                                           ([0, 50, 20, 10_000], [0, 50, 50, 300], 64)])
+def test_varlen_decreasing_bounds(fa, dev, bad, good, most):
     """A table that falls counts as its running maximum: what it did compute
     stays computed, and no row is computed twice."""
     H, D, total = 2, 64, 300
     q, k, v = (torch.from_numpy(_randn((H, total, D), s)).to(dev).half() for s in (44, 45, 46))
-    bad = torch.tensor([0, 250, 100, 10_000], dtype=torch.int32, device=dev)
-    good = torch.tensor([0, 250, 250, 300], dtype=torch.int32, device=dev)
-    for x, r in zip(fa.forward_varlen(q, k, v, bad, 256), fa.forward_varlen(q, k, v, good, 256)):
+    bad, good = (torch.tensor(x, dtype=torch.int32, device=dev) for x in (bad, good))
+    for x, r in zip(fa.forward_varlen(q, k, v, bad, most), fa.forward_varlen(q, k, v, good, most)):
         assert torch.equal(x, r)
 
 
