@@ -30,50 +30,58 @@ struct FillBuf {
 // every buffer. A well-formed cu covers one run of rows, so a workgroup inside
 // it leaves after one look at the table (about 3 us for a whole batch; filling
 // the outputs whole before the kernels took 45 us of a 686 us training pass
-// of 12 sequences, H8 D64). Only where a sequence is longer than max_seqlen or
-// the table falls does each row look for its sequence.
+// of 12 sequences, H8 D64). Every workgroup reads the whole table, so of more
+// than kCountedSeqs sequences kFillGroups workgroups take several chunks each
+// (60000 sequences of 4-12 rows, H2 D64, forward: 2480 us with a workgroup per
+// chunk, 2270-2310 so). Only where a sequence is longer than max_seqlen or the table
+// falls does each row look for its sequence.
 constexpr int kFillRows = 64;
+constexpr int kFillGroups = 512;
 __global__ void __launch_bounds__(256)
 fa_fill_outside_kernel(Geom g, FillBuf b0, FillBuf b1, FillBuf b2) {
   __shared__ uint8_t inside[kFillRows];
   const int tid = threadIdx.x;
-  const int r0 = blockIdx.x * kFillRows;
   int odd = 0;
+#pragma unroll 4
   for (int b = tid; b < g.B; b += 256) {
     const int c0 = clamp_row(g.cu[b], g.total), c1 = clamp_row(g.cu[b + 1], g.total);
     odd |= c1 < c0 || c1 - c0 > g.N;
   }
   odd = __syncthreads_or(odd);
   const int first = clamp_row(g.cu[0], g.total), last = clamp_row(g.cu[g.B], g.total);
-  if (!odd && r0 >= first && min(r0 + kFillRows, g.total) <= last) return;
-  if (tid < kFillRows) {
-    const int r = r0 + tid;
-    bool in = !odd && r >= first && r < last;
-    if (odd) {
-      // Sequences as the attention kernels take them: up to kCountedSeqs from
-      // the running maximum of the bounds on, more of them as they stand.
-      int end = 0;
-      for (int b = 0; b < g.B; ++b) {
-        const int c0 = clamp_row(g.cu[b], g.total), c1 = clamp_row(g.cu[b + 1], g.total);
-        const int s0 = g.B <= kCountedSeqs ? max(c0, end) : c0;
-        const int s1 = max(s0, c1);
-        in |= r >= s0 && r < s0 + min(s1 - s0, g.N);
-        end = max(end, s1);
+  for (int64_t at = (int64_t)blockIdx.x * kFillRows; at < g.total; at += (int64_t)gridDim.x * kFillRows) {
+    const int r0 = (int)at;
+    if (!odd && r0 >= first && min(r0 + kFillRows, g.total) <= last) continue;
+    __syncthreads();   // the rows of the chunk before are written
+    if (tid < kFillRows) {
+      const int r = r0 + tid;
+      bool in = !odd && r >= first && r < last;
+      if (odd) {
+        // Sequences as the attention kernels take them: up to kCountedSeqs from
+        // the running maximum of the bounds on, more of them as they stand.
+        int end = 0;
+        for (int b = 0; b < g.B; ++b) {
+          const int c0 = clamp_row(g.cu[b], g.total), c1 = clamp_row(g.cu[b + 1], g.total);
+          const int s0 = g.B <= kCountedSeqs ? max(c0, end) : c0;
+          const int s1 = max(s0, c1);
+          in |= r >= s0 && r < s0 + min(s1 - s0, g.N);
+          end = max(end, s1);
+        }
       }
+      inside[tid] = in;
     }
-    inside[tid] = in;
-  }
-  __syncthreads();
-  const FillBuf bufs[3] = {b0, b1, b2};
+    __syncthreads();
+    const FillBuf bufs[3] = {b0, b1, b2};
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    const FillBuf b = bufs[i];
-    if (b.p == nullptr) continue;
-    for (int64_t h = 0; h < b.heads; ++h) {
-      uint32_t* row0 = b.p + (h * g.total + r0) * b.words;
-      for (int w = tid; w < kFillRows * b.words; w += 256) {
-        const int r = w / b.words;
-        if (r0 + r < g.total && !inside[r]) row0[w] = b.value;
+    for (int i = 0; i < 3; ++i) {
+      const FillBuf b = bufs[i];
+      if (b.p == nullptr) continue;
+      for (int64_t h = 0; h < b.heads; ++h) {
+        uint32_t* row0 = b.p + (h * g.total + r0) * b.words;
+        for (int w = tid; w < kFillRows * b.words; w += 256) {
+          const int r = w / b.words;
+          if (r0 + r < g.total && !inside[r]) row0[w] = b.value;
+        }
       }
     }
   }
@@ -123,8 +131,9 @@ extern "C" int fa_varlen_fill_outside(const int32_t* cu_seqlens, int64_t B, int6
   if (total == 0) return FA_OK;
   const Geom g{cu_seqlens, (int)max_seqlen, 1, FastDiv(1), (int)total, (int)B};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(fa_fill_outside_kernel, dim3((unsigned)((total + kFillRows - 1) / kFillRows)),
-                     dim3(256), 0, s, g, b[0], b[1], b[2]);
+  int64_t groups = (total + kFillRows - 1) / kFillRows;
+  if (B > kCountedSeqs && groups > kFillGroups) groups = kFillGroups;
+  hipLaunchKernelGGL(fa_fill_outside_kernel, dim3((unsigned)groups), dim3(256), 0, s, g, b[0], b[1], b[2]);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? FA_OK : -(int)e;
 }

@@ -171,6 +171,24 @@ def test_varlen_rows_outside(fa, dev, cu, most, inside, Hkv):
         assert torch.isfinite(x.float()).all() and not x[:, ~rows].any()
 
 
+@pytest.mark.parametrize("odd", [0, 7])
+def test_varlen_rows_outside_many(fa, dev, odd):
+    """The same over more sequences than are counted and more chunks of rows
+    than workgroups; with odd, every sequence is that much longer than
+    max_seqlen and its last rows are outside."""
+    H, D, B, n, first = 1, 64, 700, 57, 11
+    total = first + B * n + 30
+    q, k, v = (torch.from_numpy(_randn((H, total, D), s)).to(dev).half() for s in (51, 52, 53))
+    cu = torch.arange(first, first + B * n + 1, n, dtype=torch.int32, device=dev)
+    stale = [torch.full((H, total, D), 7.0, device=dev).half(), torch.full((H, total), 7.0, device=dev)]
+    del stale
+    O, L = fa.forward_varlen(q, k, v, cu, n - odd)
+    r = torch.arange(total, device=dev)
+    rows = (r >= first) & (r < first + B * n) & ((r - first) % n < n - odd)
+    assert torch.isfinite(L[:, rows]).all() and torch.isneginf(L[:, ~rows]).all()
+    assert (O[:, rows] != 0).any(-1).all() and not O[:, ~rows].any()
+
+
 @pytest.mark.parametrize("bad,good,most", [([0, 250, 100, 10_000], [0, 250, 250, 300], 256),
                                            ([0, 50, 20, 10_000], [0, 50, 50, 300], 64)])
 def test_varlen_decreasing_bounds(fa, dev, bad, good, most):
