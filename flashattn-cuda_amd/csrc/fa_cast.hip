@@ -99,7 +99,7 @@ extern "C" int fa_cast_f32(const float* const src[3], void* const dst[3], const 
     if (dst[i] == nullptr) return FA_ERR_NULL_POINTER;
     if ((reinterpret_cast<uintptr_t>(src[i]) & 15u) || (reinterpret_cast<uintptr_t>(dst[i]) & 15u))
       return FA_ERR_ALIGNMENT;
-    if (n[i] < 0 || n[i] % 8 != 0) return FA_ERR_TOO_LARGE;
+    if (n[i] < 0) return FA_ERR_SEQ_LEN;
     blocks += n[i] / 8 / kCastVecs + 1;
     if (blocks > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
   }

@@ -356,13 +356,15 @@ __device__ __forceinline__ f16x8 cvt8x(const float* __restrict__ src) {
 }
 
 // Up to three fp32 tensors to convert in one launch, `vecs` groups of eight
-// values each (16-byte aligned on both sides). Workgroups of 256 threads take
-// kCastVecs groups: first src[0]'s, then src[1]'s, then src[2]'s.
+// values each (16-byte aligned on both sides) and `tail` values more. Workgroups
+// of 256 threads take kCastVecs groups: first src[0]'s, then src[1]'s, then
+// src[2]'s.
 constexpr int kCastVecs = 512;
 struct CastJobs {
   const float* src[3];
   f16* dst[3];
   int64_t vecs[3];
+  int tail[3];
   int blocks[3];   // of each
 };
 
@@ -372,7 +374,8 @@ inline CastJobs cast_jobs(const float* const src[3], void* const dst[3], const i
     j.src[i] = src[i];
     j.dst[i] = (f16*)dst[i];
     j.vecs[i] = src[i] != nullptr ? n[i] / 8 : 0;
-    j.blocks[i] = (int)((j.vecs[i] + kCastVecs - 1) / kCastVecs);
+    j.tail[i] = src[i] != nullptr ? (int)(n[i] % 8) : 0;
+    j.blocks[i] = (int)((j.vecs[i] + (j.tail[i] > 0) + kCastVecs - 1) / kCastVecs);
   }
   return j;
 }
@@ -386,6 +389,9 @@ __device__ __forceinline__ void cast_block(const CastJobs& j, int block) {
       for (int i = 0; i < kCastVecs / 256; ++i) {
         const int64_t v = (int64_t)block * kCastVecs + 256 * i + threadIdx.x;
         if (v < j.vecs[t]) reinterpret_cast<f16x8*>(j.dst[t])[v] = cvt8x<BF16>(j.src[t] + 8 * v);
+        if (v == j.vecs[t])
+          for (int e = 0; e < j.tail[t]; ++e)
+            j.dst[t][8 * v + e] = cvt2x<BF16>(j.src[t][8 * v + e], 0.f)[0];
       }
     }
     block -= j.blocks[t];

@@ -192,6 +192,7 @@ std::vector<torch::Tensor> forward_varlen(torch::Tensor q, torch::Tensor k, torc
               "q/k/v/cu_seqlens must be CUDA tensors");
   TORCH_CHECK(q.dim() == 3, "q must be 3D [H, total, D]");
   const int64_t H = q.size(0), total = q.size(1), D = q.size(2);
+  TORCH_CHECK(D == 64 || D == 128, "Head dimension must be 64 or 128");
   TORCH_CHECK(k.dim() == 3 && v.sizes() == k.sizes() && k.size(1) == total && k.size(2) == D,
               "k and v must be [H_kv, total, D] matching q");
   TORCH_CHECK(cu_seqlens.dim() == 1 && cu_seqlens.scalar_type() == torch::kInt &&

@@ -388,8 +388,8 @@ int fa_kv_append_set_bad(const void* k_new, const void* v_new, const int32_t* pa
 
 /*
  * Rounds up to three fp32 tensors to fp16 (bf16 != 0: bfloat16) in one launch,
- * to nearest even: dst[i] from src[i], n[i] values (a multiple of 8), both
- * 16-byte aligned; src[i] NULL skips i. The reference casts each input with a
+ * to nearest even: dst[i] from src[i], n[i] values (FA_ERR_SEQ_LEN below 0),
+ * both 16-byte aligned; src[i] NULL skips i. The reference casts each input with a
  * tensor operation of its own (cuda/flash_attn_fa3_db_full.cu:366-368).
  */
 int fa_cast_f32(const float* const src[3], void* const dst[3], const int64_t n[3], int bf16,

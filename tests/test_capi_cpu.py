@@ -419,3 +419,16 @@ def test_64_row_choice_at_d128(capi, causal, bh, N, cus, variant):
     (1, 32, 8, 128, 16, 32, 1), (1, 3, 2, 64, 16, 256, 0)])
 def test_decode_order_choice(capi, B, H, Hkv, D, S, cus, ordered):
     assert capi.load().fa_probe_decode_ordered(B, H, Hkv, D, S, cus) == ordered
+
+
+def test_cast_rejects_before_touching_the_device(capi):
+    import ctypes as C
+    lib = capi.load()
+    p = lambda *x: (C.c_void_p * 3)(*x)
+    n = lambda *x: (C.c_int64 * 3)(*x)
+    assert lib.fa_cast_f32(None, p(A, A, A), n(8, 8, 8), 0, None) == capi.STATUS["FA_ERR_NULL_POINTER"]
+    assert lib.fa_cast_f32(p(A, 0, 0), p(0, 0, 0), n(8, 8, 8), 0, None) == capi.STATUS["FA_ERR_NULL_POINTER"]
+    assert lib.fa_cast_f32(p(A + 4, 0, 0), p(A, 0, 0), n(8, 8, 8), 0, None) == capi.STATUS["FA_ERR_ALIGNMENT"]
+    assert lib.fa_cast_f32(p(A, 0, 0), p(A, 0, 0), n(-1, 0, 0), 0, None) == capi.STATUS["FA_ERR_SEQ_LEN"]
+    assert lib.fa_cast_f32(p(A, 0, 0), p(A, 0, 0), n(1 << 50, 0, 0), 0, None) == capi.STATUS["FA_ERR_TOO_LARGE"]
+    assert lib.fa_cast_f32(p(0, 0, 0), p(0, 0, 0), n(5, 5, 5), 0, None) == capi.STATUS["FA_OK"]   # nothing to do

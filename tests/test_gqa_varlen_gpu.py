@@ -230,6 +230,31 @@ def test_varlen_rows_outside_sequences_and_malformed_bounds(fa, dev):
     assert torch.isfinite(O2.float()).all()
 
 
+@pytest.mark.parametrize("D", [5, 32, 96])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_varlen_names_the_head_dimension(fa, dev, D, dtype):
+    """A head dimension that is not 64 or 128 is refused as such, in fp32 and 16 bits."""
+    q = torch.zeros(1, 3, D, device=dev, dtype=dtype)
+    cu = torch.tensor([0, 3], dtype=torch.int32, device=dev)
+    with pytest.raises(RuntimeError, match="Head dimension must be 64 or 128"):
+        fa.forward_varlen(q, q, q, cu, 3)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("ns", [(0, 1, 7), (8, 9, 15), (4095, 4096, 4097), (100_003, 5, 8191)])
+def test_cast_any_length(capi, dev, bf16, ns):
+    """fa_cast_f32 rounds as torch does at every length, and writes nothing past it."""
+    import ctypes as C
+    lib, dt = capi.load(), torch.bfloat16 if bf16 else torch.float16
+    src = [torch.randn(max(n, 1), generator=torch.Generator(device=dev).manual_seed(n), device=dev) * 3 for n in ns]
+    dst = [torch.full((n + 8,), 7.0, device=dev, dtype=dt) for n in ns]
+    ptr = lambda x: (C.c_void_p * 3)(*(t.data_ptr() for t in x))
+    st = lib.fa_cast_f32(ptr(src), ptr(dst), (C.c_int64 * 3)(*ns), int(bf16), torch.cuda.current_stream().cuda_stream)
+    assert st == 0
+    for s, d, n in zip(src, dst, ns):
+        assert torch.equal(d[:n], s[:n].to(dt)) and (d[n:] == 7).all()
+
+
 def test_gqa_decode(fa, dev):
     B, H, Hkv, D = 4, 8, 2, 128
     rng = np.random.default_rng(16)
