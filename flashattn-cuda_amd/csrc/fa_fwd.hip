@@ -1159,7 +1159,7 @@ extern "C" int fa_probe_default_variant(int64_t D) {
 }
 
 extern "C" int fa_probe_fwd_variants(int* out, int max_out, int64_t D, int causal) {
-  static const int all[] = {204, 408};
+  static const int all[] = {fa::kPingPong, fa::kPingPong4, fa::kPingPong4K32};
   int n = 0;
   for (int v : all) {
     if (fa::variant_fits((int)D, v, causal)) {

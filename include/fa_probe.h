@@ -13,7 +13,8 @@
  * 3 removed variant 418 and added fa_probe_choose_variant and
  * fa_probe_splitkv_plan_cus (the kernel and split choices for a given
  * compute-unit count, without a device); 4 added fa_probe_gather_bw; 5 added
- * fa_probe_unit_of and variant 432; 6 added fa_probe_decode_ordered.
+ * fa_probe_unit_of and variant 432; 6 added fa_probe_decode_ordered and
+ * lists variant 432.
  */
 #ifndef FA_PROBE_H
 #define FA_PROBE_H
@@ -93,8 +94,8 @@ int fa_probe_unit_of(int64_t heads, int64_t per_head, int nxcd, int cus, int une
 int fa_probe_decode_ordered(int64_t B, int64_t H, int64_t H_kv, int64_t D, int64_t num_splits,
                             int cus);
 
-/* Writes up to max_out codes of the variants with tiles of 64 keys (all but
- * 432) that exist for head dimension D and the causal flag into out (may be NULL) and returns how many there are. */
+/* Writes up to max_out codes of the variants that exist for head dimension D
+ * and the causal flag into out (may be NULL) and returns how many there are. */
 int fa_probe_fwd_variants(int* out, int max_out, int64_t D, int causal);
 
 /* Streams `bytes` (a multiple of 16, 16-byte aligned) from device memory at p

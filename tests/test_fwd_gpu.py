@@ -26,7 +26,7 @@ import pytest
 import torch
 
 from errlog import record
-from oracle import fp16_p_forward, half_cast, make_fwd_inputs, make_ragged_inputs, naive_attention
+from oracle import bf16_cast, fp16_p_forward, half_cast, make_fwd_inputs, make_ragged_inputs, naive_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -333,8 +333,8 @@ VARIANT_CASES = [(1, 1, 64, False), (1, 2, 130, False), (1, 2, 200, False), (1, 
 @pytest.mark.parametrize("D", [64, 128])
 def test_every_kernel_variant(fa, dev, D):
     variants = list(fa.probe.probe_fwd_variants(D, False))
-    assert set(variants) == ({204, 408} if D == 64 else {204}), variants
-    assert set(fa.probe.probe_fwd_variants(D, True)) == ({204, 408} if D == 64 else {204})
+    assert set(variants) == ({204, 408} if D == 64 else {204, 432}), variants
+    assert set(fa.probe.probe_fwd_variants(D, True)) == set(variants)
     assert fa.probe.probe_default_variant(D) in variants
     for B, H, N, causal in VARIANT_CASES:
         Q, K, V = make_fwd_inputs(B, H, N, D, seed=N + D, amp=1.0)
@@ -348,11 +348,9 @@ def test_every_kernel_variant(fa, dev, D):
             _check(O, L, Or, Lr, 1.0, tag=f"variant {v} B{B} H{H} N{N} D{D} causal={causal}")
 
 
-# The 64-row kernel (408) on ragged and small causal shapes: odd block
-# counts, diagonal tiles, rows with fewer keys than one tile.
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("N", [1, 31, 33, 64, 65, 127, 128, 129, 200, 256, 385, 1024, 1100])
-def test_64_row_d128_variant(fa, dev, causal, N):
+def test_64_row_d128_variant(fa, capi, dev, causal, N):
     """Variant 432 (D = 128, 64 rows, four tile groups of 32-key tiles) at the
     edges of its row blocks, tiles and groups: against the oracle, O-only and
     the guarded instance bitwise, and bf16 through the default path."""
@@ -367,10 +365,18 @@ def test_64_row_d128_variant(fa, dev, causal, N):
     Or, Lr = naive_attention(half_cast(Q), half_cast(K), half_cast(V), causal=causal)
     _check(O, L, Or, Lr, 1.0, tag=f"variant 432 N{N} causal={causal}")
     if N > 64:
-        Od, Ld = fa.forward_bf16(tq.bfloat16(), tk.bfloat16(), tv.bfloat16(), causal=causal)
-        # P and O rounded to bf16: 1e-2 plus half a bf16 ulp below |O| = 4; and the inputs, 3 bits shorter
-        assert (Od.float() - O.float()).abs().max().item() <= 6e-2
+        cus = torch.cuda.get_device_properties(dev).multi_processor_count
+        assert capi.load().fa_probe_choose_variant(D, int(causal), B * H, N, cus) == 432
+        Ob, Lb = fa.forward_bf16(tq, tk, tv, causal=causal)
+        Or, Lr = naive_attention(*(bf16_cast(x.astype(np.float32)) for x in (Q, K, V)), causal=causal)
+        # P rounded to bf16, and half a bf16 ulp of O (tests/test_bf16_gpu.py)
+        ulp = 2.0 ** (np.floor(np.log2(np.maximum(np.abs(Or), 2.0 ** -126))) - 8)
+        assert (np.abs(Ob.float().cpu().numpy() - Or) <= 1e-2 + ulp).all()
+        assert (np.abs(Lb.cpu().numpy() - Lr) / np.maximum(np.abs(Lr), 1)).max() <= 1e-4
 
+
+# The 64-row kernel (408) on ragged and small causal shapes: odd block
+# counts, diagonal tiles, rows with fewer keys than one tile.
 
 @pytest.mark.parametrize("N", [1, 63, 65, 127, 129, 191, 257, 383, 449, 577, 1023, 1089])
 def test_64_row_kernel_ragged_causal(fa, dev, N):
