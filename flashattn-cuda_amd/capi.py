@@ -68,6 +68,7 @@ SIGNATURES = {
     "fa_probe_splitkv_plan_cus": (C.c_int, [_i64] * 4 + [C.c_int, C.c_int]),
     "fa_probe_unit_of": (C.c_int, [_i64, _i64, C.c_int, C.c_int, C.c_int, _i64, _vp, _vp]),
     "fa_probe_decode_ordered": (C.c_int, [_i64] * 5 + [C.c_int]),
+    "fa_probe_bwd_block_rows": (C.c_int, [C.c_int, _i64, _i64, C.c_int]),
     "fa_probe_read_bw": (C.c_int, [_vp, _i64, C.c_int, _vp, _vp]),
     "fa_probe_gather_bw": (C.c_int, [_vp, _vp, _vp, _i64, C.c_int, C.c_int, _vp, _vp]),
 }

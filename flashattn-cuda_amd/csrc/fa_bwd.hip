@@ -40,6 +40,7 @@
 #include <type_traits>
 
 #include "fa_mi355x.h"
+#include "fa_probe.h"
 #include "fa_tile.hpp"
 
 namespace fa {
@@ -1248,6 +1249,19 @@ extern "C" int64_t fa_bwd_gqa_workspace_floats(int64_t B, int64_t H, int64_t H_k
 
 namespace fa {
 namespace bwd {
+// Whether workgroups own 64 rows instead of 128, where `blocks` is the number
+// of 128-row blocks (each has a dK/dV and a dQ workgroup): where those fill
+// half of the CUs at most, or, causal and of long rows, all of them once (the
+// longest block then sets the time). us, 128 -> 64 rows: D = 64 B1 H8 N1024
+// 24.8 -> 18.4, B1 H4 N2048 39.0 -> 28.2, causal B1 H8 N2048 40.3 -> 32.7, B1
+// H4 N4000 86.2 -> 49.9; D = 128 37.6 -> 29.3, 60.1 -> 44.6, 63.4 -> 50.8, 112.2
+// -> 81.3. Beyond: B1 H8 N1500 D = 64 (192 workgroups) 37.0 vs 39.2, causal B2
+// H16 N512 (256) 19.3 vs 20.7, B1 H8 N4096 132.9 vs 144.6, causal 84.5 vs 89.1.
+static bool narrow_blocks(int64_t blocks, int64_t N, int causal, int cus) {
+  const int64_t wide = 2 * blocks;
+  return 2 * wide <= cus || (causal && wide <= cus && N >= 1024);
+}
+
 template <bool BF16>
 static int bwd_run(const void* q, const void* k, const void* v, const void* o, const void* dout,
                    const Fp32Inputs& in, const float* lse, float* dq, float* dk, float* dv, float* workspace,
@@ -1261,15 +1275,7 @@ static int bwd_run(const void* q, const void* k, const void* v, const void* o, c
     return geo.cu == nullptr ? (int64_t)(geo.N + br - 1) / br
                              : varlen_units(geo.B, geo.total, geo.N, br);
   };
-  // 64-row blocks where 128-row ones fill half of the CUs at most, or, causal
-  // and of long rows, all of them once (the longest block then sets the time).
-  // us, 128 -> 64 rows: D = 64 B1 H8 N1024 24.8 -> 18.4, B1 H4 N2048 39.0 ->
-  // 28.2, causal B1 H8 N2048 40.3 -> 32.7, B1 H4 N4000 86.2 -> 49.9; D = 128
-  // 37.6 -> 29.3, 60.1 -> 44.6, 63.4 -> 50.8, 112.2 -> 81.3. Beyond: B1 H8 N1500
-  // D = 64 (192 workgroups) 37.0 vs 39.2, causal B2 H16 N512 (256) 19.3 vs 20.7,
-  // B1 H8 N4096 132.9 vs 144.6, causal 84.5 vs 89.1.
-  const int64_t wide = 2 * heads * blocks_of(block_rows<2>());
-  const bool rows4 = 2 * wide <= topo.cus || (causal && wide <= topo.cus && geo.N >= 1024);
+  const bool rows4 = narrow_blocks(heads * blocks_of(block_rows<2>()), geo.N, causal, topo.cus);
   const int64_t per_head = blocks_of(rows4 ? block_rows<4>() : block_rows<2>());
   if (2 * heads * per_head > (int64_t(1) << 31) - 1) return FA_ERR_TOO_LARGE;
   const UnitMap um = unit_map(heads, per_head, topo, causal != 0 || geo.cu != nullptr);
@@ -1301,6 +1307,13 @@ static int bwd_gqa(bool bf16, const void* q, const void* k, const void* v, const
 }
 }  // namespace bwd
 }  // namespace fa
+
+extern "C" int fa_probe_bwd_block_rows(int causal, int64_t bh, int64_t N, int cus) {
+  using namespace fa::bwd;
+  if (bh <= 0 || N <= 0 || cus <= 0) return 0;
+  return narrow_blocks(bh * ((N + block_rows<2>() - 1) / block_rows<2>()), N, causal, cus)
+             ? block_rows<4>() : block_rows<2>();
+}
 
 extern "C" int fa_bwd_f16(const void* q, const void* k, const void* v, const void* o,
                           const void* dout, const float* lse, float* dq, float* dk, float* dv,

@@ -14,7 +14,7 @@
  * fa_probe_splitkv_plan_cus (the kernel and split choices for a given
  * compute-unit count, without a device); 4 added fa_probe_gather_bw; 5 added
  * fa_probe_unit_of and variant 432; 6 added fa_probe_decode_ordered and
- * lists variant 432.
+ * fa_probe_bwd_block_rows, and lists variant 432.
  */
 #ifndef FA_PROBE_H
 #define FA_PROBE_H
@@ -93,6 +93,11 @@ int fa_probe_unit_of(int64_t heads, int64_t per_head, int nxcd, int cus, int une
  * once run in index order), else 0. No device needed. */
 int fa_probe_decode_ordered(int64_t B, int64_t H, int64_t H_kv, int64_t D, int64_t num_splits,
                             int cus);
+
+/* Rows that a workgroup of the backward owns (128 or 64) for bh = B*H heads of
+ * N rows on a device of `cus` compute units; 0 for a bad argument. No device
+ * needed. */
+int fa_probe_bwd_block_rows(int causal, int64_t bh, int64_t N, int cus);
 
 /* Writes up to max_out codes of the variants that exist for head dimension D
  * and the causal flag into out (may be NULL) and returns how many there are. */

@@ -113,6 +113,61 @@ def test_bf16_backward(fa, dev, D, B, H, Hkv, N, causal):
           f"dQ/dK/dV max err {errs[0]:.2e} {errs[1]:.2e} {errs[2]:.2e}")
 
 
+# Heads enough for the 128-row blocks (the shapes above run 64-row ones), at an
+# N that is no multiple of a block or tile, grouped heads among them: two KV
+# heads and their query heads against the oracle.
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,H,Hkv,N,causal", [(2, 32, 8, 1100, True), (1, 32, 8, 1100, False), (1, 16, 16, 1030, True)])
+def test_bf16_wide_blocks(fa, capi, dev, D, B, H, Hkv, N, causal):
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    lib, g = capi.load(), H // Hkv
+    if H == 32:
+        assert lib.fa_probe_choose_variant(D, int(causal), B * H, N, cus) == 204
+    assert lib.fa_probe_bwd_block_rows(int(causal), B * H, N, cus) == 128
+    rng = np.random.default_rng(N + D + H)
+    Q, G = (rng.standard_normal((B, H, N, D)).astype(np.float32) for _ in range(2))
+    K, V = (rng.standard_normal((B, Hkv, N, D)).astype(np.float32) for _ in range(2))
+    tq, tk, tv, tg = (torch.from_numpy(x).to(dev).bfloat16() for x in (Q, K, V, G))
+    O, L = fa.forward_bf16(tq, tk, tv, causal=causal)
+    (O2,) = fa.forward_bf16(tq, tk, tv, causal=causal, want_L=False)
+    grads = fa.backward_bf16(tq, tk, tv, O, tg, L, causal=causal)
+    torch.cuda.synchronize()
+    assert torch.equal(O, O2)
+    for b, hk in ((0, 0), (B - 1, Hkv - 1)):
+        hs = slice(hk * g, (hk + 1) * g)
+        q, do = bf16_cast(Q[b:b + 1, hs]), bf16_cast(G[b:b + 1, hs])
+        k, v = (np.repeat(bf16_cast(x[b:b + 1, hk:hk + 1]), g, axis=1) for x in (K, V))
+        Or, Lr = naive_attention(q, k, v, causal=causal)
+        err = np.abs(O[b:b + 1, hs].float().cpu().numpy() - Or)
+        assert (err <= 1e-2 + bf16_half_ulp(Or)).all(), f"O max err {err.max():.3e}"
+        assert (np.abs(L[b:b + 1, hs].cpu().numpy() - Lr) / np.maximum(np.abs(Lr), 1)).max() <= 1e-4
+        rQ, rK, rV = naive_attention_backward(q, k, v, do, causal)
+        got = [grads[0][b:b + 1, hs], grads[1][b:b + 1, hk], grads[2][b:b + 1, hk]]
+        for name, x, r, n in zip(("dQ", "dK", "dV"), got, (rQ, rK.sum(axis=1), rV.sum(axis=1)), (1, g, g)):
+            err = np.abs(x.cpu().numpy() - r)
+            assert (err <= BWD_ATOL * n + BWD_RTOL * np.abs(r)).all(), f"{name} max err {err.max():.3e}"
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("N", [1, 65, 129, 321])
+@pytest.mark.parametrize("B,H,rows", [(16, 16, 128), (1, 2, 64)])
+def test_bf16_block_widths(fa, capi, dev, D, causal, N, B, H, rows):
+    """Both workgroup widths of the backward in bf16 at the edges of their blocks and tiles."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert capi.load().fa_probe_bwd_block_rows(int(causal), B * H, N, cus) == rows
+    rng = np.random.default_rng(N)
+    X = [rng.standard_normal((B, H, N, D)).astype(np.float32) for _ in range(4)]
+    tq, tk, tv, tg = (torch.from_numpy(x).to(dev).bfloat16() for x in X)
+    O, L = fa.forward_bf16(tq, tk, tv, causal=causal)
+    got = fa.backward_bf16(tq, tk, tv, O, tg, L, causal=causal)
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        ref = naive_attention_backward(*(bf16_cast(x[b:b + 1, h:h + 1]) for x in X), causal)
+        for name, x, r in zip(("dQ", "dK", "dV"), got, ref):
+            err = np.abs(x[b:b + 1, h:h + 1].cpu().numpy() - r)
+            assert (err <= BWD_ATOL + BWD_RTOL * np.abs(r)).all(), f"{name} max err {err.max():.3e}"
+
+
 def test_bf16_backward_identities_headline(fa, dev):
     """B1 H8 N4096 D64: sum_j dV_j = sum_i dO_i and sum_j dK_j = 0 per head."""
     B, H, N, D = 1, 8, 4096, 64

@@ -221,6 +221,30 @@ def test_gqa_backward(fa, dev, D, H, Hkv, N, causal):
              f"GQA H{H} Hkv{Hkv} N{N} D{D} causal={causal}")
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hkv,causal", [(8, True), (4, False)])
+def test_gqa_backward_wide_blocks(fa, capi, dev, D, Hkv, causal):
+    """Grouped heads through the 128-row blocks (the shapes above run 64-row
+    ones): two KV heads and their query heads against the oracle."""
+    B, H, N = 1, 32, 1100
+    g = H // Hkv
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert capi.load().fa_probe_bwd_block_rows(int(causal), B * H, N, cus) == 128
+    rng = np.random.default_rng(N + D + Hkv)
+    Q, G = (rng.standard_normal((B, H, N, D)).astype(np.float32) for _ in range(2))
+    K, V = (rng.standard_normal((B, Hkv, N, D)).astype(np.float32) for _ in range(2))
+    tq, tk, tv, tg = (torch.from_numpy(x).to(dev).half() for x in (Q, K, V, G))
+    O, L = fa.forward(tq, tk, tv, causal=causal)
+    grads = [x.cpu().numpy() for x in fa.backward(tq, tk, tv, O, tg, L, causal=causal)]
+    for hk in (0, Hkv - 1):
+        hs = slice(hk * g, (hk + 1) * g)
+        k, v = (np.repeat(half_cast(x[:, hk:hk + 1]), g, axis=1) for x in (K, V))
+        rQ, rK, rV = naive_attention_backward(half_cast(Q[:, hs]), k, v, half_cast(G[:, hs]), causal)
+        _compare([grads[0][:, hs]], [rQ], TIGHT_ATOL, TIGHT_RTOL, f"KV head {hk}")
+        _compare([x[:, hk] for x in grads[1:]], [rK.sum(axis=1), rV.sum(axis=1)], TIGHT_ATOL * g, TIGHT_RTOL,
+                 f"KV head {hk} dK dV")
+
+
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("B,H,Hkv,N,D", [(1, 1, 1, 1, 64), (1, 3, 1, 33, 64), (2, 4, 2, 70, 128), (1, 8, 8, 512, 64)])
 def test_fp32_inputs_are_rounded_first(fa, dev, bf16, B, H, Hkv, N, D):
@@ -248,9 +272,11 @@ def test_fp32_inputs_are_rounded_first(fa, dev, bf16, B, H, Hkv, N, D):
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("N", [1, 33, 64, 65, 127, 129, 200, 321])
 @pytest.mark.parametrize("B,H", [(16, 16), (1, 2)])
-def test_block_widths(fa, dev, D, causal, N, B, H):
+def test_block_widths(fa, capi, dev, D, causal, N, B, H):
     """Both workgroup widths (256 heads run 128-row blocks, 2 heads 64-row ones)
     at the edges of their blocks, tiles and tile pairs."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert capi.load().fa_probe_bwd_block_rows(int(causal), B * H, N, cus) == (64 if B == 1 else 128)
     rng = np.random.default_rng(N)
     Q, K, V, dO = (rng.standard_normal((B, H, N, D)).astype(np.float16) for _ in range(4))
     tq, tk, tv, tg = (torch.from_numpy(x).to(dev) for x in (Q, K, V, dO))

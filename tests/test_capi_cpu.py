@@ -432,3 +432,11 @@ def test_cast_rejects_before_touching_the_device(capi):
     assert lib.fa_cast_f32(p(A, 0, 0), p(A, 0, 0), n(-1, 0, 0), 0, None) == capi.STATUS["FA_ERR_SEQ_LEN"]
     assert lib.fa_cast_f32(p(A, 0, 0), p(A, 0, 0), n(1 << 50, 0, 0), 0, None) == capi.STATUS["FA_ERR_TOO_LARGE"]
     assert lib.fa_cast_f32(p(0, 0, 0), p(0, 0, 0), n(5, 5, 5), 0, None) == capi.STATUS["FA_OK"]   # nothing to do
+
+
+@pytest.mark.parametrize("causal,bh,N,cus,rows", [
+    (0, 8, 1024, 256, 64), (0, 8, 1025, 256, 128), (0, 64, 128, 256, 64), (0, 65, 128, 256, 128),
+    (1, 8, 2048, 256, 64), (1, 8, 2049, 256, 128), (1, 16, 1024, 256, 64), (1, 18, 896, 256, 128), (1, 8, 1500, 256, 64),
+    (0, 1, 1, 256, 64), (0, 1, 1024, 32, 64), (0, 2, 1024, 32, 128), (0, 0, 64, 256, 0)])
+def test_backward_block_choice(capi, causal, bh, N, cus, rows):
+    assert capi.load().fa_probe_bwd_block_rows(causal, bh, N, cus) == rows
