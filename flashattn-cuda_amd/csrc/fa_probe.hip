@@ -53,7 +53,7 @@ __global__ void probe_tr16_raw_kernel(const uint16_t* in, uint16_t* out) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) lds[4 * l + i] = in[4 * l + i];
   __syncthreads();
-  f16x4 v = lds_read_tr16(reinterpret_cast<const char*>(lds) + 8 * l);
+  f16x4 v = lds_tr16((lds_cp)(size_t)(lds_addr(lds) + 8 * l));
   // Store the vector whole: extracting elements through __builtin_bit_cast was
   // observed to be miscompiled (all four lanes of the vector read element 0).
   *reinterpret_cast<f16x4*>(out + 4 * l) = v;
@@ -71,21 +71,26 @@ __global__ void probe_permlane_kernel(const float* in, float* out) {
   out[192 + l] = sum_xor32(x);
 }
 
-// Stores a [64][D] tile with the forward kernel's K and V layouts, then reads
-// every operand fragment the kernel reads.
-//   kout: [2 kb][D/16 kk][64 lanes][8]    (load_k_frag)
-//   vout: [4 j][D/32 db][64 lanes][8]     (load_v_frag)
+// LDS offset of chunk c of row r in a backward tile.
 template <int D>
-__global__ void probe_frag_kernel(const f16* tile, f16* kout, f16* vout) {
+__device__ int t_off(int r, int c) { return r * 2 * D + (c ^ t_swz<D>(r)) * 16; }
+
+// Stores a [64][D] tile in the layouts of the forward's K tiles and of the
+// backward's tiles, then reads every operand fragment the kernels read.
+//   kout: [2 kb][D/16 kk][64 lanes][8]    forward K rows (load_k_frag)
+//   rout: the same, backward rows         (load_row_frag)
+//   cout: [4 j][D/32 db][64 lanes][8]     backward columns (load_col_frag)
+template <int D>
+__global__ void probe_frag_kernel(const f16* tile, f16* kout, f16* rout, f16* cout) {
   constexpr int TILE = 64 * D * 2;
   constexpr int CPR = D / 8;
-  __shared__ __attribute__((aligned(16))) char smem[2 * TILE];
+  __shared__ __attribute__((aligned(1024))) char smem[2 * TILE];
   const int l = threadIdx.x;
   for (int id = l; id < 64 * CPR; id += 64) {
     const int r = id / CPR, cc = id % CPR;
     const u32x4 x = *reinterpret_cast<const u32x4*>(tile + r * D + cc * 8);
     *reinterpret_cast<u32x4*>(smem + k_off<D>(r, cc)) = x;
-    *reinterpret_cast<u32x4*>(smem + TILE + v_off<D>(r, cc)) = x;
+    *reinterpret_cast<u32x4*>(smem + TILE + t_off<D>(r, cc)) = x;
   }
   __syncthreads();
   for (int kb = 0; kb < 2; ++kb)
@@ -93,11 +98,17 @@ __global__ void probe_frag_kernel(const f16* tile, f16* kout, f16* vout) {
       f16x8 x = load_k_frag<D>(smem, kb, kk, l);
       *reinterpret_cast<f16x8*>(kout + (((kb * (D / 16) + kk) * 64) + l) * 8) = x;
     }
-  for (int j = 0; j < 4; ++j)
-    for (int db = 0; db < D / 32; ++db) {
-      f16x8 x = load_v_frag<D>(smem + TILE, j, db, l);
-      *reinterpret_cast<f16x8*>(vout + (((j * (D / 32) + db) * 64) + l) * 8) = x;
-    }
+  // The backward reads a tile by halves of 32 rows.
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t half = lds_addr(smem) + TILE + h * 32 * 2 * D;
+    const uint32_t rb = row_base<D>(half, l), cb = col_base<D>(half, l);
+    for (int kk = 0; kk < D / 16; ++kk)
+      *reinterpret_cast<f16x8*>(rout + (((h * (D / 16) + kk) * 64) + l) * 8) = load_row_frag<D>(rb, 0, kk);
+    for (int j = 0; j < 2; ++j)
+      for (int db = 0; db < D / 32; ++db)
+        *reinterpret_cast<f16x8*>(cout + ((((2 * h + j) * (D / 32) + db) * 64) + l) * 8) =
+            load_col_frag<D>(cb, 0, j, db);
+  }
 }
 
 // One wave, one 64-key tile, no softmax: S^T = K Q^T, P = fp16(S), O^T = V^T P^T,
@@ -107,13 +118,13 @@ template <int D>
 __global__ void probe_chain_kernel(const f16* q, const f16* k, const f16* v, float* o) {
   constexpr int TILE = 64 * D * 2;
   constexpr int CPR = D / 8;
-  __shared__ __attribute__((aligned(16))) char smem[2 * TILE];
+  __shared__ __attribute__((aligned(1024))) char smem[2 * TILE];
   const int l = threadIdx.x;
   for (int id = l; id < 64 * CPR; id += 64) {
     const int r = id / CPR, cc = id % CPR;
     *reinterpret_cast<u32x4*>(smem + k_off<D>(r, cc)) =
         *reinterpret_cast<const u32x4*>(k + r * D + cc * 8);
-    *reinterpret_cast<u32x4*>(smem + TILE + v_off<D>(r, cc)) =
+    *reinterpret_cast<u32x4*>(smem + TILE + t_off<D>(r, cc)) =
         *reinterpret_cast<const u32x4*>(v + r * D + cc * 8);
   }
   __syncthreads();
@@ -128,7 +139,10 @@ __global__ void probe_chain_kernel(const f16* q, const f16* k, const f16* v, flo
   f16x8 pf[4] = {pack_p(s[0], 0), pack_p(s[0], 1), pack_p(s[1], 0), pack_p(s[1], 1)};
   for (int db = 0; db < D / 32; ++db) {
     f32x16 acc = f32x16{};
-    for (int j = 0; j < 4; ++j) acc = mfma32(load_v_frag<D>(smem + TILE, j, db, l), pf[j], acc);
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t cb = col_base<D>(lds_addr(smem) + TILE + (j >> 1) * 32 * 2 * D, l);
+      acc = mfma32(load_col_frag<D>(cb, 0, j & 1, db), pf[j], acc);
+    }
     for (int r = 0; r < 16; ++r)
       o[(l & 31) * D + 32 * db + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3)] = acc[r];
   }
@@ -168,14 +182,15 @@ extern "C" int fa_probe_permlane(const float* in, float* out, void* stream) {
   return finish();
 }
 
-extern "C" int fa_probe_frags(const void* tile, void* kout, void* vout, int64_t D, void* stream) {
-  if (!tile || !kout || !vout) return 1;
+extern "C" int fa_probe_frags(const void* tile, void* kout, void* rout, void* cout, int64_t D,
+                              void* stream) {
+  if (!tile || !kout || !rout || !cout) return 1;
   if (D == 64) {
     hipLaunchKernelGGL(fa::probe_frag_kernel<64>, dim3(1), dim3(64), 0, (hipStream_t)stream,
-                       (const fa::f16*)tile, (fa::f16*)kout, (fa::f16*)vout);
+                       (const fa::f16*)tile, (fa::f16*)kout, (fa::f16*)rout, (fa::f16*)cout);
   } else if (D == 128) {
     hipLaunchKernelGGL(fa::probe_frag_kernel<128>, dim3(1), dim3(64), 0, (hipStream_t)stream,
-                       (const fa::f16*)tile, (fa::f16*)kout, (fa::f16*)vout);
+                       (const fa::f16*)tile, (fa::f16*)kout, (fa::f16*)rout, (fa::f16*)cout);
   } else {
     return 2;
   }

@@ -147,10 +147,12 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 
 // ---------------------------------------------------------------------------
-// LDS tile layouts. A K or V tile is BC rows (keys) x D fp16, row stride 2*D
+// LDS tile layouts. A tile is rows (keys or queries) x D fp16, row stride 2*D
 // bytes, stored as 16-byte chunks (8 halves). Chunk c of row r lives at chunk
 // slot pos(r, c) of that row; pos is an XOR swizzle chosen so that the
-// operand reads below hit distinct LDS banks within each 16-lane group.
+// operand reads below hit distinct LDS banks within each 16-lane group. k_swz
+// is that of the forward's K tiles (row reads only; its V tiles are blocks,
+// beside its kernel), t_swz below that of the backward's.
 // ---------------------------------------------------------------------------
 template <int D>
 __device__ __forceinline__ int k_swz(int r) {
@@ -161,27 +163,12 @@ __device__ __forceinline__ int k_swz(int r) {
   }
 }
 
-template <int D>
-__device__ __forceinline__ int v_swz(int r) {
-  if constexpr (D == 64) {
-    return ((r >> 1) & 1) << 2;
-  } else {
-    return (r & 3) << 2;
-  }
-}
-
 // XOR swizzles are involutions: slot = c ^ swz(r) and c = slot ^ swz(r).
 template <int D>
 __device__ __forceinline__ int k_slot(int r, int c) { return c ^ k_swz<D>(r); }
 
 template <int D>
-__device__ __forceinline__ int v_slot(int r, int c) { return c ^ v_swz<D>(r); }
-
-template <int D>
 __device__ __forceinline__ int k_off(int r, int c) { return r * (2 * D) + k_slot<D>(r, c) * 16; }
-
-template <int D>
-__device__ __forceinline__ int v_off(int r, int c) { return r * (2 * D) + v_slot<D>(r, c) * 16; }
 
 // LDS pointers for the pipelined kernel's operand reads: arithmetic on them
 // stays in the 32-bit LDS address space, so constant offsets fold into the
@@ -200,18 +187,15 @@ __device__ __forceinline__ f16x8 lds_b128(lds_cp p) {
   return *reinterpret_cast<const __attribute__((address_space(3))) f16x8*>(p);
 }
 
+// ds_read_b64_tr_b16: within each group of 16 lanes, lane s supplies the
+// address of 4 consecutive halves M[s][0..3]; it receives
+// out[e] = M[4*e + s/4][s%4]. If lane s points at row (k0 + s/4),
+// columns (d0 + 4*(s%4)) .. +3 of a row-major [key][d] tile, lane s receives
+// the column d0 + s for keys k0 .. k0+3.
 __device__ __forceinline__ f16x4 lds_tr16(lds_cp p) {
   typedef __attribute__((address_space(3))) fp16x4_t lds_fp16x4;
   fp16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4*)(p));
   return __builtin_bit_cast(f16x4, v);
-}
-
-// V fragment (see load_v_frag) whose k-step-0 address is p.
-template <int D>
-__device__ __forceinline__ f16x8 v_frag_lds(lds_cp p) {
-  f16x4 lo = lds_tr16(p);
-  f16x4 up = lds_tr16(p + 8 * 2 * D);
-  return f16x8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
 }
 
 // A operand of S^T = K Q^T for key block kb (32 keys) and k-step kk (16 of D).
@@ -225,45 +209,6 @@ __device__ __forceinline__ int k_frag_off(int kk, int lane) {
 template <int D>
 __device__ __forceinline__ f16x8 load_k_frag(const char* ks, int kb, int kk, int lane) {
   return *reinterpret_cast<const f16x8*>(ks + 32 * kb * 2 * D + k_frag_off<D>(kk, lane));
-}
-
-// ds_read_b64_tr_b16: within each group of 16 lanes, lane s supplies the
-// address of 4 consecutive halves M[s][0..3]; it receives
-// out[e] = M[4*e + s/4][s%4]. If lane s points at row (k0 + s/4),
-// columns (d0 + 4*(s%4)) .. +3 of a row-major [key][d] tile, lane s receives
-// the column d0 + s for keys k0 .. k0+3.
-__device__ __forceinline__ f16x4 lds_read_tr16(const char* p) {
-  typedef __attribute__((address_space(3))) fp16x4_t lds_fp16x4;
-  fp16x4_t v = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4*)(p));
-  return __builtin_bit_cast(f16x4, v);
-}
-
-// A operand of O^T = V^T P^T for PV k-step j (16 keys of the 64-key tile) and
-// d-block db (32 of D). Slot i of lane l must hold V[key(j, i, l)][32*db + l%32]
-// with key(j, i, l) = 16*j + 8*(i/4) + 4*(l/32) + i%4, the key order of the
-// S^T accumulator registers (see pack_p). Lane l reads rows r0 = 4*(l/32) +
-// (l%16)/4 (+16 j) and r0 + 8; the V swizzle depends on the row only modulo
-// 4, so k-step j and the upper 4 keys are constant row shifts of
-// v_frag_off(db, lane).
-template <int D>
-__device__ __forceinline__ int v_frag_off(int db, int lane) {
-  const int s = lane & 15;
-  const int d = 32 * db + 16 * ((lane >> 4) & 1) + 4 * (s & 3);
-  const int r0 = 4 * (lane >> 5) + (s >> 2);
-  return v_off<D>(r0, d >> 3) + 8 * ((d >> 2) & 1);
-}
-
-// The fragment whose k-step j = 0 row-0 address is p (= tile + v_frag_off).
-template <int D>
-__device__ __forceinline__ f16x8 v_frag_at(const char* p) {
-  f16x4 lo = lds_read_tr16(p);
-  f16x4 up = lds_read_tr16(p + 8 * 2 * D);
-  return f16x8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
-}
-
-template <int D>
-__device__ __forceinline__ f16x8 load_v_frag(const char* vs, int j, int db, int lane) {
-  return v_frag_at<D>(vs + 16 * j * 2 * D + v_frag_off<D>(db, lane));
 }
 
 // One layout for both reads (the backward's tiles, read as rows and
@@ -315,8 +260,10 @@ __device__ __forceinline__ f16x8 load_row_frag(uint32_t base, int off, int kk) {
 }
 
 // Columns 32 db .. + 31 of rows 16 j .. + 15 as an A operand (transposed),
-// `off` bytes on: as load_v_frag. Eight rows up, t_swz differs in its bit 1,
-// address bit 5.
+// `off` bytes on: slot i of lane l holds column 32 db + l % 32 of row
+// 16 j + 8 (i / 4) + 4 (l / 32) + i % 4, the row order of the score
+// accumulators (see pack_p). Eight rows up, t_swz differs in its bit 1, address
+// bit 5.
 template <int D>
 __device__ __forceinline__ f16x8 load_col_frag(uint32_t base, int off, int j, int db) {
   const f16x4 lo = lds_tr16((lds_cp)(size_t)(base ^ (64 * db)) + off + 16 * j * 2 * D);

@@ -565,10 +565,12 @@ std::vector<torch::Tensor> probe_frags(torch::Tensor tile) {
   const int64_t D = tile.size(1);
   auto tc = tile.contiguous();
   auto kout = torch::empty({2, D / 16, 64, 8}, tile.options());
-  auto vout = torch::empty({4, D / 32, 64, 8}, tile.options());
-  check_status(fa_probe_frags(tc.data_ptr(), kout.data_ptr(), vout.data_ptr(), D, current_stream(tile)),
+  auto rout = torch::empty_like(kout);
+  auto cout = torch::empty({4, D / 32, 64, 8}, tile.options());
+  check_status(fa_probe_frags(tc.data_ptr(), kout.data_ptr(), rout.data_ptr(), cout.data_ptr(), D,
+                              current_stream(tile)),
                "fa_probe_frags");
-  return {kout, vout};
+  return {kout, rout, cout};
 }
 
 // One streaming read of x (any dtype, contiguous, 16-byte multiple) into the

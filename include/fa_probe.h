@@ -14,7 +14,8 @@
  * fa_probe_splitkv_plan_cus (the kernel and split choices for a given
  * compute-unit count, without a device); 4 added fa_probe_gather_bw; 5 added
  * fa_probe_unit_of and variant 432; 6 added fa_probe_decode_ordered and
- * fa_probe_bwd_block_rows, and lists variant 432.
+ * fa_probe_bwd_block_rows, lists variant 432, and fa_probe_frags dumps the
+ * backward's fragments.
  */
 #ifndef FA_PROBE_H
 #define FA_PROBE_H
@@ -43,12 +44,14 @@ int fa_probe_tr16_raw(const void* in, void* out, void* stream);
  * through the forward kernel's helpers. */
 int fa_probe_permlane(const float* in, float* out, void* stream);
 
-/* Stores a [64][D] fp16 tile with the forward kernel's K and V LDS layouts and
- * dumps every operand fragment the kernel reads:
- *   kout [2][D/16][64][8], vout [4][D/32][64][8] fp16. D in {64, 128}. */
-int fa_probe_frags(const void* tile, void* kout, void* vout, int64_t D, void* stream);
+/* Stores a [64][D] fp16 tile in the LDS layouts of the forward's K tiles and of
+ * the backward's tiles and dumps every operand fragment the kernels read:
+ *   kout [2][D/16][64][8] the forward's rows, rout the same of the backward,
+ *   cout [4][D/32][64][8] the backward's columns, fp16. D in {64, 128}. */
+int fa_probe_frags(const void* tile, void* kout, void* rout, void* cout, int64_t D,
+                   void* stream);
 
-/* One 64-key tile through the kernel's loaders and MFMA chain without softmax:
+/* One 64-key tile through the kernels' loaders and MFMA chain without softmax:
  * o[32][D] = fp16(q[32][D] @ k[64][D]^T) @ v[64][D], fp32 out. */
 int fa_probe_chain(const void* q, const void* k, const void* v, float* o, int64_t D,
                    void* stream);

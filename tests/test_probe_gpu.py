@@ -1,5 +1,5 @@
-"""GPU tier: on-device checks of the matrix-core and LDS layouts the forward
-kernel is built on, with negative controls (the method of the reference's
+"""GPU tier: on-device checks of the matrix-core and LDS layouts the
+kernels are built on, with negative controls (the method of the reference's
 tests/test_mma_probe.py:18-57, rebuilt for gfx950 instructions)."""
 import torch
 import pytest
@@ -58,9 +58,7 @@ def test_ds_read_tr16_semantics(fa, dev):
 def test_operand_fragments_exact(fa, dev, D):
     tile = (torch.arange(64 * D, dtype=torch.int32) % 30011).to(torch.int16).view(torch.half)
     tile = tile.view(64, D)
-    kout, vout = fa.probe.probe_frags(tile.to(dev))
-    kout = kout.cpu().view(torch.int16)
-    vout = vout.cpu().view(torch.int16)
+    kout, rout, cout = (x.cpu().view(torch.int16) for x in fa.probe.probe_frags(tile.to(dev)))
     t = tile.view(torch.int16)
     for kb in range(2):
         for kk in range(D // 16):
@@ -68,12 +66,13 @@ def test_operand_fragments_exact(fa, dev, D):
                 row = 32 * kb + (l % 32)
                 col = 16 * kk + 8 * (l // 32)
                 assert torch.equal(kout[kb, kk, l], t[row, col:col + 8]), (kb, kk, l)
+                assert torch.equal(rout[kb, kk, l], t[row, col:col + 8]), (kb, kk, l)
     for j in range(4):
         for db in range(D // 32):
             for l in range(64):
                 keys = [16 * j + 8 * (i // 4) + 4 * (l // 32) + (i % 4) for i in range(8)]
                 exp = t[keys, 32 * db + (l % 32)]
-                assert torch.equal(vout[j, db, l], exp), (j, db, l)
+                assert torch.equal(cout[j, db, l], exp), (j, db, l)
 
 
 @pytest.mark.parametrize("D", [64, 128])
