@@ -371,7 +371,7 @@ __device__ __forceinline__ f16x8 pack_px(const f32x16& p, int half_sel) {
 // >> (31+s) with 2^s >= d (the rounding adds less than 2^s to the numerator's
 // 2^(31+s), so the quotient is exact). A few scalar instructions where a
 // division by a kernel argument takes about forty vector ones; a workgroup's
-// address waits for several (B1 H8 N1024 D64: 8.39 -> 8.54 us with plain
+// address waits for several (B1 H8 N1024 D64: 8.20 -> 8.54 us with plain
 // divisions in unit_of).
 struct FastDiv {
   uint32_t d, mul, shift;
@@ -433,7 +433,7 @@ struct Unit {
 // starts its workgroups in order, so this decides what shares an L2 and what
 // is left for the end:
 //   * an XCD gets heads / nxcd whole heads (their K/V then live in its L2),
-//     `merge` of them at a time, level by level: unit i of each of them before
+//     one set of them at a time, level by level: unit i of each of them before
 //     unit i + 1 of any. The longest units of several heads start first and
 //     the short ones fill the end; one head after the other leaves the last
 //     head's long units to a few CUs.
