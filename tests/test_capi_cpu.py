@@ -335,7 +335,7 @@ def test_kernel_and_split_choice_follow_the_cu_count(capi):
     differently, and both choices follow the measured crossovers."""
     lib = capi.load()
     choose, plan = lib.fa_probe_choose_variant, lib.fa_probe_splitkv_plan_cus
-    # D = 128 always runs the 128-row kernel
+    # D = 128: the 128-row kernel from one block a CU on (non-causal), and for a single 64-row block
     assert choose(128, 0, 8, 4096, 256) == 204 and choose(128, 1, 1, 64, 32) == 204
     # D = 64 at 256 CUs: fewer 128-row blocks than CUs -> the 64-row kernel
     assert choose(64, 0, 8, 2048, 256) == 408      # 128 blocks < 256

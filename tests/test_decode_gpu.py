@@ -196,11 +196,14 @@ def test_split_count_invariance(fa, dev):
     assert torch.equal(po[:, :, 0].half(), O1)
 
 
-@pytest.mark.parametrize("B,Hkv", [(40, 4), (300, 4), (300, 2)])
-def test_sequence_order_is_a_permutation(fa, dev, B, Hkv):
+@pytest.mark.parametrize("B,Hkv,S,ordered", [(40, 4, 3, 0), (40, 4, 16, 1), (256, 2, 16, 1), (300, 4, 3, 0), (300, 2, 3, 0)])
+def test_sequence_order_is_a_permutation(fa, capi, dev, B, Hkv, S, ordered):
     """Workgroups take sequences longest first (ranked in the kernel for
-    B <= 256, identity order above): every sequence is still decoded exactly
-    once, repeated and zero lengths included, against the oracle."""
+    B <= 256 and more workgroups than run at once, index order else): every
+    sequence is still decoded exactly once, repeated and zero lengths included,
+    against the oracle."""
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    assert capi.load().fa_probe_decode_ordered(B, 4, Hkv, 64, S, cus) == ordered
     rng = np.random.default_rng(B + Hkv)
     ctx = rng.integers(0, 60, B)
     ctx[::7] = 33                                   # ties broken by index
@@ -217,7 +220,7 @@ def test_sequence_order_is_a_permutation(fa, dev, B, Hkv):
     q = rng.standard_normal((B, H, D)).astype(np.float16)
     kp = rng.standard_normal((P, Hkv, 16, D)).astype(np.float16)
     vp = rng.standard_normal((P, Hkv, 16, D)).astype(np.float16)
-    O, L = fa.decode_paged(*_dev(dev, q, kp, vp, table, ctx.astype(np.int32)), num_splits=3)
+    O, L = fa.decode_paged(*_dev(dev, q, kp, vp, table, ctx.astype(np.int32)), num_splits=S)
     g = H // Hkv
     Or, Lr = decode_attention(q, np.repeat(kp, g, axis=1), np.repeat(vp, g, axis=1), table, ctx)
     O, L = O.float().cpu().numpy(), L.cpu().numpy()
