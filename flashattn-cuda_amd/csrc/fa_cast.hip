@@ -37,53 +37,71 @@ struct FillBuf {
 // falls does each row look for its sequence.
 constexpr int kFillRows = 64;
 constexpr int kFillGroups = 512;
-__global__ void __launch_bounds__(256)
-fa_fill_outside_kernel(Geom g, FillBuf b0, FillBuf b1, FillBuf b2) {
-  __shared__ uint8_t inside[kFillRows];
-  const int tid = threadIdx.x;
+
+// Whether a sequence falls or is longer than max_seqlen, the same in every thread.
+template <int UNROLL>
+__device__ __forceinline__ int odd_table(const Geom& g) {
   int odd = 0;
-#pragma unroll 4
-  for (int b = tid; b < g.B; b += 256) {
+#pragma unroll UNROLL
+  for (int b = threadIdx.x; b < g.B; b += 256) {
     const int c0 = clamp_row(g.cu[b], g.total), c1 = clamp_row(g.cu[b + 1], g.total);
     odd |= c1 < c0 || c1 - c0 > g.N;
   }
-  odd = __syncthreads_or(odd);
+  return __syncthreads_or(odd);
+}
+
+// Rows r0 .. r0 + kFillRows - 1.
+__device__ __forceinline__ void fill_chunk(const Geom& g, const FillBuf& b0, const FillBuf& b1,
+                                           const FillBuf& b2, int odd, int r0, uint8_t* inside) {
+  const int tid = threadIdx.x;
   const int first = clamp_row(g.cu[0], g.total), last = clamp_row(g.cu[g.B], g.total);
-  for (int64_t at = (int64_t)blockIdx.x * kFillRows; at < g.total; at += (int64_t)gridDim.x * kFillRows) {
-    const int r0 = (int)at;
-    if (!odd && r0 >= first && min(r0 + kFillRows, g.total) <= last) continue;
-    __syncthreads();   // the rows of the chunk before are written
-    if (tid < kFillRows) {
-      const int r = r0 + tid;
-      bool in = !odd && r >= first && r < last;
-      if (odd) {
-        // Sequences as the attention kernels take them: up to kCountedSeqs from
-        // the running maximum of the bounds on, more of them as they stand.
-        int end = 0;
-        for (int b = 0; b < g.B; ++b) {
-          const int c0 = clamp_row(g.cu[b], g.total), c1 = clamp_row(g.cu[b + 1], g.total);
-          const int s0 = g.B <= kCountedSeqs ? max(c0, end) : c0;
-          const int s1 = max(s0, c1);
-          in |= r >= s0 && r < s0 + min(s1 - s0, g.N);
-          end = max(end, s1);
-        }
+  if (!odd && r0 >= first && min(r0 + kFillRows, g.total) <= last) return;
+  if (tid < kFillRows) {
+    const int r = r0 + tid;
+    bool in = !odd && r >= first && r < last;
+    if (odd) {
+      // Sequences as the attention kernels take them: up to kCountedSeqs from
+      // the running maximum of the bounds on, more of them as they stand.
+      int end = 0;
+      for (int b = 0; b < g.B; ++b) {
+        const int c0 = clamp_row(g.cu[b], g.total), c1 = clamp_row(g.cu[b + 1], g.total);
+        const int s0 = g.B <= kCountedSeqs ? max(c0, end) : c0;
+        const int s1 = max(s0, c1);
+        in |= r >= s0 && r < s0 + min(s1 - s0, g.N);
+        end = max(end, s1);
       }
-      inside[tid] = in;
     }
-    __syncthreads();
-    const FillBuf bufs[3] = {b0, b1, b2};
+    inside[tid] = in;
+  }
+  __syncthreads();
+  const FillBuf bufs[3] = {b0, b1, b2};
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const FillBuf b = bufs[i];
-      if (b.p == nullptr) continue;
-      for (int64_t h = 0; h < b.heads; ++h) {
-        uint32_t* row0 = b.p + (h * g.total + r0) * b.words;
-        for (int w = tid; w < kFillRows * b.words; w += 256) {
-          const int r = w / b.words;
-          if (r0 + r < g.total && !inside[r]) row0[w] = b.value;
-        }
+  for (int i = 0; i < 3; ++i) {
+    const FillBuf b = bufs[i];
+    if (b.p == nullptr) continue;
+    for (int64_t h = 0; h < b.heads; ++h) {
+      uint32_t* row0 = b.p + (h * g.total + r0) * b.words;
+      for (int w = tid; w < kFillRows * b.words; w += 256) {
+        const int r = w / b.words;
+        if (r0 + r < g.total && !inside[r]) row0[w] = b.value;
       }
     }
+  }
+}
+
+__global__ void __launch_bounds__(256)
+fa_fill_outside_kernel(Geom g, FillBuf b0, FillBuf b1, FillBuf b2) {
+  __shared__ uint8_t inside[kFillRows];
+  fill_chunk(g, b0, b1, b2, odd_table<1>(g), blockIdx.x * kFillRows, inside);
+}
+
+__global__ void __launch_bounds__(256)
+fa_fill_outside_many_kernel(Geom g, FillBuf b0, FillBuf b1, FillBuf b2) {
+  __shared__ uint8_t inside[kFillRows];
+  const int odd = odd_table<4>(g);
+  for (int64_t r0 = (int64_t)blockIdx.x * kFillRows; r0 < g.total; r0 += (int64_t)gridDim.x * kFillRows) {
+    fill_chunk(g, b0, b1, b2, odd, (int)r0, inside);
+    __syncthreads();   // before the next chunk's `inside`
   }
 }
 
@@ -131,9 +149,11 @@ extern "C" int fa_varlen_fill_outside(const int32_t* cu_seqlens, int64_t B, int6
   if (total == 0) return FA_OK;
   const Geom g{cu_seqlens, (int)max_seqlen, 1, FastDiv(1), (int)total, (int)B};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  int64_t groups = (total + kFillRows - 1) / kFillRows;
-  if (B > kCountedSeqs && groups > kFillGroups) groups = kFillGroups;
-  hipLaunchKernelGGL(fa_fill_outside_kernel, dim3((unsigned)groups), dim3(256), 0, s, g, b[0], b[1], b[2]);
+  const int64_t chunks = (total + kFillRows - 1) / kFillRows;
+  if (B > kCountedSeqs && chunks > kFillGroups)
+    hipLaunchKernelGGL(fa_fill_outside_many_kernel, dim3(kFillGroups), dim3(256), 0, s, g, b[0], b[1], b[2]);
+  else
+    hipLaunchKernelGGL(fa_fill_outside_kernel, dim3((unsigned)chunks), dim3(256), 0, s, g, b[0], b[1], b[2]);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? FA_OK : -(int)e;
 }
