@@ -604,19 +604,26 @@ __device__ __forceinline__ SeqBlock counted_block(const Geom& g, int u, int rows
 }
 
 // The same where no sequence is longer than a block: unit u is sequence u's,
-// which starts at the largest of the bounds up to it. One scan: the two scans
-// and the search of counted_block made forwards of 256 sequences of 64 rows,
-// H32 over 8 D64, 10 % slower (us: in sequence order, without a look at the
-// other bounds, 173; counted 191; so 170; of 500 sequences 338, 363, 354).
+// which starts at the largest of the bounds up to it. One scan, two bounds a
+// load: the two scans and the search of counted_block made forwards of 256
+// sequences of 64 rows, H32 over 8 D64, 10 % slower (us: in sequence order,
+// without a look at the other bounds, 173; counted 191; so 170; of 500
+// sequences 338, 363, 338; with a bound a load 354).
 template <int J>
 __device__ __forceinline__ SeqBlock single_block(const Geom& g, int u, int lane) {
+  typedef int pair __attribute__((ext_vector_type(2), aligned(4)));
   const int next = g.cu[u + 1];
   int c = 0;
 #pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const int b = 64 * j + lane;
-    if (b <= u) c = max(c, clamp_row(g.cu[b], g.total));
+  for (int j = 0; j < (J + 1) / 2; ++j) {
+    const int b = 128 * j + 2 * lane;
+    if (b <= u) {   // cu[b + 1] is there: u < B
+      const pair x = *reinterpret_cast<const pair*>(g.cu + b);
+      c = max(c, x[0]);
+      if (b < u) c = max(c, x[1]);
+    }
   }
+  c = clamp_row(c, g.total);
   const int start = __builtin_amdgcn_readlane(scan_max(c), 63);
   return SeqBlock{start, min(max(start, clamp_row(next, g.total)) - start, g.N), 0};
 }
